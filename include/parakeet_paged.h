@@ -38,7 +38,7 @@
 extern "C" {
 #endif
 
-#define PK_ABI_VERSION 9
+#define PK_ABI_VERSION 10
 
 enum pk_dtype { PK_DTYPE_F32 = 0, PK_DTYPE_F16 = 1, PK_DTYPE_BF16 = 2 };
 
@@ -337,6 +337,37 @@ typedef struct pk_resnorm_args {
   int64_t norm_out_stride;
 } pk_resnorm_args;
 int pk_residual_norm(const pk_resnorm_args* args, void* stream);
+
+/* ---------------------------------------------------------------------------
+ * pk_linear -- `count` linear layers, one after another on `stream` (each may
+ * read what the ones before it wrote):
+ *   out = act(x weight^T + bias)
+ * fp16 / bf16 operands, fp32 accumulation, bias and activation in fp32, one
+ * rounding of the output (SiLU is not rounded before its input, as two launches
+ * would).  Replaces the projections of feedforward.py:20-26 (linear1 with its
+ * SiLU, linear2), attention.py:92,122 and the pointwise convolutions of
+ * convolution.py:152,158.
+ * x [rows][k], weight [n][k], out [rows][n]: row strides in elements, rows
+ * 16-byte aligned with unit inner stride; bias [n] or NULL.  out overlaps no
+ * operand.  n a multiple of 64, k of 256 (else PK_ERR_UNSUPPORTED).
+ */
+enum pk_activation { PK_ACT_NONE = 0, PK_ACT_SILU = 1 };
+typedef struct pk_linear_args {
+  int32_t dtype;
+  int32_t device;
+  int32_t rows;
+  int32_t n;
+  int32_t k;
+  int32_t activation;
+  const void* x;
+  int64_t x_stride;
+  const void* weight;
+  int64_t weight_stride;
+  const void* bias;
+  void* out;
+  int64_t out_stride;
+} pk_linear_args;
+int pk_linear(const pk_linear_args* args, int32_t count, void* stream);
 
 /* ---------------------------------------------------------------------------
  * Pre-encode front end: pcm -> log-mel (pk_fe_step) -> 8x convolution

@@ -1,0 +1,514 @@
+// gfx950 linear layers of the encoder (parakeet/modules/feedforward.py:4-26,
+// attention.py:92,122, convolution.py:152,158):
+//
+//   out = act( x W^T + bias )
+//
+//   lin_row_kernel   a few rows: 16 x 16 outputs a workgroup, K split over its
+//                    waves, both operands straight from memory into registers
+//   lin_tile_kernel  16 x 32 to 256 x 256 outputs a workgroup, both operands
+//                    staged in LDS by buffer loads
+//
+// 16-bit operands, fp32 accumulation, one rounding of each output.
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstdint>
+
+#include "pk_common.h"
+#include "pk_device.h"
+
+namespace pk {
+
+template <typename ST>
+struct MmaL;
+template <>
+struct MmaL<_Float16> {
+  typedef _Float16 H8 __attribute__((ext_vector_type(8)));
+  __device__ static inline f32x4_t k32(u32x4 a, u32x4 b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(H8, a), __builtin_bit_cast(H8, b), c, 0, 0, 0);
+  }
+};
+template <>
+struct MmaL<bf16_t> {
+  typedef __bf16 H8 __attribute__((ext_vector_type(8)));
+  __device__ static inline f32x4_t k32(u32x4 a, u32x4 b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(H8, a), __builtin_bit_cast(H8, b), c, 0, 0, 0);
+  }
+};
+
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+enum { kEpiNone = 0, kEpiSilu = 1 };
+
+template <typename ST>
+struct LinK {
+  const ST* x;  // [M][K] rows, stride x_s
+  int64_t x_s;
+  const ST* w;  // [N][K], stride w_s
+  int64_t w_s;
+  const ST* bias;  // [N] or nullptr
+  ST* out;         // [M][N], stride out_s
+  int64_t out_s;
+  int32_t M, N, K;
+  int32_t mtiles, xm;
+};
+
+template <typename ST>
+__device__ static inline u32x2 pack4(const float* f) {
+  u32x2 v;
+  if constexpr (sizeof(ST) == 2 && __is_same(ST, bf16_t)) {
+    v.x = bf16_pair_bits(f[0], f[1]);
+    v.y = bf16_pair_bits(f[2], f[3]);
+  } else {
+    v.x = Tr<_Float16>::two(f);
+    v.y = Tr<_Float16>::two(f + 2);
+  }
+  return v;
+}
+
+template <int EPI>
+__device__ static inline float epi_act(float v) {
+  if constexpr (EPI == kEpiSilu) return v / (1.f + __expf(-v));
+  return v;
+}
+
+// Tile (m, n) of workgroup i: workgroup i runs on XCD i % 8.  xm > 0: the XCDs
+// take an xm x 8/xm grid of equal blocks of tiles (the host picks xm so that a
+// block's rows and weight columns together are fewest: what each XCD's L2
+// fetches); xm == 0 (the tiles do not divide): contiguous runs, rows fastest.
+__device__ static inline void xcd_tile(int i, int total, int mtiles, int xm, int& m, int& n) {
+  const int x = i & 7, j = i >> 3;
+  if (xm > 0) {
+    const int ml = mtiles / xm, nl = total / mtiles / (8 / xm);
+    m = (x % xm) * ml + j % ml;
+    n = (x / xm) * nl + j / ml;
+    return;
+  }
+  const int q = total >> 3, r = total & 7;
+  const int t = x * q + min(x, r) + j;
+  m = t % mtiles;
+  n = t / mtiles;
+}
+
+// Bound by latency: the launch, one round trip to memory and the waves' sum; 16
+// rows x 512 -> 512 outputs takes 3.4 us in a graph (2.6 us of it the launch and
+// the round trip) against 4.2 for torch's library GEMM, 60 rows 3.4 against 6.1.
+// An operand read touches 16 rows x 64 bytes, half of each 128-byte line, which
+// limits a CU to about 37 GB/s: larger tiles take lin_tile_kernel.
+//
+// One workgroup: 16*MT rows x 16*NT outputs; wave w multiplies columns
+// [w K/NW, (w+1) K/NW) of both operands and the waves' partial sums are added
+// in LDS in wave order.  W is the product's A operand (its rows the 16 M rows)
+// and x the B operand, so a lane ends with 4 consecutive outputs of one row.
+template <typename ST, int MT, int NT, int NW, int EPI>
+__global__ void __launch_bounds__(64 * NW) lin_row_kernel(const LinK<ST> p) {
+#pragma clang fp contract(off)
+  constexpr int ROWS = 16 * MT;
+  constexpr int kRed = NW * MT * NT * 64 * 16;
+  __shared__ __align__(16) unsigned char smem[kRed];
+
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int l16 = lane & 15, kg = lane >> 4;
+  int mt_i, nt_i;
+  xcd_tile(blockIdx.x, gridDim.x, p.mtiles, p.xm, mt_i, nt_i);
+  const int row0 = mt_i * ROWS, n0 = nt_i * 16 * NT;
+
+  f32x4_t acc[MT][NT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[m][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  constexpr int UK = 4;  // 32-column steps a chunk
+  const int kw = p.K / NW;
+  const ST* wp[NT];
+  const ST* xp[MT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) wp[n] = p.w + (int64_t)(n0 + 16 * n + l16) * p.w_s + wave * kw + kg * 8;
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+    xp[m] = p.x + (int64_t)min(row0 + 16 * m + l16, p.M - 1) * p.x_s + wave * kw + kg * 8;
+  u32x4 wf[2][UK][NT], xf[2][UK][MT];
+  auto load = [&](int b, int k) {
+#pragma unroll
+    for (int u = 0; u < UK; ++u) {
+#pragma unroll
+      for (int n = 0; n < NT; ++n) wf[b][u][n] = ld16(wp[n] + k + 32 * u);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) xf[b][u][m] = ld16(xp[m] + k + 32 * u);
+    }
+  };
+  auto mul = [&](int b) {
+#pragma unroll
+    for (int u = 0; u < UK; ++u)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[m][n] = MmaL<ST>::k32(wf[b][u][n], xf[b][u][m], acc[m][n]);
+  };
+  // two chunks in registers: the next one's loads are in flight during a chunk's products
+  load(0, 0);
+  for (int k = 0; k < kw; k += 64 * UK) {
+    if (k + 32 * UK < kw) load(1, k + 32 * UK);
+    __builtin_amdgcn_sched_barrier(0);
+    mul(0);
+    if (k + 64 * UK < kw) load(0, k + 64 * UK);
+    __builtin_amdgcn_sched_barrier(0);
+    if (k + 32 * UK < kw) mul(1);
+  }
+  f32x4_t* const red = reinterpret_cast<f32x4_t*>(smem);  // [NW][MT*NT][64]
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) red[((wave * MT + m) * NT + n) * 64 + lane] = acc[m][n];
+  __syncthreads();
+  for (int i = threadIdx.x; i < MT * NT * 64; i += 64 * NW) {
+    f32x4_t s = red[i];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) s += red[w * MT * NT * 64 + i];
+    const int il = i & 63, t = i >> 6;
+    const int row = row0 + 16 * (t / NT) + (il & 15);
+    const int n = n0 + 16 * (t % NT) + 4 * (il >> 4);
+    float f[4] = {s.x, s.y, s.z, s.w};
+    if (p.bias) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f[e] += from_st(p.bias[n + e]);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f[e] = epi_act<EPI>(f[e]);
+    if (row < p.M) *reinterpret_cast<u32x2*>(p.out + (int64_t)row * p.out_s + n) = pack4<ST>(f);
+  }
+}
+
+// `bytes` readable from base; a read past them gives zeros
+__device__ static inline __amdgpu_buffer_rsrc_t bytes_rsrc(const void* base, uint32_t bytes) {
+  // word 3 0x00020000: 32-bit data format, the setting untyped loads need on CDNA
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);
+}
+
+// 16 bytes a lane to lds + 16 lane (lds wave-uniform)
+__device__ static inline void load_lds16(const __amdgpu_buffer_rsrc_t r, unsigned char* lds, uint32_t off, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, off, soff, 0, 0);
+}
+
+// vmcnt(n): at most n of the wave's memory reads still in flight
+template <int N>
+__device__ static inline void wait_vm() {
+  __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N & 0x30) << 10));
+}
+
+// Many rows: BM x BN outputs a workgroup, WM x WN x WK waves, both operands
+// staged in LDS BK columns a stage (S stages in flight, buffer loads straight to
+// LDS).  A row's 16-byte chunks are permuted within each 128 bytes by the row's
+// low three bits, so the 16 rows of an operand read fall on distinct banks.
+// Small tiles split K over the waves (WK): each staged byte is then read from LDS
+// once or twice, and the sum over the waves costs one exchange at the end.
+// Bound by: latency up to about one tile a CU (128 x 512 -> 2048 with SiLU 4.5 us,
+// torch's GEMM and SiLU 10.2); LDS reads on the large forms (128 x 128 tiles take
+// 0.53 us a stage, of which 0.41 remain with the loads left out and 0.27 with the
+// products left out).  840 x 1024 -> 4096 with SiLU 13.6 us (518 TFLOP/s) against
+// 21.3, 840 x 4096 -> 1024 17.1 against 19.5 for torch's.
+template <typename ST, int BM, int BN, int WM, int WN, int WK, int BK, int S, int EPI>
+__global__ void __launch_bounds__(64 * WM * WN * WK) lin_tile_kernel(const LinK<ST> p) {
+#pragma clang fp contract(off)
+  constexpr int NW = WM * WN * WK;
+  constexpr int TM = BM / WM / 16, TN = BN / WN / 16;  // 16x16 products a wave
+  constexpr int CH = BK / 8;                           // 16-byte chunks a row
+  constexpr int kStage = (BM + BN) * BK * 2;
+  constexpr int LPS = kStage / 1024 / NW;  // loads a wave issues a stage
+  static_assert(BK % 64 == 0, "the permutation stays within a row's stage: whole groups of 8 chunks");
+  static_assert(kStage % (1024 * NW) == 0 && (BM * CH) % 64 == 0, "whole waves of chunks");
+  constexpr int KS = BK / 32 / WK;  // 32-column steps a wave does a stage
+  constexpr int OS = BN + 8;        // LDS row stride of the staged output
+  constexpr int kOut = BM * OS * 2;
+  constexpr int kRed = WK > 1 ? (WK - 1) * BM * BN * 4 : 0;
+  constexpr int kSmem = S * kStage > kOut + kRed ? S * kStage : kOut + kRed;
+  __shared__ __align__(16) unsigned char smem[kSmem];
+
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, kg = lane >> 4;
+  const int wk = wave / (WM * WN), wm = (wave / WN) % WM, wn = wave % WN;
+  int mt_i, nt_i;
+  xcd_tile(blockIdx.x, gridDim.x, p.mtiles, p.xm, mt_i, nt_i);
+  const int row0 = mt_i * BM, n0 = nt_i * BN;
+
+  // chunk c of a stage: row c / CH of [x rows ; w rows], LDS position c % CH
+  const __amdgpu_buffer_rsrc_t rx = bytes_rsrc(p.x, (uint32_t)((p.M - 1) * p.x_s + p.K) * 2u);
+  const __amdgpu_buffer_rsrc_t rw = bytes_rsrc(p.w, (uint32_t)((p.N - 1) * p.w_s + p.K) * 2u);
+  uint32_t off[LPS];
+#pragma unroll
+  for (int i = 0; i < LPS; ++i) {
+    const int c = (i * NW + wave) * 64 + lane;
+    const int r = c / CH, pos = c % CH;
+    const int ch = (pos & ~7) | ((pos ^ r) & 7);
+    off[i] = r < BM ? (uint32_t)(min(row0 + r, p.M - 1) * p.x_s + ch * 8) * 2u
+                    : (uint32_t)((n0 + r - BM) * p.w_s + ch * 8) * 2u;
+  }
+  auto issue = [&](int st, int k) {
+#pragma unroll
+    for (int i = 0; i < LPS; ++i) {
+      const int base = (i * NW + wave) * 64;  // wave-uniform: whole waves of one operand
+      load_lds16(base < BM * CH ? rx : rw, smem + st * kStage + base * 16, off[i], k * 2);
+    }
+  };
+  f32x4_t acc[TM][TN];
+#pragma unroll
+  for (int m = 0; m < TM; ++m)
+#pragma unroll
+    for (int n = 0; n < TN; ++n) acc[m][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  const int iters = p.K / BK;
+#pragma unroll
+  for (int s = 0; s < S - 1; ++s)
+    if (s < iters) issue(s, s * BK);
+  int st = 0;
+  for (int it = 0; it < iters; ++it) {
+    // this stage's loads are in; the later stages' may still be in flight
+    if (it + S - 2 < iters)
+      wait_vm<(S - 2) * LPS>();
+    else
+      wait_vm<0>();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();  // every wave's part of the stage; the slot refilled below is read by none
+    asm volatile("" ::: "memory");
+    if (it + S - 1 < iters) issue(st == 0 ? S - 1 : st - 1, (it + S - 1) * BK);
+    const unsigned char* xs = smem + st * kStage;
+    const unsigned char* ws = xs + BM * BK * 2;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int ch = (wk * KS + s) * 4 + kg;
+      u32x4 xf[TM], wf[TN];
+#pragma unroll
+      for (int m = 0; m < TM; ++m) {
+        const int r = (wm * TM + m) * 16 + l16;
+        xf[m] = *reinterpret_cast<const u32x4*>(xs + r * BK * 2 + ((ch & ~7) | ((ch ^ r) & 7)) * 16);
+      }
+#pragma unroll
+      for (int n = 0; n < TN; ++n) {
+        const int r = (wn * TN + n) * 16 + l16;
+        wf[n] = *reinterpret_cast<const u32x4*>(ws + r * BK * 2 + ((ch & ~7) | ((ch ^ r) & 7)) * 16);
+      }
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int n = 0; n < TN; ++n) acc[m][n] = MmaL<ST>::k32(wf[n], xf[m], acc[m][n]);
+    }
+    st = st == S - 1 ? 0 : st + 1;
+  }
+  __syncthreads();
+  // the K halves' sums meet in LDS
+  if constexpr (WK > 1) {
+    f32x4_t* const red = reinterpret_cast<f32x4_t*>(smem + kOut);
+    if (wk > 0) {
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int n = 0; n < TN; ++n) red[((wave - WM * WN) * TM * TN + m * TN + n) * 64 + lane] = acc[m][n];
+    }
+    __syncthreads();
+    if (wk == 0) {
+#pragma unroll
+      for (int w = 1; w < WK; ++w)
+#pragma unroll
+        for (int m = 0; m < TM; ++m)
+#pragma unroll
+          for (int n = 0; n < TN; ++n) acc[m][n] += red[((wave + (w - 1) * WM * WN) * TM * TN + m * TN + n) * 64 + lane];
+    }
+  }
+  // through LDS to whole 16-byte chunks of a row
+  ST* const os = reinterpret_cast<ST*>(smem);
+  if (wk == 0) {
+#pragma unroll
+    for (int n = 0; n < TN; ++n) {
+      const int c = (wn * TN + n) * 16 + kg * 4;
+      float b[4] = {0.f, 0.f, 0.f, 0.f};
+      if (p.bias) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) b[e] = from_st(p.bias[n0 + c + e]);
+      }
+#pragma unroll
+      for (int m = 0; m < TM; ++m) {
+        float f[4] = {acc[m][n].x, acc[m][n].y, acc[m][n].z, acc[m][n].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f[e] = epi_act<EPI>(f[e] + b[e]);
+        *reinterpret_cast<u32x2*>(os + ((wm * TM + m) * 16 + l16) * OS + c) = pack4<ST>(f);
+      }
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < BM * BN / 8; i += 64 * NW) {
+    const int r = i / (BN / 8), c = (i % (BN / 8)) * 8;
+    if (row0 + r < p.M) st16(p.out + (int64_t)(row0 + r) * p.out_s + n0 + c, *reinterpret_cast<const u32x4*>(os + r * OS + c));
+  }
+}
+
+namespace {
+
+// the split of the XCDs over rows (see xcd_tile)
+int xcd_split(int mtiles, int ntiles, int bm, int bn) {
+  int best = 0;
+  int64_t cost = 0;
+  for (int xm = 1; xm <= 8; xm *= 2) {
+    if (mtiles % xm != 0 || ntiles % (8 / xm) != 0) continue;
+    const int64_t c = (int64_t)(mtiles / xm) * bm + (int64_t)(ntiles / (8 / xm)) * bn;
+    if (best == 0 || c < cost) {
+      best = xm;
+      cost = c;
+    }
+  }
+  return best;
+}
+
+template <typename ST>
+dim3 tile_grid(LinK<ST>& k, int bm, int bn) {
+  k.mtiles = (k.M + bm - 1) / bm;
+  k.xm = xcd_split(k.mtiles, k.N / bn, bm, bn);
+  return dim3((unsigned)(k.mtiles * (k.N / bn)));
+}
+
+template <typename ST, int BM, int BN, int WM, int WN, int WK, int BK, int S, int EPI>
+int launch_tile(LinK<ST> k, hipStream_t s) {
+  const dim3 grid = tile_grid(k, BM, BN);
+  hipLaunchKernelGGL((lin_tile_kernel<ST, BM, BN, WM, WN, WK, BK, S, EPI>), grid, dim3(64 * WM * WN * WK), 0, s, k);
+  return check_launch("pk_linear");
+}
+
+template <typename ST, int MT, int NT, int NW, int EPI>
+int launch_row(LinK<ST> k, hipStream_t s) {
+  const dim3 grid = tile_grid(k, 16 * MT, 16 * NT);
+  hipLaunchKernelGGL((lin_row_kernel<ST, MT, NT, NW, EPI>), grid, dim3(64 * NW), 0, s, k);
+  return check_launch("pk_linear");
+}
+
+// The forms without a prologue and what a launch of each takes, fitted to launches
+// in a graph with cold weights (K 512 - 4096, 16 - 3584 rows, bf16): `a` us plus `s`
+// us a 1024 columns for workgroups that are alone on their CU, 0.8 s for each
+// further one resident with it (`occ` fit), and again a - 2 for each further
+// round.  Small tiles read more bytes an output but put more CUs on a short
+// launch; the large ones are bound by LDS reads (a 64x32 wave tile reads 6 KB
+// for 8 products).  The cheapest by this model is launched; at the measured
+// shapes it is the fastest form or within 5% of it.
+struct Form {
+  int bm, bn, kmul, occ;
+  float a, s;
+};
+constexpr Form kForms[] = {
+    {16, 16, 512, 4, 2.6f, 1.75f},    // lin_row_kernel
+    {16, 32, 256, 1, 3.45f, 0.97f},   //
+    {16, 32, 128, 2, 3.1f, 1.43f},    //
+    {32, 32, 128, 1, 3.0f, 1.9f},     //
+    {32, 32, 256, 1, 3.75f, 1.36f},   //
+    {32, 64, 128, 1, 3.3f, 2.6f},     //
+    {32, 64, 128, 1, 4.0f, 2.03f},    //
+    {64, 64, 64, 2, 3.75f, 3.35f},    //
+    {64, 128, 64, 2, 4.2f, 5.5f},     //
+    {128, 128, 64, 1, 5.0f, 8.5f},    //
+    {128, 128, 64, 2, 5.7f, 9.1f},    //
+    {256, 256, 64, 1, 10.0f, 28.0f},  //
+};
+constexpr int kNumForms = sizeof(kForms) / sizeof(kForms[0]);
+
+// us of a launch in form f, or a negative number where it does not fit
+float form_cost(const Form& f, int64_t M, int64_t N, int64_t K, int cus) {
+  if (N % f.bn != 0 || K % f.kmul != 0) return -1.f;
+  const int64_t tiles = (M + f.bm - 1) / f.bm * (N / f.bn);
+  const int64_t per = (tiles + cus - 1) / cus, rounds = (per + f.occ - 1) / f.occ;
+  const float c = f.s * (float)K / 1024.f;
+  return f.a + (float)(rounds - 1) * (f.a - 2.f) + (float)rounds * c + 0.8f * c * (float)(per - rounds);
+}
+
+int best_form(int64_t M, int64_t N, int64_t K, int cus) {
+  int best = -1;
+  float cost = 0.f;
+  for (int i = 0; i < kNumForms; ++i) {
+    const float c = form_cost(kForms[i], M, N, K, cus);
+    if (c >= 0.f && (best < 0 || c < cost)) {
+      best = i;
+      cost = c;
+    }
+  }
+  return best;
+}
+
+template <typename ST, int EPI>
+int launch_form(const LinK<ST>& k, int form, hipStream_t s) {
+  switch (form) {
+    case 0: return launch_row<ST, 1, 1, 4, EPI>(k, s);
+    case 1: return launch_tile<ST, 16, 32, 1, 1, 8, 256, 5, EPI>(k, s);
+    case 2: return launch_tile<ST, 16, 32, 1, 1, 4, 128, 6, EPI>(k, s);
+    case 3: return launch_tile<ST, 32, 32, 2, 2, 2, 128, 6, EPI>(k, s);
+    case 4: return launch_tile<ST, 32, 32, 1, 1, 8, 256, 4, EPI>(k, s);
+    case 5: return launch_tile<ST, 32, 64, 2, 2, 2, 128, 5, EPI>(k, s);
+    case 6: return launch_tile<ST, 32, 64, 1, 2, 4, 128, 5, EPI>(k, s);
+    case 7: return launch_tile<ST, 64, 64, 2, 2, 2, 64, 4, EPI>(k, s);
+    case 8: return launch_tile<ST, 64, 128, 2, 4, 1, 64, 3, EPI>(k, s);
+    case 9: return launch_tile<ST, 128, 128, 2, 4, 1, 64, 4, EPI>(k, s);
+    case 10: return launch_tile<ST, 128, 128, 2, 2, 1, 64, 2, EPI>(k, s);
+    default: return launch_tile<ST, 256, 256, 2, 4, 1, 64, 2, EPI>(k, s);
+  }
+}
+
+bool row_ok(int64_t rows, int64_t stride, int64_t width) {
+  return stride >= 0 && stride % 8 == 0 && (rows <= 1 || stride >= width) &&
+         (rows - 1) * stride + width < (int64_t{1} << 31);
+}
+
+template <typename ST>
+int linear_typed(const pk_linear_args* a, hipStream_t s) {
+  const char* what = "pk_linear";
+  if (a->rows < 0) return fail(PK_ERR_INVALID, "%s: rows %d < 0", what, a->rows);
+  if (a->n <= 0 || a->n % 64 != 0 || a->k <= 0 || a->k % 256 != 0)
+    return fail(PK_ERR_UNSUPPORTED, "%s: n %d must be a multiple of 64 and k %d of 256", what, a->n, a->k);
+  if (a->activation != PK_ACT_NONE && a->activation != PK_ACT_SILU)
+    return fail(PK_ERR_INVALID, "%s: unknown activation %d", what, a->activation);
+  if (a->rows == 0) return PK_OK;
+  const void* ptrs[4] = {a->x, a->weight, a->out, a->bias ? a->bias : a->weight};
+  for (const void* q : ptrs) {
+    if (!q) return fail(PK_ERR_INVALID, "%s: a tensor pointer is NULL", what);
+    if (!aligned16(q)) return fail(PK_ERR_INVALID, "%s: tensors must be 16-byte aligned", what);
+  }
+  if (!row_ok(a->rows, a->x_stride, a->k) || !row_ok(a->n, a->weight_stride, a->k) ||
+      !row_ok(a->rows, a->out_stride, a->n))
+    return fail(PK_ERR_INVALID, "%s: row strides must be multiples of 8 elements, at least the row, and a tensor below "
+                "2^31 elements", what);
+  LinK<ST> k{};
+  k.x = static_cast<const ST*>(a->x);
+  k.x_s = a->x_stride;
+  k.w = static_cast<const ST*>(a->weight);
+  k.w_s = a->weight_stride;
+  k.bias = static_cast<const ST*>(a->bias);
+  k.out = static_cast<ST*>(a->out);
+  k.out_s = a->out_stride;
+  k.M = a->rows;
+  k.N = a->n;
+  k.K = a->k;
+  DeviceGuard dg(a->device);
+  if (!dg.ok) return fail(PK_ERR_HIP, "%s: cannot select device %d", what, a->device);
+  const int form = best_form(k.M, k.N, k.K, cu_count());
+  if (a->activation == PK_ACT_SILU) return launch_form<ST, kEpiSilu>(k, form, s);
+  return launch_form<ST, kEpiNone>(k, form, s);
+}
+
+int linear_any(const pk_linear_args* a, hipStream_t s) {
+  switch (a->dtype) {
+    case PK_DTYPE_F16: return linear_typed<_Float16>(a, s);
+    case PK_DTYPE_BF16: return linear_typed<bf16_t>(a, s);
+    case PK_DTYPE_F32: return fail(PK_ERR_UNSUPPORTED, "pk_linear: fp16 and bf16 only");
+    default: return fail(PK_ERR_INVALID, "pk_linear: unknown dtype %d", a->dtype);
+  }
+}
+
+}  // namespace
+}  // namespace pk
+
+extern "C" int pk_linear(const pk_linear_args* args, int32_t count, void* stream) {
+  pk::clear_error();
+  if (!args) return pk::fail(PK_ERR_INVALID, "pk_linear: args is NULL");
+  if (count < 0) return pk::fail(PK_ERR_INVALID, "pk_linear: count %d < 0", count);
+  for (int32_t i = 0; i < count; ++i) {
+    const int rc = pk::linear_any(args + i, static_cast<hipStream_t>(stream));
+    if (rc != PK_OK) return rc;
+  }
+  return PK_OK;
+}

@@ -15,7 +15,7 @@ from pathlib import Path
 LIB_NAME = "libparakeet_paged.so"
 LIB_PATH = Path(__file__).resolve().parent / LIB_NAME
 
-ABI_VERSION = 9
+ABI_VERSION = 10
 
 DTYPE_F32 = 0
 DTYPE_F16 = 1
@@ -27,6 +27,9 @@ PK_ERR_UNSUPPORTED = -2
 PK_ERR_EXHAUSTED = -3
 PK_ERR_HIP = -4
 PK_ERR_STATE = -5
+
+ACT_NONE = 0
+ACT_SILU = 1
 
 PCM_S16 = 0
 PCM_F32 = 1
@@ -194,6 +197,24 @@ class ResNormArgs(ctypes.Structure):
     ]
 
 
+class LinearArgs(ctypes.Structure):
+    _fields_ = [
+        ("dtype", c_int32),
+        ("device", c_int32),
+        ("rows", c_int32),
+        ("n", c_int32),
+        ("k", c_int32),
+        ("activation", c_int32),
+        ("x", c_void_p),
+        ("x_stride", c_int64),
+        ("weight", c_void_p),
+        ("weight_stride", c_int64),
+        ("bias", c_void_p),
+        ("out", c_void_p),
+        ("out_stride", c_int64),
+    ]
+
+
 class FeStream(ctypes.Structure):
     _fields_ = [
         ("slot", c_int32),
@@ -322,6 +343,7 @@ SIGNATURES = {
     "pk_streaming_mask": (c_int, [POINTER(MaskArgs), c_void_p]),
     "pk_conv_step": (c_int, [POINTER(ConvArgs), c_void_p]),
     "pk_residual_norm": (c_int, [POINTER(ResNormArgs), c_void_p]),
+    "pk_linear": (c_int, [POINTER(LinearArgs), c_int32, c_void_p]),
     "pk_fe_step": (c_int, [POINTER(FeArgs), c_void_p]),
     "pk_subsample": (c_int, [POINTER(SubArgs), c_void_p]),
     "pk_rnnt_workspace_bytes": (c_int64, [c_int32, c_int32, c_int32, c_int32, c_int32]),

@@ -117,7 +117,7 @@ class ConformerAttention(nn.Module):
 
     def forward(self, x: Tensor, pos_emb: Tensor, attn_mask: Tensor, cache: ModelCache = None):
         B, T = x.shape[:2]
-        qkv = self.qkv(x)
+        qkv = ops.module_linear(x, self.qkv)
         query, key, value = qkv.chunk(3, dim=-1)
         # [1, P, D] is one table for every stream; [B, P, D] gives each stream
         # its own (the reference broadcasts both, attention.py:102-106)
@@ -135,7 +135,7 @@ class ConformerAttention(nn.Module):
             out = ops.paged_relpos_attn(
                 query, key, value, pos, bias_u, bias_v, mask, num_heads=self.num_heads, left=0, pages=None, append=False
             )
-        return self.linear_out(out.reshape(B, T, self.num_heads * self.d_k))
+        return ops.module_linear(out.reshape(B, T, self.num_heads * self.d_k), self.linear_out)
 
 
 __all__ = ["ConformerAttention", "PositionalEncoding"]

@@ -47,7 +47,23 @@ class ConformerFeedForward(nn.Module):
         self.dropout = nn.Dropout(dropout)
 
     def forward(self, x: Tensor) -> Tensor:
-        return self.linear2(self.dropout(self.activation(self.linear1(x))))
+        # linear1 with its SiLU is one launch where the library takes it
+        l1, l2 = self.linear1, self.linear2
+        if self._fused() and ops.linear_applies(x, l1.weight, l1.bias, silu=True):
+            rows = x.numel() // x.shape[-1]
+            if ops.plain_module(l2, nn.Linear) and ops.layer_applies(x.dtype, x.device, rows, l2.weight, l2.bias):
+                return ops.feed_forward(x, l1.weight, l1.bias, l2.weight, l2.bias)
+            return l2(ops.linear(x, l1.weight, l1.bias, silu=True))
+        return l2(self.dropout(self.activation(l1(x))))
+
+    def _fused(self) -> bool:
+        drop = self.dropout
+        return (
+            ops.plain_module(self.linear1, nn.Linear)
+            and ops.plain_module(self.activation, nn.SiLU)
+            and ops.plain_module(drop, nn.Dropout)
+            and not (drop.training and drop.p > 0.0)
+        )
 
 
 class CausalConv1d(nn.Conv1d):
@@ -98,7 +114,7 @@ class ConformerConvolution(nn.Module):
         )
 
     def forward(self, x: Tensor, pad_mask: Tensor, cache=None):
-        h = F.linear(x, self.pointwise_conv1.weight.squeeze(-1), self.pointwise_conv1.bias)
+        h = ops.functional_linear(x, self.pointwise_conv1.weight.squeeze(-1), self.pointwise_conv1.bias)
         if isinstance(cache, ConvCacheRef):
             bn, dw = self.batch_norm, self.depthwise_conv
             y = cache.cache.conv_step(cache.layer_idx, h, pad_mask, dw.weight, dw.bias, bn.weight, bn.bias, bn.eps)
@@ -111,7 +127,7 @@ class ConformerConvolution(nn.Module):
                 frames = cache.transpose(1, 2).unsqueeze(1).contiguous()
             y = self._middle(h, pad_mask, frames)
             new_cache = frames[:, 0].transpose(1, 2)
-        out = F.linear(y, self.pointwise_conv2.weight.squeeze(-1), self.pointwise_conv2.bias)
+        out = ops.functional_linear(y, self.pointwise_conv2.weight.squeeze(-1), self.pointwise_conv2.bias)
         return out, new_cache
 
 

@@ -14,7 +14,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from ._lib import AttnArgs, ConvArgs, FeArgs, KvAppendArgs, KvGatherArgs, MaskArgs, PagedLayout, ResNormArgs, SubArgs, check, lib
+from ._lib import AttnArgs, ConvArgs, FeArgs, KvAppendArgs, KvGatherArgs, LinearArgs, MaskArgs, PagedLayout, ResNormArgs, SubArgs, check, lib
 
 _DTYPES = {
     torch.float32: _lib.DTYPE_F32,
@@ -517,6 +517,132 @@ def residual_norm(
 
 # ---------------------------------------------------------------------------
 # pre-encode front end
+
+
+def _transformed(x: torch.Tensor) -> bool:
+    """Whether something follows or rewrites the torch calls made on ``x``
+    (autocast, tracing, compilation, function transforms, forward-mode
+    derivatives, dispatch modes): a kernel call would pass it by."""
+    return (
+        type(x) not in (torch.Tensor, torch.nn.Parameter)
+        or torch.is_autocast_enabled("cuda")
+        or torch.compiler.is_compiling()
+        or torch.jit.is_tracing()
+        or torch._C._functorch.is_functorch_wrapped_tensor(x)
+        or torch.autograd.forward_ad._current_level >= 0
+        or torch._C._len_torch_dispatch_stack() > 0
+        or torch._C._len_torch_function_stack() > 0
+    )
+
+
+def plain_module(m: torch.nn.Module, cls: type) -> bool:
+    """Whether calling ``m`` is exactly ``cls.forward`` on its own parameters:
+    no subclass, replaced forward or forward hook that a kernel call would skip."""
+    mod = torch.nn.modules.module
+    return (
+        type(m) is cls
+        and "forward" not in m.__dict__
+        and not m._forward_hooks
+        and not m._forward_pre_hooks
+        and not mod._global_forward_hooks
+        and not mod._global_forward_pre_hooks
+    )
+
+
+# past this many products torch's library GEMM is at least as fast as pk_linear:
+# 840 x 1024 x 4096 17.3 us against 19.1, 1792 x 1024 x 4096 27.6 against 27.6,
+# 3584 x 1024 x 4096 39.8 against 39.5, 3584 x 3072 x 1024 37 against 27.
+# With SiLU (fused here, a launch of its own there) it never is in the measured
+# range: 3584 x 4096 x 1024 40 against 46, 4096 x 2048 x 512 16.2 against 27.3
+_LINEAR_PRODUCTS = 4_500_000_000
+
+
+def layer_applies(dtype: torch.dtype, device: torch.device, rows: int, weight: torch.Tensor, bias: torch.Tensor | None, silu: bool = False) -> bool:
+    """Whether :func:`linear` takes a layer on ``rows`` rows of ``dtype``, and is
+    the faster way to run it."""
+    if type(weight) not in (torch.Tensor, torch.nn.Parameter) or weight.dtype != dtype or weight.device != device:
+        return False
+    n, k = weight.shape
+    if n % 64 or k % 256 or n == 0 or k == 0 or rows == 0:
+        return False
+    ld = weight.stride(0)
+    if weight.stride(1) != 1 or ld % 8 or ld < k or weight.data_ptr() % 16:
+        return False
+    if max((n - 1) * ld + k, rows * k, rows * n) >= 1 << 31:
+        return False
+    if bias is not None and (bias.dtype != dtype or bias.device != device or not bias.is_contiguous() or bias.data_ptr() % 16):
+        return False
+    if not silu and rows * n * k > _LINEAR_PRODUCTS:
+        return False
+    return not (torch.is_grad_enabled() and (weight.requires_grad or (bias is not None and bias.requires_grad)))
+
+
+def linear_applies(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, silu: bool = False) -> bool:
+    """Whether :func:`linear` takes this call, and is the faster way to run it;
+    otherwise the caller runs torch's own linear, which takes every form."""
+    if x.dtype not in (torch.float16, torch.bfloat16) or x.device.type != "cuda" or x.dim() == 0:
+        return False
+    k = x.shape[-1]
+    if weight.dim() != 2 or weight.shape[1] != k or (torch.is_grad_enabled() and x.requires_grad) or _transformed(x):
+        return False
+    return k > 0 and layer_applies(x.dtype, x.device, x.numel() // k, weight, bias, silu)
+
+
+def _linear_args(a: LinearArgs, code: int, dev: torch.device, x: torch.Tensor, rows: int, weight, bias, out, silu: bool) -> None:
+    n, k = weight.shape
+    a.dtype, a.device = code, dev.index
+    a.rows, a.n, a.k = rows, n, k
+    a.activation = _lib.ACT_SILU if silu else _lib.ACT_NONE
+    a.x, a.x_stride = x.data_ptr(), k
+    a.weight, a.weight_stride = weight.data_ptr(), weight.stride(0)
+    a.bias = bias.data_ptr() if bias is not None else None
+    a.out, a.out_stride = out.data_ptr(), n
+
+
+def _aligned_rows(x: torch.Tensor) -> torch.Tensor:
+    x = x.contiguous()
+    return x if x.data_ptr() % 16 == 0 else x.clone()
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None, *, silu: bool = False) -> torch.Tensor:
+    """``x @ weight.T + bias``, and SiLU of it, in one launch, for layers that
+    :func:`linear_applies` accepts (feedforward.py:20-26, attention.py:92,122)."""
+    x = _aligned_rows(x)
+    n, k = weight.shape
+    out = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
+    a = LinearArgs()
+    _linear_args(a, _DTYPES[x.dtype], x.device, x, x.numel() // k, weight, bias, out, silu)
+    check(lib().pk_linear(ctypes.byref(a), 1, _stream(x.device)), "pk_linear")
+    return out
+
+
+def module_linear(x: torch.Tensor, m: torch.nn.Module) -> torch.Tensor:
+    """``m(x)`` of a torch ``Linear``: :func:`linear` where it applies."""
+    if plain_module(m, torch.nn.Linear) and linear_applies(x, m.weight, m.bias):
+        return linear(x, m.weight, m.bias)
+    return m(x)
+
+
+def functional_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
+    """``torch.nn.functional.linear``: :func:`linear` where it applies."""
+    if linear_applies(x, weight, bias):
+        return linear(x, weight, bias)
+    return torch.nn.functional.linear(x, weight, bias)
+
+
+def feed_forward(x: torch.Tensor, w1: torch.Tensor, b1: torch.Tensor | None, w2: torch.Tensor, b2: torch.Tensor | None) -> torch.Tensor:
+    """``linear2(SiLU(linear1(x)))`` (feedforward.py:20-26), for two layers that
+    :func:`linear_applies` accepts: two launches, one call."""
+    x = _aligned_rows(x)
+    rows = x.numel() // w1.shape[1]
+    h = torch.empty((rows, w1.shape[0]), dtype=x.dtype, device=x.device)
+    out = torch.empty((*x.shape[:-1], w2.shape[0]), dtype=x.dtype, device=x.device)
+    a = (LinearArgs * 2)()
+    code = _DTYPES[x.dtype]
+    _linear_args(a[0], code, x.device, x, rows, w1, b1, h, True)
+    _linear_args(a[1], code, x.device, h, rows, w2, b2, out, False)
+    check(lib().pk_linear(a, 2, _stream(x.device)), "pk_linear")
+    return out
 
 
 @dataclass

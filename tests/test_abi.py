@@ -219,3 +219,25 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
         ops.residual_norm(x, x, w, w, alpha=0.5)
     with pytest.raises(ValueError, match="must match"):
         ops.residual_norm(x, x[:, :4], w, w)
+
+
+def test_linear_args_validated_before_launch():
+    L = _lib.lib()
+    assert [f[0] for f in _lib.LinearArgs._fields_] == _struct_fields("pk_linear_args")
+    a = _lib.LinearArgs()
+    assert L.pk_linear(None, 1, None) == _lib.PK_ERR_INVALID
+    a.dtype, a.rows, a.n, a.k = _lib.DTYPE_F16, 4, 512, 512
+    a.x_stride = a.weight_stride = a.out_stride = 512
+    assert L.pk_linear(ctypes.byref(a), 1, None) == _lib.PK_ERR_INVALID  # NULL tensors
+    assert "NULL" in _lib.last_error()
+    a.n = 500
+    assert L.pk_linear(ctypes.byref(a), 1, None) == _lib.PK_ERR_UNSUPPORTED
+    a.n, a.k = 512, 384
+    assert L.pk_linear(ctypes.byref(a), 1, None) == _lib.PK_ERR_UNSUPPORTED
+    a.k, a.activation = 512, 9
+    assert L.pk_linear(ctypes.byref(a), 1, None) == _lib.PK_ERR_INVALID
+    a.activation, a.dtype = 0, _lib.DTYPE_F32
+    assert L.pk_linear(ctypes.byref(a), 1, None) == _lib.PK_ERR_UNSUPPORTED
+    a.dtype, a.rows = _lib.DTYPE_BF16, 0  # nothing to do: no pointer is read
+    assert L.pk_linear(ctypes.byref(a), 1, None) == _lib.PK_OK
+    assert L.pk_linear(ctypes.byref(a), 0, None) == _lib.PK_OK

@@ -1,0 +1,110 @@
+"""pk_linear and the layers that take it against float64 (feedforward.py:20-26,
+attention.py:92,122, convolution.py:152,158).
+
+The bound: operands are exact 16-bit values, products accumulate in fp32 (K
+terms: relative 2^-24 sqrt(K) of the sum of magnitudes, far below one rounding),
+and each output is rounded once, relative 2^-11 (fp16) or 2^-8 (bf16).  Held at
+1.05 roundings of the value plus the accumulation's 2^-24 K |x||w|.  SiLU adds
+the fp32 exponential's few 2^-23."""
+
+import math
+
+import pytest
+import torch
+import torch.nn.functional as F
+from torch import nn
+
+from parakeet_amd import ops
+from parakeet_amd.modules.encoder import ConformerFeedForward
+
+EPS = {torch.float16: 2.0**-11, torch.bfloat16: 2.0**-8}
+TINY = {torch.float16: 2.0**-24, torch.bfloat16: 2.0**-130}
+
+
+def _check(got, x, w, b, dtype, silu):
+    y = x.double() @ w.double().T + (b.double() if b is not None else 0.0)
+    mag = x.double().abs() @ w.double().abs().T
+    ref = F.silu(y) if silu else y
+    bar = 1.05 * EPS[dtype] * ref.abs() + 2.0**-22 * mag + TINY[dtype]
+    err = (got.double() - ref).abs()
+    assert bool((err <= bar).all()), (tuple(x.shape), tuple(w.shape), float((err - bar).max()))
+
+
+# every form of the launch rule, its edges: one row, a row short of and past a
+# tile, several tiles a CU; K of one stage and of many
+CASES = [
+    (1, 64, 512), (16, 512, 512), (17, 2048, 512), (2, 512, 2048), (33, 1024, 4096), (63, 1536, 768),
+    (65, 4096, 1024), (129, 512, 256), (255, 3072, 1024), (480, 1024, 4096), (840, 1024, 1024), (841, 2048, 1024),
+    (840, 4096, 1024), (1793, 1024, 1024), (4095, 512, 512), (1000, 64, 256), (4097, 2048, 512), (3600, 4096, 1024),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,n,k", CASES)
+def test_linear_matches_float64(cuda, dtype, rows, n, k):
+    print(f"\n[linear] {dtype} rows={rows} n={n} k={k}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(rows * 7 + n + k)
+    x = torch.randn(rows, k, generator=g, device=cuda).to(dtype)
+    w = (torch.randn(n, k, generator=g, device=cuda) / math.sqrt(k)).to(dtype)
+    b = torch.randn(n, generator=g, device=cuda).to(dtype)
+    for bias, silu in ((None, False), (b, True), (b, False)):
+        _check(ops.linear(x, w, bias, silu=silu), x, w, bias, dtype, silu)
+
+
+@pytest.mark.gpu
+def test_linear_reads_strided_weights_and_odd_views(cuda):
+    g = torch.Generator(device="cuda").manual_seed(1)
+    big = (torch.randn(128, 1024, generator=g, device=cuda) / 16).half()
+    w = big[:, 256:768]  # rows 1024 apart
+    x = torch.randn(3, 5, 1024, generator=g, device=cuda).half()[..., 1:513]  # neither contiguous nor aligned
+    assert ops.linear_applies(x, w, None)
+    _check(ops.linear(x, w).reshape(15, 128), x.reshape(15, 512), w, None, torch.float16, False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [(1, 1), (64, 2), (60, 14), (2100, 4)])
+def test_feed_forward_block(cuda, rows):
+    d, dtype = 512, torch.float16
+    print(f"\n[ff] {rows}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    with torch.device(cuda):
+        ff = ConformerFeedForward(d, 4 * d, 0.1, use_bias=True).to(dtype).eval().requires_grad_(False)
+    x = torch.randn(*rows, d, generator=g, device=cuda).to(dtype)
+    with torch.no_grad():
+        got = ff(x)
+    h = F.silu(F.linear(x.double(), ff.linear1.weight.double(), ff.linear1.bias.double()))
+    ref = F.linear(h, ff.linear2.weight.double(), ff.linear2.bias.double())
+    mag = h.abs() @ ff.linear2.weight.double().abs().T
+    # the hidden layer's rounding adds at most 2^-11 of each product's magnitude
+    assert bool(((got.double() - ref).abs() <= EPS[dtype] * (1.05 * ref.abs() + 1.1 * mag)).all())
+
+
+@pytest.mark.gpu
+def test_feed_forward_keeps_gradients_hooks_dropout_and_autocast(cuda):
+    """What a kernel call would pass by keeps torch's own path."""
+    with torch.device(cuda):
+        ff = ConformerFeedForward(512, 2048, 0.5).half()
+    x = torch.randn(4, 2, 512, device=cuda).half()
+    ff.train()
+    y = ff(x.requires_grad_())  # gradients
+    y.float().sum().backward()
+    assert x.grad is not None and ff.linear1.weight.grad is not None
+    with torch.no_grad():
+        assert not torch.equal(ff(x), ff(x))  # dropout draws
+        ff.eval()
+        seen = []
+        hook = ff.linear1.register_forward_hook(lambda m, i, o: seen.append(o.shape))
+        a = ff(x)
+        hook.remove()
+        assert seen == [torch.Size([4, 2, 2048])]
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert ff(x.float()).dtype == torch.bfloat16 and ff(x).dtype == torch.bfloat16
+        b = torch.func.vmap(ff)(x)
+        c = ff(x)
+        for t in (b, c):
+            assert float((t - a).abs().max()) <= 2.0**-8 * float(a.abs().max())
+        ff.linear2 = nn.Sequential(ff.linear2)
+        assert torch.equal(ff(x), ff.linear2(ops.linear(x, ff.linear1.weight, ff.linear1.bias, silu=True)))
+        f32 = ConformerFeedForward(512, 2048, 0.0).to(cuda).eval()
+        assert f32(x.float()).dtype == torch.float32
