@@ -309,13 +309,16 @@ int pk_conv_step(const pk_conv_args* args, void* stream);
  *   norm_out     = LayerNorm(residual_out) * ln_weight + ln_bias  (biased
  *                  variance, fp32 two-pass statistics over the channels of the
  *                  rounded residual_out, each output rounded once)
+ *   norm2_out    = LayerNorm(norm_out) * ln2_weight + ln2_bias with ln2_eps, where
+ *                  ln2_weight is not NULL (a layer's norm_out, and the next
+ *                  layer's norm_feed_forward1 of it, encoder.py:58-60,80)
  * Replaces, per layer, parakeet/modules/encoder.py:61,63,68,70,74,76,78,80: the
  * four `residual += ...` updates, the two `x * 0.5` scalings, and the LayerNorms
  * norm_self_att, norm_conv, norm_feed_forward2 and norm_out that read them.
  * residual, branch, residual_out, norm_out: [rows][d_model] of `dtype` with row
  * strides in elements (channels contiguous, 16-byte aligned rows);
- * residual_out may be residual (updated in place), norm_out may be branch; no
- * other overlap.  ln_weight, ln_bias: [d_model].  d_model a multiple of 8
+ * residual_out may be residual (updated in place), or NULL where nothing reads
+ * it; norm_out may be branch; no other overlap.  ln_weight, ln_bias: [d_model].  d_model a multiple of 8
  * (fp16/bf16) or 4 (fp32), at most 4096 (fp16/bf16) or 2048 (fp32).
  */
 typedef struct pk_resnorm_args {
@@ -335,6 +338,11 @@ typedef struct pk_resnorm_args {
   int64_t residual_out_stride;
   void* norm_out;
   int64_t norm_out_stride;
+  const void* ln2_weight;
+  const void* ln2_bias;
+  float ln2_eps;
+  void* norm2_out;
+  int64_t norm2_out_stride;
 } pk_resnorm_args;
 int pk_residual_norm(const pk_resnorm_args* args, void* stream);
 
@@ -350,8 +358,19 @@ int pk_residual_norm(const pk_resnorm_args* args, void* stream);
  * x [rows][k], weight [n][k], out [rows][n]: row strides in elements, rows
  * 16-byte aligned with unit inner stride; bias [n] or NULL.  out overlaps no
  * operand.  n a multiple of 64, k of 256 (else PK_ERR_UNSUPPORTED).
+ *
+ * With a prologue the product reads, instead of x (encoder.py:58-81),
+ *   PK_PRO_NORM            LayerNorm(x)
+ *   PK_PRO_RESIDUAL_NORM   LayerNorm(r), r = x + alpha * branch -> residual_out
+ *   PK_PRO_RESIDUAL_NORM2  LayerNorm(y), y = LayerNorm0(x + alpha * branch) ->
+ *                          residual_out (a layer's norm_out and the next layer's first norm)
+ * with pk_residual_norm's roundings, for the sizes that pk_linear_takes_norm
+ * accepts (few rows, k 512 or 1024; the first and last with PK_ACT_SILU): past
+ * them pk_residual_norm and a plain pk_linear are faster.  branch, residual_out:
+ * [rows][k]; residual_out is neither x nor branch.  ln_*, ln0_*: [k].
  */
 enum pk_activation { PK_ACT_NONE = 0, PK_ACT_SILU = 1 };
+enum pk_prologue { PK_PRO_NONE = 0, PK_PRO_NORM = 1, PK_PRO_RESIDUAL_NORM = 2, PK_PRO_RESIDUAL_NORM2 = 3 };
 typedef struct pk_linear_args {
   int32_t dtype;
   int32_t device;
@@ -366,7 +385,21 @@ typedef struct pk_linear_args {
   const void* bias;
   void* out;
   int64_t out_stride;
+  int32_t prologue;
+  float alpha;
+  const void* branch;
+  int64_t branch_stride;
+  const void* ln_weight;
+  const void* ln_bias;
+  const void* ln0_weight;
+  const void* ln0_bias;
+  float ln_eps;
+  float ln0_eps;
+  void* residual_out;
+  int64_t residual_out_stride;
 } pk_linear_args;
+/* 1 if pk_linear takes a prologue for this layer on the current device */
+int pk_linear_takes_norm(int32_t rows, int32_t n, int32_t k);
 int pk_linear(const pk_linear_args* args, int32_t count, void* stream);
 
 /* ---------------------------------------------------------------------------

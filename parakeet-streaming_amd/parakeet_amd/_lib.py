@@ -31,6 +31,11 @@ PK_ERR_STATE = -5
 ACT_NONE = 0
 ACT_SILU = 1
 
+PRO_NONE = 0
+PRO_NORM = 1
+PRO_RESIDUAL_NORM = 2
+PRO_RESIDUAL_NORM2 = 3
+
 PCM_S16 = 0
 PCM_F32 = 1
 
@@ -194,6 +199,11 @@ class ResNormArgs(ctypes.Structure):
         ("residual_out_stride", c_int64),
         ("norm_out", c_void_p),
         ("norm_out_stride", c_int64),
+        ("ln2_weight", c_void_p),
+        ("ln2_bias", c_void_p),
+        ("ln2_eps", ctypes.c_float),
+        ("norm2_out", c_void_p),
+        ("norm2_out_stride", c_int64),
     ]
 
 
@@ -212,6 +222,18 @@ class LinearArgs(ctypes.Structure):
         ("bias", c_void_p),
         ("out", c_void_p),
         ("out_stride", c_int64),
+        ("prologue", c_int32),
+        ("alpha", ctypes.c_float),
+        ("branch", c_void_p),
+        ("branch_stride", c_int64),
+        ("ln_weight", c_void_p),
+        ("ln_bias", c_void_p),
+        ("ln0_weight", c_void_p),
+        ("ln0_bias", c_void_p),
+        ("ln_eps", ctypes.c_float),
+        ("ln0_eps", ctypes.c_float),
+        ("residual_out", c_void_p),
+        ("residual_out_stride", c_int64),
     ]
 
 
@@ -343,6 +365,7 @@ SIGNATURES = {
     "pk_streaming_mask": (c_int, [POINTER(MaskArgs), c_void_p]),
     "pk_conv_step": (c_int, [POINTER(ConvArgs), c_void_p]),
     "pk_residual_norm": (c_int, [POINTER(ResNormArgs), c_void_p]),
+    "pk_linear_takes_norm": (c_int, [c_int32, c_int32, c_int32]),
     "pk_linear": (c_int, [POINTER(LinearArgs), c_int32, c_void_p]),
     "pk_fe_step": (c_int, [POINTER(FeArgs), c_void_p]),
     "pk_subsample": (c_int, [POINTER(SubArgs), c_void_p]),

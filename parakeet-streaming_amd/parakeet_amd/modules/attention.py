@@ -116,8 +116,11 @@ class ConformerAttention(nn.Module):
                 self.projected_pos(self._pos_src)
 
     def forward(self, x: Tensor, pos_emb: Tensor, attn_mask: Tensor, cache: ModelCache = None):
-        B, T = x.shape[:2]
-        qkv = ops.module_linear(x, self.qkv)
+        return self.attend(ops.module_linear(x, self.qkv), pos_emb, attn_mask, cache)
+
+    def attend(self, qkv: Tensor, pos_emb: Tensor, attn_mask: Tensor, cache: ModelCache = None):
+        """:meth:`forward` from the qkv projection's output [B, T, 3 D]."""
+        B, T = qkv.shape[:2]
         query, key, value = qkv.chunk(3, dim=-1)
         # [1, P, D] is one table for every stream; [B, P, D] gives each stream
         # its own (the reference broadcasts both, attention.py:102-106)
@@ -125,8 +128,8 @@ class ConformerAttention(nn.Module):
         if pos.dim() == 3 and pos.shape[0] == 1:
             pos = pos[0]
         mask = attn_mask.bool() if attn_mask is not None else None
-        bias_u = self.pos_bias_u.to(x.dtype).contiguous()
-        bias_v = self.pos_bias_v.to(x.dtype).contiguous()
+        bias_u = self.pos_bias_u.to(qkv.dtype).contiguous()
+        bias_v = self.pos_bias_v.to(qkv.dtype).contiguous()
         if cache is not None:
             out = cache.attend(
                 self.layer_idx, query, key, value, pos, bias_u, bias_v, mask, num_heads=self.num_heads

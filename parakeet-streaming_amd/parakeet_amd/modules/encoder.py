@@ -114,15 +114,20 @@ class ConformerConvolution(nn.Module):
         )
 
     def forward(self, x: Tensor, pad_mask: Tensor, cache=None):
-        h = ops.functional_linear(x, self.pointwise_conv1.weight.squeeze(-1), self.pointwise_conv1.bias)
+        return self.after_pointwise1(
+            ops.functional_linear(x, self.pointwise_conv1.weight.squeeze(-1), self.pointwise_conv1.bias), pad_mask, cache
+        )
+
+    def after_pointwise1(self, h: Tensor, pad_mask: Tensor, cache=None):
+        """:meth:`forward` from the first pointwise convolution's output [B, T, 2 D]."""
         if isinstance(cache, ConvCacheRef):
             bn, dw = self.batch_norm, self.depthwise_conv
             y = cache.cache.conv_step(cache.layer_idx, h, pad_mask, dw.weight, dw.bias, bn.weight, bn.bias, bn.eps)
             new_cache = None
         else:
-            B, K = x.shape[0], self.kernel_size
+            B, K = h.shape[0], self.kernel_size
             if cache is None:
-                frames = torch.zeros((B, 1, K - 1, self.d_model), dtype=x.dtype, device=x.device)
+                frames = torch.zeros((B, 1, K - 1, self.d_model), dtype=h.dtype, device=h.device)
             else:
                 frames = cache.transpose(1, 2).unsqueeze(1).contiguous()
             y = self._middle(h, pad_mask, frames)
@@ -149,6 +154,8 @@ class ConformerLayer(nn.Module):
         self.norm_out = nn.LayerNorm(hidden_size)
 
     def forward(self, x: Tensor, pos_emb: Tensor, pad_mask: Tensor, attn_mask: Tensor, cache: ModelCache):
+        if self.fuses(x, cache):
+            return self.finish(self.fused_step(x, pos_emb, pad_mask, attn_mask, cache))
         # each residual update and the LayerNorm that reads it are one step
         # (``residual_norm``); the layer's input is not modified
         residual, h = self.residual_norm(x, self.feed_forward1(self.norm_feed_forward1(x)), self.norm_self_att, 0.5)
@@ -159,6 +166,55 @@ class ConformerLayer(nn.Module):
         residual, h = self.residual_norm(residual, conv_out, self.norm_feed_forward2, 1.0, in_place=True)
         _, out = self.residual_norm(residual, self.feed_forward2(h), self.norm_out, 0.5, in_place=True)
         return out
+
+    def fuses(self, x: Tensor, cache) -> bool:
+        """Whether :meth:`fused_step` is this layer's step on ``x``: every module
+        of it is the class's own (no subclass, hook, replaced forward or active
+        dropout that the fused launches would pass by) on one 16-bit dtype, and
+        no gradient is asked for."""
+        attn, conv = self.self_attn, self.conv
+        return (
+            isinstance(cache, ModelCache)
+            and "residual_norm" not in self.__dict__
+            and x.is_contiguous()
+            and ops.plain_module(attn, ConformerAttention)
+            and ops.plain_module(attn.qkv, nn.Linear)
+            and ops.plain_module(conv, ConformerConvolution)
+            and ops.plain_module(conv.pointwise_conv1, nn.Conv1d)
+            and all(
+                ops.plain_module(ff, ConformerFeedForward) and ff._fused() and ops.linear_applies(x, ff.linear1.weight, ff.linear1.bias, silu=True)
+                for ff in (self.feed_forward1, self.feed_forward2)
+            )
+            and all(
+                ops.norm_applies(n, x)
+                for n in (self.norm_feed_forward1, self.norm_self_att, self.norm_conv, self.norm_feed_forward2, self.norm_out)
+            )
+            and attn.qkv.weight.dtype == conv.pointwise_conv1.weight.dtype == x.dtype
+        )
+
+    def fused_step(self, x, pos_emb: Tensor, pad_mask: Tensor, attn_mask: Tensor, cache: ModelCache) -> ops.Pending:
+        """The layer's step up to its last residual update and norm, which the
+        next reader's launch takes with it (or :meth:`residual_norm`).  ``x``: the
+        layer's input, or the layer before's :class:`ops.Pending` one."""
+        ff1, ff2, attn, conv = self.feed_forward1, self.feed_forward2, self.self_attn, self.conv
+        own = isinstance(x, ops.Pending)  # then the residual is this step's own buffer
+        x, h = ops.norm_linear(x, self.norm_feed_forward1, ff1.linear1.weight, ff1.linear1.bias, silu=True)
+        r, qkv = ops.norm_linear(
+            x, self.norm_self_att, attn.qkv.weight, attn.qkv.bias, branch=ops.module_linear(h, ff1.linear2), alpha=0.5, in_place=own
+        )
+        a = attn.attend(qkv, pos_emb, attn_mask, cache)
+        r, h = ops.norm_linear(
+            r, self.norm_conv, conv.pointwise_conv1.weight.squeeze(-1), conv.pointwise_conv1.bias, branch=a, in_place=True
+        )
+        c, conv_cache = conv.after_pointwise1(h, pad_mask=pad_mask, cache=cache.conv_ref(self.layer_idx))
+        cache.update_conv_cache(self.layer_idx, conv_cache)
+        r, h = ops.norm_linear(r, self.norm_feed_forward2, ff2.linear1.weight, ff2.linear1.bias, branch=c, silu=True, in_place=True)
+        return ops.Pending(r, ops.module_linear(h, ff2.linear2), self.norm_out, 0.5)
+
+    @staticmethod
+    def finish(p: ops.Pending) -> Tensor:
+        """The update and norm that :meth:`fused_step` left."""
+        return ConformerLayer.residual_norm(p.x, p.branch, p.norm, p.alpha, in_place=True)[1]
 
     @staticmethod
     def residual_norm(residual: Tensor, branch: Tensor, norm: nn.LayerNorm, alpha: float, in_place: bool = False):
@@ -284,8 +340,18 @@ class ConformerEncoder(nn.Module):
             device=x.device,
             lengths=length,
         )
+        # a layer's last residual update and norm run in the next layer's first launch
+        pend = None
         for layer in self.layers:
+            y = x if pend is None else pend.x
+            if ops.plain_module(layer, ConformerLayer) and layer.fuses(y, state.cache):
+                pend = layer.fused_step(x if pend is None else pend, pos_emb, pad_mask, att_mask, state.cache)
+                continue
+            if pend is not None:
+                x, pend = ConformerLayer.finish(pend), None
             x = layer(x, pos_emb=pos_emb, pad_mask=pad_mask, attn_mask=att_mask, cache=state.cache)
+        if pend is not None:
+            x = ConformerLayer.finish(pend)
         if isinstance(length, Tensor):
             state.processed_frames.add_(length)
             state.cache_lengths.add_(length)

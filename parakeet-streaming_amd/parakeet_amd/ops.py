@@ -519,6 +519,24 @@ def residual_norm(
 # pre-encode front end
 
 
+def residual_norm2(pend: "Pending", norm2: torch.nn.LayerNorm) -> tuple[torch.Tensor, torch.Tensor]:
+    """``y = norm(x + alpha * branch)`` of a :class:`Pending` update and
+    ``norm2(y)``, in one launch: a layer's norm_out and the next layer's
+    norm_feed_forward1 (encoder.py:58-60,80)."""
+    x, br = _aligned_rows(pend.x), _aligned_rows(pend.branch)
+    D = x.shape[-1]
+    y, z = torch.empty_like(x), torch.empty_like(x)
+    a = ResNormArgs()
+    a.dtype, a.device = dtype_code(x.dtype), x.device.index
+    a.rows, a.d_model, a.alpha = x.numel() // D, D, float(pend.alpha)
+    a.residual, a.residual_stride, a.branch, a.branch_stride = x.data_ptr(), D, br.data_ptr(), D
+    a.ln_weight, a.ln_bias, a.ln_eps = _ln(pend.norm)
+    a.ln2_weight, a.ln2_bias, a.ln2_eps = _ln(norm2)
+    a.norm_out, a.norm_out_stride, a.norm2_out, a.norm2_out_stride = y.data_ptr(), D, z.data_ptr(), D
+    check(lib().pk_residual_norm(ctypes.byref(a), _stream(x.device)), "pk_residual_norm")
+    return y, z
+
+
 def _transformed(x: torch.Tensor) -> bool:
     """Whether something follows or rewrites the torch calls made on ``x``
     (autocast, tracing, compilation, function transforms, forward-mode
@@ -628,6 +646,93 @@ def functional_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor 
     if linear_applies(x, weight, bias):
         return linear(x, weight, bias)
     return torch.nn.functional.linear(x, weight, bias)
+
+
+@dataclass
+class Pending:
+    """A residual update and norm not yet run: ``norm(x + alpha * branch)``, left
+    for the launch that reads it."""
+
+    x: torch.Tensor
+    branch: torch.Tensor
+    norm: torch.nn.LayerNorm
+    alpha: float
+
+
+def _ln(m: torch.nn.LayerNorm):
+    return m.weight.data_ptr(), m.bias.data_ptr(), float(m.eps)
+
+
+def norm_applies(m: torch.nn.Module, x: torch.Tensor) -> bool:
+    """Whether ``m`` is a LayerNorm over x's channels that the kernels compute."""
+    return (
+        plain_module(m, torch.nn.LayerNorm)
+        and m.normalized_shape == (x.shape[-1],)
+        and m.weight is not None
+        and m.bias is not None
+        and m.weight.dtype == x.dtype == m.bias.dtype
+        and m.weight.device == x.device == m.bias.device
+        and m.weight.is_contiguous()
+        and m.bias.is_contiguous()
+        and m.weight.data_ptr() % 16 == 0
+        and m.bias.data_ptr() % 16 == 0
+        and not (torch.is_grad_enabled() and (m.weight.requires_grad or m.bias.requires_grad))
+    )
+
+
+def norm_linear(
+    x: torch.Tensor | Pending,
+    norm: torch.nn.LayerNorm,
+    weight: torch.Tensor,
+    bias: torch.Tensor | None,
+    *,
+    branch: torch.Tensor | None = None,
+    alpha: float = 1.0,
+    silu: bool = False,
+    in_place: bool = False,
+) -> tuple[torch.Tensor, torch.Tensor]:
+    """``(r, linear(norm(r)))`` with ``r = x + alpha * branch`` (encoder.py:58-81):
+    one launch for few rows, else the residual update with its norm and the
+    linear layer.  ``x`` may be :class:`Pending` (then ``branch`` is None and
+    ``r`` is its norm), or ``branch`` None (then ``r`` is ``x``).  ``in_place``:
+    x is not read again and r may be written over it."""
+    pend = x if isinstance(x, Pending) else None
+    first = pend.x if pend is not None else x
+    n, k = weight.shape
+    dev, dt = first.device, first.dtype
+    rows = first.numel() // k
+    if not (lib().pk_linear_takes_norm(rows, n, k) and (silu or branch is not None) and layer_applies(dt, dev, rows, weight, bias, silu)):
+        if pend is not None:
+            r, h = residual_norm2(pend, norm)
+        elif branch is not None:
+            r, h = residual_norm(x, branch, norm.weight, norm.bias, alpha=alpha, eps=norm.eps, in_place=in_place)
+        else:
+            r, h = x, norm(x)
+        if layer_applies(dt, dev, rows, weight, bias, silu):
+            return r, linear(h, weight, bias, silu=silu)
+        y = torch.nn.functional.linear(h, weight, bias)
+        return r, torch.nn.functional.silu(y) if silu else y
+    first = _aligned_rows(first)
+    br = pend.branch if pend is not None else branch
+    out = torch.empty((*first.shape[:-1], n), dtype=dt, device=dev)
+    a = LinearArgs()
+    _linear_args(a, _DTYPES[dt], dev, first, rows, weight, bias, out, silu)
+    a.ln_weight, a.ln_bias, a.ln_eps = _ln(norm)
+    r = first
+    if br is None:
+        a.prologue = _lib.PRO_NORM
+    else:
+        br = _aligned_rows(br)
+        r = torch.empty_like(first)
+        a.branch, a.branch_stride = br.data_ptr(), k
+        a.residual_out, a.residual_out_stride = r.data_ptr(), k
+        if pend is not None:
+            a.prologue, a.alpha = _lib.PRO_RESIDUAL_NORM2, pend.alpha
+            a.ln0_weight, a.ln0_bias, a.ln0_eps = _ln(pend.norm)
+        else:
+            a.prologue, a.alpha = _lib.PRO_RESIDUAL_NORM, alpha
+    check(lib().pk_linear(ctypes.byref(a), 1, _stream(dev)), "pk_linear")
+    return r, out
 
 
 def feed_forward(x: torch.Tensor, w1: torch.Tensor, b1: torch.Tensor | None, w2: torch.Tensor, b2: torch.Tensor | None) -> torch.Tensor:

@@ -108,3 +108,105 @@ def test_feed_forward_keeps_gradients_hooks_dropout_and_autocast(cuda):
         assert torch.equal(ff(x), ff.linear2(ops.linear(x, ff.linear1.weight, ff.linear1.bias, silu=True)))
         f32 = ConformerFeedForward(512, 2048, 0.0).to(cuda).eval()
         assert f32(x.float()).dtype == torch.float32
+
+
+def _norm(D, dtype, device, g):
+    n = nn.LayerNorm(D).to(device=device, dtype=dtype).requires_grad_(False)
+    n.weight.copy_(1.0 + 0.2 * torch.randn(D, generator=g, device=device))
+    n.bias.copy_(0.2 * torch.randn(D, generator=g, device=device))
+    return n
+
+
+# rows of one tile and a remainder, one tile a CU with 32, 64 and 128 outputs,
+# and past them (the separate launches)
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,n,k", [(1, 2048, 512), (17, 1536, 512), (100, 2048, 512), (250, 2048, 512), (700, 2048, 512),
+                                      (2, 4096, 1024), (33, 3072, 1024), (64, 4096, 1024), (120, 4096, 1024), (300, 2048, 1024)])
+def test_norm_linear_matches_its_parts(cuda, dtype, rows, n, k):
+    """The residual is torch's own bit for bit; the product reads a norm that is
+    within one rounding of the fp32 LayerNorm (statistics in another order), so
+    outputs differ from the product of that norm by at most the sum of the
+    operand's roundings (relative 2 eps of each product) and their own."""
+    print(f"\n[norm-linear] {dtype} rows={rows} n={n} k={k}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(rows + n + k)
+    x = (2.0 * torch.randn(rows, k, generator=g, device=cuda) + 0.5).to(dtype)
+    br = torch.randn(rows, k, generator=g, device=cuda).to(dtype)
+    w = (torch.randn(n, k, generator=g, device=cuda) / math.sqrt(k)).to(dtype)
+    n0, n1 = _norm(k, dtype, cuda, g), _norm(k, dtype, cuda, g)
+
+    def ln(v, m):
+        return F.layer_norm(v.double(), (k,), m.weight.double(), m.bias.double(), m.eps)
+
+    def check(out, h, silu):
+        y = h @ w.double().T
+        mag = h.abs() @ w.double().abs().T
+        ref = F.silu(y) if silu else y
+        err = (out.double() - ref).abs()
+        bar = 1.05 * EPS[dtype] * ref.abs() + (1.1 * EPS[dtype] * (2 * mag) if silu else EPS[dtype] * 2 * mag) + TINY[dtype]
+        assert bool((err <= bar).all()), float((err - bar).max())
+        # the roundings are independent: their sum grows as the root of their number
+        rms = float((err.square().mean() / ref.square().mean()).sqrt())
+        assert rms <= 2.0 * EPS[dtype], rms
+
+    with torch.no_grad():
+        r, out = ops.norm_linear(x, n1, w, None, silu=True)
+        assert r is x
+        check(out, ln(x, n1), True)
+        want = x + br * 0.5
+        for silu in (False, True):
+            r, out = ops.norm_linear(x, n1, w, None, branch=br, alpha=0.5, silu=silu)
+            assert torch.equal(r, want)
+            check(out, ln(want, n1), silu)
+        r, out = ops.norm_linear(ops.Pending(x, br, n0, 1.0), n1, w, None, silu=True)
+        y, _ = ops.residual_norm2(ops.Pending(x, br, n0, 1.0), n1)
+        assert float((r.double() - ln(x + br, n0)).abs().max()) <= 4 * EPS[dtype] * 4.0
+        assert float((r - y).abs().float().max()) <= 8 * EPS[dtype]
+        check(out, ln(r, n1), True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,D,rows", [(torch.float16, 512, 5), (torch.bfloat16, 1024, 257), (torch.float32, 176, 3)])
+def test_residual_norm2_is_two_norms(cuda, dtype, D, rows):
+    g = torch.Generator(device="cuda").manual_seed(D)
+    x, br = (torch.randn(rows, D, generator=g, device=cuda).to(dtype) for _ in range(2))
+    n0, n1 = _norm(D, dtype, cuda, g), _norm(D, dtype, cuda, g)
+    y, z = ops.residual_norm2(ops.Pending(x, br, n0, 0.5), n1)
+    r, want = ops.residual_norm(x, br, n0.weight, n0.bias, alpha=0.5, eps=n0.eps)
+    _, want2 = ops.residual_norm(want, torch.zeros_like(want), n1.weight, n1.bias, eps=n1.eps)
+    assert torch.equal(y, want) and torch.equal(z, want2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("streams", [3, 200])
+def test_encoder_fused_layers_match_module_by_module(cuda, streams):
+    """The fused step of the layers against the same encoder run module by module
+    (a forward hook on a layer's submodule keeps its torch call), over several steps."""
+    from parakeet_amd.modules.encoder import ConformerEncoder
+
+    torch.manual_seed(streams)
+    with torch.device(cuda):
+        enc = ConformerEncoder(
+            feat_in=80, hidden_size=512, ff_expansion_factor=4, num_layers=3, num_heads=8, subsampling_factor=8,
+            pos_emb_max_len=500, conv_kernel_size=9, att_context_size=[70, 1], subsampling_conv_channels=256, use_bias=False,
+        )
+    for layer in enc.layers:
+        layer.self_attn.pos_bias_u.data.normal_(std=0.02)
+        layer.self_attn.pos_bias_v.data.normal_(std=0.02)
+    enc = enc.half().eval().requires_grad_(False)
+    states = [enc.init_streaming_state(batch_size=streams, device=cuda, dtype=torch.float16) for _ in range(3)]
+    length = torch.full((streams,), 2, dtype=torch.int64, device=cuda)
+    with torch.no_grad():
+        for step in range(4):
+            x = torch.randn(streams, 2, 512, device=cuda).half()
+            assert enc.layers[0].fuses(x, states[0].cache)
+            a, _ = enc(x, states[0], length=length)
+            hooks = [m.register_forward_hook(lambda *_: None) for m in (enc.layers[1].feed_forward1.linear1, enc.layers[2].norm_conv)]
+            assert not enc.layers[1].fuses(x, states[1].cache) and not enc.layers[2].fuses(x, states[1].cache)
+            b, _ = enc(x, states[1], length=length)
+            hooks += [enc.layers[0].self_attn.register_forward_hook(lambda *_: None)]
+            c, _ = enc(x, states[2], length=length)
+            for h in hooks:
+                h.remove()
+            for t in (b, c):  # three layers of independent fp16 roundings
+                assert float((t.float() - a.float()).norm() / a.float().norm()) <= 4e-3
