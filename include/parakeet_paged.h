@@ -368,9 +368,19 @@ int pk_residual_norm(const pk_resnorm_args* args, void* stream);
  * accepts (few rows, k 512 or 1024; the first and last with PK_ACT_SILU): past
  * them pk_residual_norm and a plain pk_linear are faster.  branch, residual_out:
  * [rows][k]; residual_out is neither x nor branch.  ln_*, ln0_*: [k].
+ *   PK_PRO_NORM_SILU       SiLU(LayerNorm(x)) of fp32 rows x (k 512 or 1024, any
+ *                          number of rows; past pk_linear_takes_norm residual_out
+ *                          is its [rows][k] scratch), convolution.py:156-158
+ * PK_ACT_GLU_CONV (convolution.py:37-47,150-155): the layer is a convolution
+ * module's first pointwise convolution, weight [2 d_model][k]; out becomes the
+ * causal depthwise convolution over [cache ; GLU], fp32 [rows][d_model] (out_stride
+ * in fp32 elements), the cache updated in place as pk_conv_step does.  conv gives
+ * batch, chunk (<= 16), d_model, kernel (9), cache, slots, layer, pad_mask or
+ * lengths, dw_weight and dw_bias; rows = batch * chunk.  With PK_PRO_NONE or
+ * PK_PRO_RESIDUAL_NORM.
  */
-enum pk_activation { PK_ACT_NONE = 0, PK_ACT_SILU = 1 };
-enum pk_prologue { PK_PRO_NONE = 0, PK_PRO_NORM = 1, PK_PRO_RESIDUAL_NORM = 2, PK_PRO_RESIDUAL_NORM2 = 3 };
+enum pk_activation { PK_ACT_NONE = 0, PK_ACT_SILU = 1, PK_ACT_GLU_CONV = 2 };
+enum pk_prologue { PK_PRO_NONE = 0, PK_PRO_NORM = 1, PK_PRO_RESIDUAL_NORM = 2, PK_PRO_RESIDUAL_NORM2 = 3, PK_PRO_NORM_SILU = 4 };
 typedef struct pk_linear_args {
   int32_t dtype;
   int32_t device;
@@ -397,9 +407,11 @@ typedef struct pk_linear_args {
   float ln0_eps;
   void* residual_out;
   int64_t residual_out_stride;
+  const pk_conv_args* conv;
 } pk_linear_args;
-/* 1 if pk_linear takes a prologue for this layer on the current device */
-int pk_linear_takes_norm(int32_t rows, int32_t n, int32_t k);
+/* 1 if pk_linear takes a prologue with a residual or PK_PRO_NORM for this layer on
+ * the current device; chunk: PK_ACT_GLU_CONV's frames a stream, else 1 */
+int pk_linear_takes_norm(int32_t rows, int32_t n, int32_t k, int32_t chunk);
 int pk_linear(const pk_linear_args* args, int32_t count, void* stream);
 
 /* ---------------------------------------------------------------------------

@@ -41,10 +41,13 @@ struct MmaL<bf16_t> {
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-enum { kEpiNone = 0, kEpiSilu = 1 };
+// kEpiConv: GLU and the causal depthwise convolution with its cache (store_conv)
+enum { kEpiNone = 0, kEpiSilu = 1, kEpiConv = 2 };
 // what stands before the product: LayerNorm(x); r = x + alpha * branch, then
 // LayerNorm(r); the same with a LayerNorm between, y = LayerNorm'(r)
-enum { kProNorm = 1, kProResNorm = 2, kProResNorm2 = 3 };
+// kProNormSilu: SiLU(LayerNorm(x)) of fp32 rows
+enum { kProNorm = 1, kProResNorm = 2, kProResNorm2 = 3, kProNormSilu = 4 };
+constexpr int kTaps = 9;  // depthwise taps of kEpiConv
 
 template <typename ST>
 struct LinK {
@@ -66,6 +69,20 @@ struct LinK {
   int64_t out_s;
   int32_t M, N, K;
   int32_t mtiles, xm;
+  int32_t rpt;      // rows a tile (kEpiConv: whole streams of T frames)
+  const float* xf;  // kProNormSilu: [M][K] fp32 rows, stride x_s
+  // kEpiConv: rows are [batch][T] frames, W [2 D][K] (values, then gates); y
+  // [batch T][D] fp32, the cache as in pk_conv_step
+  float* y;
+  int64_t y_s;
+  ST* cache;
+  const int32_t* slots;
+  const uint8_t* pad;
+  const int64_t* lengths;
+  int64_t len_scalar;
+  const ST* dw;   // [D][kTaps]
+  const ST* dwb;  // [D] or nullptr
+  int32_t num_slots, num_layers, layer, T, batch;
 };
 
 template <typename ST>
@@ -212,9 +229,32 @@ __device__ static inline void wait_vm() {
   __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N & 0x30) << 10));
 }
 
-// A tile's output: the sums of the WK parts of K meet in LDS, then bias and
-// activation, then through LDS to whole 16-byte chunks of a row.  Waves are
-// numbered (wk WM + wm) WN + wn; smem is free when every wave is here.
+// The sums of the WK parts of K meet in LDS (at smem + at); waves are numbered
+// (wk WM + wm) WN + wn, the waves wk == 0 end with the sums.
+template <int BM, int BN, int WMN, int WK, int TM, int TN>
+__device__ static inline void sum_parts(unsigned char* smem, int at, f32x4_t (&acc)[TM][TN], int wave, int lane) {
+  if constexpr (WK > 1) {
+    f32x4_t* const red = reinterpret_cast<f32x4_t*>(smem + at);
+    if (wave >= WMN) {
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int n = 0; n < TN; ++n) red[((wave - WMN) * TM * TN + m * TN + n) * 64 + lane] = acc[m][n];
+    }
+    __syncthreads();
+    if (wave < WMN) {
+#pragma unroll
+      for (int w = 1; w < WK; ++w)
+#pragma unroll
+        for (int m = 0; m < TM; ++m)
+#pragma unroll
+          for (int n = 0; n < TN; ++n) acc[m][n] += red[((wave + (w - 1) * WMN) * TM * TN + m * TN + n) * 64 + lane];
+    }
+  }
+}
+
+// A tile's output: bias and activation, then through LDS to whole 16-byte chunks
+// of a row.  smem is free when every wave is here.
 template <typename ST, int BM, int BN, int WM, int WN, int WK, int TM, int TN, int EPI>
 __device__ static inline void store_tile(const LinK<ST>& p, unsigned char* smem, f32x4_t (&acc)[TM][TN], int row0, int n0,
                                          int wave, int lane) {
@@ -223,24 +263,7 @@ __device__ static inline void store_tile(const LinK<ST>& p, unsigned char* smem,
   constexpr int kOut = BM * OS * 2;
   const int l16 = lane & 15, kg = lane >> 4;
   const int wk = wave / (WM * WN), wm = (wave / WN) % WM, wn = wave % WN;
-  if constexpr (WK > 1) {
-    f32x4_t* const red = reinterpret_cast<f32x4_t*>(smem + kOut);
-    if (wk > 0) {
-#pragma unroll
-      for (int m = 0; m < TM; ++m)
-#pragma unroll
-        for (int n = 0; n < TN; ++n) red[((wave - WM * WN) * TM * TN + m * TN + n) * 64 + lane] = acc[m][n];
-    }
-    __syncthreads();
-    if (wk == 0) {
-#pragma unroll
-      for (int w = 1; w < WK; ++w)
-#pragma unroll
-        for (int m = 0; m < TM; ++m)
-#pragma unroll
-          for (int n = 0; n < TN; ++n) acc[m][n] += red[((wave + (w - 1) * WM * WN) * TM * TN + m * TN + n) * 64 + lane];
-    }
-  }
+  sum_parts<BM, BN, WM * WN, WK>(smem, kOut, acc, wave, lane);
   ST* const os = reinterpret_cast<ST*>(smem);
   if (wk == 0) {
 #pragma unroll
@@ -265,6 +288,143 @@ __device__ static inline void store_tile(const LinK<ST>& p, unsigned char* smem,
     const int r = i / (BN / 8), c = (i % (BN / 8)) * 8;
     if (row0 + r < p.M) st16(p.out + (int64_t)(row0 + r) * p.out_s + n0 + c, *reinterpret_cast<const u32x4*>(os + r * OS + c));
   }
+}
+
+// The first pointwise convolution's tile up to the depthwise convolution
+// (convolution.py:37-47,152-155), in place of a launch that reads its output
+// back: the weight rows of a tile alternate 16 values and their 16 gates, so a
+// lane holds both; GLU in fp32, zero where padded, rounded once to the storage
+// type (what the cache holds); then a thread takes 2 channels of a stream: its
+// cache rows (loaded before the product, `cw`), the tile's frames, fp32 sums in
+// pk_conv_step's order, the next cache in place.  A tile holds whole streams, so
+// no other workgroup touches these channels of their caches.  840 rows (60
+// streams x 14) x 1024 -> 2048: 12.8 us and 4.8 for the norm after it, against
+// 10.8 for the product and 14.8 for the convolution step as launches of their own;
+// 256 rows x 512 7.7 (residual and norm in it) against 13 for the three.
+struct ConvItem {
+  uint32_t cw[kTaps - 1], tw[kTaps];  // 2 channels of the cache rows; 2 x kTaps taps
+};
+template <typename ST>
+__device__ static inline ST* conv_cache(const LinK<ST>& p, int b, int c) {
+  const int slot = p.slots ? p.slots[b] : b;
+  if ((uint32_t)slot >= (uint32_t)p.num_slots) return nullptr;  // such a stream is left untouched
+  return p.cache + ((int64_t)slot * p.num_layers + p.layer) * (kTaps - 1) * (p.N / 2) + c;
+}
+template <typename ST, int CB>
+__device__ static inline void conv_load(const LinK<ST>& p, int i, int mt_i, int c0, ConvItem& it) {
+  const int per = p.rpt / p.T;
+  const int s = i / (CB / 2), c = c0 + (i % (CB / 2)) * 2, b = mt_i * per + s;
+  if (s >= per || b >= p.batch) return;
+  const uint32_t* tp = reinterpret_cast<const uint32_t*>(p.dw + (int64_t)c * kTaps);  // c even: 4-byte aligned
+#pragma unroll
+  for (int k = 0; k < kTaps; ++k) it.tw[k] = tp[k];
+  const ST* q = conv_cache(p, b, c);
+  if (!q) return;
+#pragma unroll
+  for (int r = 0; r < kTaps - 1; ++r) it.cw[r] = *reinterpret_cast<const uint32_t*>(q + (int64_t)r * (p.N / 2));
+}
+template <typename ST>
+__device__ static inline void two_of(uint32_t w, float& lo, float& hi) {
+  if constexpr (__is_same(ST, bf16_t)) {
+    lo = __uint_as_float(w << 16);
+    hi = __uint_as_float(w & 0xffff0000u);
+  } else {
+    float f[2];
+    Tr<_Float16>::two(w, f);
+    lo = f[0];
+    hi = f[1];
+  }
+}
+template <typename ST>
+__device__ static inline uint32_t pack2(float lo, float hi) {
+  if constexpr (__is_same(ST, bf16_t)) return bf16_pair_bits(lo, hi);
+  const float f[2] = {lo, hi};
+  return Tr<_Float16>::two(f);
+}
+template <typename ST, int BM, int BN, int WM, int WN, int WK, int TM, int TN>
+__device__ static inline void store_conv(const LinK<ST>& p, unsigned char* smem, f32x4_t (&acc)[TM][TN], int mt_i, int nt_i,
+                                         ConvItem& it, int wave, int lane) {
+  constexpr int NTH = 64 * WM * WN * WK;
+  constexpr int CB = BN / 2, GS = CB + 8;
+  constexpr int kOut = BM * GS * 2;
+  const int D = p.N / 2, c0 = nt_i * CB, row0 = mt_i * p.rpt;
+  const int l16 = lane & 15, kg = lane >> 4;
+  const int wm = (wave / WN) % WM, wn = wave % WN;
+  sum_parts<BM, BN, WM * WN, WK>(smem, kOut, acc, wave, lane);
+  ST* const gl = reinterpret_cast<ST*>(smem);  // [BM][GS] GLU outputs
+  if (wave < WM * WN) {
+#pragma unroll
+    for (int m = 0; m < TM; ++m) {
+      const int lr = (wm * TM + m) * 16 + l16, row = min(row0 + lr, p.M - 1);
+      const int b = row / p.T, t = row - b * p.T;
+      const bool valid = p.pad ? p.pad[row] == 0 : (int64_t)t < (p.lengths ? p.lengths[b] : p.len_scalar);
+#pragma unroll
+      for (int n = 0; n < TN / 2; ++n) {
+        const int c = (wn * (TN / 2) + n) * 16 + kg * 4;
+        float f[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float a = acc[m][2 * n][e], g = acc[m][2 * n + 1][e];
+          if (p.bias) {
+            a += from_st(p.bias[c0 + c + e]);
+            g += from_st(p.bias[D + c0 + c + e]);
+          }
+          f[e] = valid ? a / (1.f + __expf(-g)) : 0.f;
+        }
+        *reinterpret_cast<u32x2*>(gl + lr * GS + c) = pack4<ST>(f);
+      }
+    }
+  }
+  __syncthreads();
+  const int per = p.rpt / p.T;
+  for (int i = threadIdx.x; i < per * (CB / 2); i += NTH) {
+    const int s = i / (CB / 2), cl = (i % (CB / 2)) * 2, c = c0 + cl, b = mt_i * per + s;
+    if (b >= p.batch) break;  // streams ascend
+    if (i >= NTH) conv_load<ST, CB>(p, i, mt_i, c0, it);  // past the ones loaded ahead
+    ST* const q = conv_cache(p, b, c);
+    if (!q) continue;
+    float w[2][kTaps], win[kTaps][2], bias[2] = {0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < kTaps; ++k) {
+      // element e of the pair's 2 kTaps taps: channel e / kTaps, tap e % kTaps
+      float lo, hi;
+      two_of<ST>(it.tw[k], lo, hi);
+      w[(2 * k) / kTaps][(2 * k) % kTaps] = lo;
+      w[(2 * k + 1) / kTaps][(2 * k + 1) % kTaps] = hi;
+    }
+    if (p.dwb) {
+      bias[0] = from_st(p.dwb[c]);
+      bias[1] = from_st(p.dwb[c + 1]);
+    }
+#pragma unroll
+    for (int r = 0; r < kTaps - 1; ++r) two_of<ST>(it.cw[r], win[r][0], win[r][1]);
+    float* yp = p.y + (int64_t)b * p.T * p.y_s + c;
+    for (int t = 0; t < p.T; ++t) {
+      two_of<ST>(*reinterpret_cast<const uint32_t*>(gl + (s * p.T + t) * GS + cl), win[kTaps - 1][0], win[kTaps - 1][1]);
+      float2 o = {bias[0], bias[1]};
+#pragma unroll
+      for (int k = 0; k < kTaps; ++k) {
+        o.x = fmaf(w[0][k], win[k][0], o.x);
+        o.y = fmaf(w[1][k], win[k][1], o.y);
+      }
+      *reinterpret_cast<float2*>(yp + t * p.y_s) = o;
+#pragma unroll
+      for (int k = 0; k < kTaps - 1; ++k) {
+        win[k][0] = win[k + 1][0];
+        win[k][1] = win[k + 1][1];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < kTaps - 1; ++r)
+      *reinterpret_cast<uint32_t*>(q + (int64_t)r * D) = pack2<ST>(win[r][0], win[r][1]);
+  }
+}
+
+// row of W that a tile's output column n (of BN) multiplies
+template <int BN, int EPI>
+__device__ static inline int w_row(int nt_i, int n, int N) {
+  if constexpr (EPI == kEpiConv) return ((n & 16) ? N / 2 : 0) + nt_i * (BN / 2) + (n >> 5) * 16 + (n & 15);
+  return nt_i * BN + n;
 }
 
 // Many rows: BM x BN outputs a workgroup, WM x WN x WK waves, both operands
@@ -300,7 +460,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) lin_tile_kernel(const LinK<
   const int wk = wave / (WM * WN), wm = (wave / WN) % WM, wn = wave % WN;
   int mt_i, nt_i;
   xcd_tile(blockIdx.x, gridDim.x, p.mtiles, p.xm, mt_i, nt_i);
-  const int row0 = mt_i * BM, n0 = nt_i * BN;
+  const int row0 = mt_i * p.rpt, n0 = nt_i * BN;
 
   // chunk c of a stage: row c / CH of [x rows ; w rows], LDS position c % CH
   const __amdgpu_buffer_rsrc_t rx = bytes_rsrc(p.x, (uint32_t)((p.M - 1) * p.x_s + p.K) * 2u);
@@ -312,7 +472,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) lin_tile_kernel(const LinK<
     const int r = c / CH, pos = c % CH;
     const int ch = (pos & ~7) | ((pos ^ r) & 7);
     off[i] = r < BM ? (uint32_t)(min(row0 + r, p.M - 1) * p.x_s + ch * 8) * 2u
-                    : (uint32_t)((n0 + r - BM) * p.w_s + ch * 8) * 2u;
+                    : (uint32_t)(w_row<BN, EPI>(nt_i, r - BM, p.N) * p.w_s + ch * 8) * 2u;
   }
   auto issue = [&](int st, int k) {
 #pragma unroll
@@ -328,6 +488,11 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) lin_tile_kernel(const LinK<
     for (int n = 0; n < TN; ++n) acc[m][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   const int iters = p.K / BK;
+  ConvItem cv;
+  if constexpr (EPI == kEpiConv) {
+    conv_load<ST, BN / 2>(p, threadIdx.x, mt_i, nt_i * (BN / 2), cv);
+    __builtin_amdgcn_sched_barrier(0);  // ahead of the stages, whose counts the waits below rely on
+  }
 #pragma unroll
   for (int s = 0; s < S - 1; ++s)
     if (s < iters) issue(s, s * BK);
@@ -366,7 +531,10 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) lin_tile_kernel(const LinK<
     st = st == S - 1 ? 0 : st + 1;
   }
   __syncthreads();
-  store_tile<ST, BM, BN, WM, WN, WK, TM, TN, EPI>(p, smem, acc, row0, n0, wave, lane);
+  if constexpr (EPI == kEpiConv)
+    store_conv<ST, BM, BN, WM, WN, WK, TM, TN>(p, smem, acc, mt_i, nt_i, cv, wave, lane);
+  else
+    store_tile<ST, BM, BN, WM, WN, WK, TM, TN, EPI>(p, smem, acc, row0, n0, wave, lane);
 }
 
 // A Conformer layer's residual update and LayerNorm (encoder.py:58-81) in the
@@ -403,7 +571,7 @@ __global__ void __launch_bounds__(64 * WN * WK) lin_norm_kernel(const LinK<ST> p
   const int wk = wave / WN, wn = wave % WN;
   int mt_i, nt_i;
   xcd_tile(blockIdx.x, gridDim.x, p.mtiles, p.xm, mt_i, nt_i);
-  const int row0 = mt_i * BM, n0 = nt_i * BN;
+  const int row0 = mt_i * p.rpt, n0 = nt_i * BN;
 
   const __amdgpu_buffer_rsrc_t rw = bytes_rsrc(p.w, (uint32_t)((p.N - 1) * p.w_s + p.K) * 2u);
   unsigned char* const ring = smem + kAct;
@@ -412,7 +580,7 @@ __global__ void __launch_bounds__(64 * WN * WK) lin_norm_kernel(const LinK<ST> p
   for (int i = 0; i < LPS; ++i) {
     const int c = (i * NW + wave) * 64 + lane;
     const int r = c / CH, pos = c % CH;
-    off[i] = (uint32_t)((n0 + r) * p.w_s + ((pos & ~7) | ((pos ^ r) & 7)) * 8) * 2u;
+    off[i] = (uint32_t)(w_row<BN, EPI>(nt_i, r, p.N) * p.w_s + ((pos & ~7) | ((pos ^ r) & 7)) * 8) * 2u;
   }
   auto issue = [&](int st, int k) {
 #pragma unroll
@@ -420,15 +588,23 @@ __global__ void __launch_bounds__(64 * WN * WK) lin_norm_kernel(const LinK<ST> p
   };
 
   // the rows first (their use comes first), then the first weight stages
+  constexpr bool kRes = PRO == kProResNorm || PRO == kProResNorm2;
   u32x4 xv[RPW][KV], bv[RPW][KV], lwv[KV], lbv[KV], lwv0[KV], lbv0[KV];
+  ConvItem cv;
+  if constexpr (EPI == kEpiConv) conv_load<ST, BN / 2>(p, threadIdx.x, mt_i, nt_i * (BN / 2), cv);
 #pragma unroll
   for (int v = 0; v < KV; ++v) {
     const int c = (lane + 64 * v) * 8;
 #pragma unroll
     for (int r = 0; r < RPW; ++r) {
       const int row = min(row0 + wave * RPW + r, p.M - 1);
-      xv[r][v] = ld16(p.x + row * p.x_s + c);
-      if constexpr (PRO != kProNorm) bv[r][v] = ld16(p.br + row * p.br_s + c);
+      if constexpr (PRO == kProNormSilu) {  // 8 fp32 values: 2 chunks
+        xv[r][v] = ld16(p.xf + row * p.x_s + c);
+        bv[r][v] = ld16(p.xf + row * p.x_s + c + 4);
+      } else {
+        xv[r][v] = ld16(p.x + row * p.x_s + c);
+        if constexpr (kRes) bv[r][v] = ld16(p.br + row * p.br_s + c);
+      }
     }
     lwv[v] = ld16(p.lnw + c);
     lbv[v] = ld16(p.lnb + c);
@@ -472,13 +648,18 @@ __global__ void __launch_bounds__(64 * WN * WK) lin_norm_kernel(const LinK<ST> p
 #pragma unroll
   for (int r = 0; r < RPW; ++r) {
     const int lr = wave * RPW + r;
-    const bool write = PRO != kProNorm && nt_i == 0 && row0 + lr < p.M;  // one workgroup of the row tile
+    const bool write = kRes && nt_i == 0 && lr < p.rpt && row0 + lr < p.M;  // one workgroup of the row tile
     ST* const rout = p.rout + (int64_t)(row0 + lr) * p.rout_s;
     float f[KV][8];
 #pragma unroll
     for (int v = 0; v < KV; ++v) {
-      Tr<ST>::unpack(xv[r][v], f[v]);
-      if constexpr (PRO != kProNorm) {
+      if constexpr (PRO == kProNormSilu) {
+        Tr<float>::unpack(xv[r][v], f[v]);
+        Tr<float>::unpack(bv[r][v], f[v] + 4);
+      } else {
+        Tr<ST>::unpack(xv[r][v], f[v]);
+      }
+      if constexpr (kRes) {
         float b[8];
         Tr<ST>::unpack(bv[r][v], b);
 #pragma unroll
@@ -500,6 +681,10 @@ __global__ void __launch_bounds__(64 * WN * WK) lin_norm_kernel(const LinK<ST> p
 #pragma unroll
     for (int v = 0; v < KV; ++v) {
       const int c = lane + 64 * v;
+      if constexpr (PRO == kProNormSilu) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[v][e] = epi_act<kEpiSilu>(f[v][e]);
+      }
       *reinterpret_cast<u32x4*>(smem + lr * K * 2 + ((c & ~7) | ((c ^ lr) & 7)) * 16) = Tr<ST>::pack(f[v]);
     }
   }
@@ -552,7 +737,56 @@ __global__ void __launch_bounds__(64 * WN * WK) lin_norm_kernel(const LinK<ST> p
     st = st == S - 1 ? 0 : st + 1;
   }
   __syncthreads();
-  store_tile<ST, BM, BN, 1, WN, WK, TM, TN, EPI>(p, smem, acc, row0, n0, wave, lane);
+  if constexpr (EPI == kEpiConv)
+    store_conv<ST, BM, BN, 1, WN, WK, TM, TN>(p, smem, acc, mt_i, nt_i, cv, wave, lane);
+  else
+    store_tile<ST, BM, BN, 1, WN, WK, TM, TN, EPI>(p, smem, acc, row0, n0, wave, lane);
+}
+
+// SiLU(LayerNorm(x)) of fp32 rows (convolution.py:156-157), a wave a row, for the
+// row counts past lin_norm_kernel: bound by a launch and its 6 bytes an element
+// (4.8 us in the trace for 840 rows x 1024, 5.2 for 4096 x 512)
+template <typename ST, int KV>
+__global__ void __launch_bounds__(256) norm_silu_kernel(const float* x, int64_t x_s, const ST* lnw, const ST* lnb, float eps,
+                                                        ST* out, int64_t out_s, int rows) {
+#pragma clang fp contract(off)
+  constexpr int K = 512 * KV;
+  const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;  // the whole wave: no barrier below
+  float f[KV][8];
+  u32x4 wv[KV], bv[KV];
+  float s = 0.f;
+#pragma unroll
+  for (int v = 0; v < KV; ++v) {
+    const int c = (lane + 64 * v) * 8;
+    Tr<float>::unpack(ld16(x + row * x_s + c), f[v]);
+    Tr<float>::unpack(ld16(x + row * x_s + c + 4), f[v] + 4);
+    wv[v] = ld16(lnw + c);
+    bv[v] = ld16(lnb + c);
+  }
+#pragma unroll
+  for (int v = 0; v < KV; ++v)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s += f[v][e];
+  const float mean = group_sum<64>(s) * (1.f / (float)K);
+  float q = 0.f;
+#pragma unroll
+  for (int v = 0; v < KV; ++v)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      f[v][e] -= mean;
+      q = fmaf(f[v][e], f[v][e], q);
+    }
+  const float rstd = rsqrtf(group_sum<64>(q) * (1.f / (float)K) + eps);
+#pragma unroll
+  for (int v = 0; v < KV; ++v) {
+    float w[8], b[8];
+    Tr<ST>::unpack(wv[v], w);
+    Tr<ST>::unpack(bv[v], b);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[v][e] = epi_act<kEpiSilu>(fmaf(f[v][e] * rstd, w[e], b[e]));
+    st16(out + row * out_s + (lane + 64 * v) * 8, Tr<ST>::pack(f[v]));
+  }
 }
 
 namespace {
@@ -574,7 +808,8 @@ int xcd_split(int mtiles, int ntiles, int bm, int bn) {
 
 template <typename ST>
 dim3 tile_grid(LinK<ST>& k, int bm, int bn) {
-  k.mtiles = (k.M + bm - 1) / bm;
+  k.rpt = k.T > 0 ? bm / k.T * k.T : bm;
+  k.mtiles = (k.M + k.rpt - 1) / k.rpt;
   k.xm = xcd_split(k.mtiles, k.N / bn, bm, bn);
   return dim3((unsigned)(k.mtiles * (k.N / bn)));
 }
@@ -622,9 +857,10 @@ constexpr Form kForms[] = {
 constexpr int kNumForms = sizeof(kForms) / sizeof(kForms[0]);
 
 // us of a launch in form f, or a negative number where it does not fit
-float form_cost(const Form& f, int64_t M, int64_t N, int64_t K, int cus) {
-  if (N % f.bn != 0 || K % f.kmul != 0) return -1.f;
-  const int64_t tiles = (M + f.bm - 1) / f.bm * (N / f.bn);
+float form_cost(const Form& f, int64_t M, int64_t N, int64_t K, int cus, int T = 1) {
+  if (N % f.bn != 0 || K % f.kmul != 0 || T > f.bm) return -1.f;
+  const int rpt = f.bm / T * T;
+  const int64_t tiles = (M + rpt - 1) / rpt * (N / f.bn);
   const int64_t per = (tiles + cus - 1) / cus, rounds = (per + f.occ - 1) / f.occ;
   const float c = f.s * (float)K / 1024.f;
   return f.a + (float)(rounds - 1) * (f.a - 2.f) + (float)rounds * c + 0.8f * c * (float)(per - rounds);
@@ -674,10 +910,11 @@ int launch_norm(LinK<ST> k, hipStream_t s) {
 // rows (32 outputs) 5.0 us against 5.9, 128 rows (64) 5.3 against 6.9, 256 rows
 // (128) 6.1 against 7.7, 512 rows (128, two tiles a CU) 8.2 against 8.7; 1024 ->
 // 4096: 16 rows 7.3 against 7.6, 120 rows 8.9 against 9.6, 256 rows 12.7 against 11.2.
-int norm_form(int64_t M, int64_t N, int64_t K, int cus) {
-  if (K != 512 && K != 1024) return 0;
+int norm_form(int64_t M, int64_t N, int64_t K, int cus, int T = 1) {
+  if ((K != 512 && K != 1024) || T > 16) return 0;
+  const int rpt = 16 / T * T;
   for (int bn = 32; bn <= 128; bn *= 2)
-    if (N % bn == 0 && (M + 15) / 16 * (N / bn) <= cus) return bn;
+    if (N % bn == 0 && (M + rpt - 1) / rpt * (N / bn) <= cus) return bn;
   return 0;
 }
 
@@ -694,6 +931,28 @@ int launch_norm_k(const LinK<ST>& k, int bn, hipStream_t s) {
   return launch_norm_form<ST, 2, PRO, EPI>(k, bn, s);
 }
 
+// kEpiConv without a prologue: the tile forms whose waves hold values and gates
+template <typename ST>
+int launch_conv_form(const LinK<ST>& k, int cus, hipStream_t s) {
+  constexpr int forms[] = {6, 7, 8, 10};
+  int best = -1;
+  float cost = 0.f;
+  for (int f : forms) {
+    const float c = form_cost(kForms[f], k.M, k.N, k.K, cus, k.T);
+    if (c >= 0.f && (best < 0 || c < cost)) {
+      best = f;
+      cost = c;
+    }
+  }
+  switch (best) {
+    case 6: return launch_tile<ST, 32, 64, 1, 2, 4, 128, 5, kEpiConv>(k, s);
+    case 7: return launch_tile<ST, 64, 64, 2, 2, 2, 64, 4, kEpiConv>(k, s);
+    case 8: return launch_tile<ST, 64, 128, 2, 4, 1, 64, 3, kEpiConv>(k, s);
+    case 10: return launch_tile<ST, 128, 128, 2, 2, 1, 64, 2, kEpiConv>(k, s);
+    default: return fail(PK_ERR_UNSUPPORTED, "pk_linear: no form for %d -> %d with the convolution", k.K, k.N);
+  }
+}
+
 bool row_ok(int64_t rows, int64_t stride, int64_t width) {
   return stride >= 0 && stride % 8 == 0 && (rows <= 1 || stride >= width) &&
          (rows - 1) * stride + width < (int64_t{1} << 31);
@@ -705,16 +964,38 @@ int linear_typed(const pk_linear_args* a, hipStream_t s) {
   if (a->rows < 0) return fail(PK_ERR_INVALID, "%s: rows %d < 0", what, a->rows);
   if (a->n <= 0 || a->n % 64 != 0 || a->k <= 0 || a->k % 256 != 0)
     return fail(PK_ERR_UNSUPPORTED, "%s: n %d must be a multiple of 64 and k %d of 256", what, a->n, a->k);
-  if (a->activation != PK_ACT_NONE && a->activation != PK_ACT_SILU)
+  if (a->activation < PK_ACT_NONE || a->activation > PK_ACT_GLU_CONV)
     return fail(PK_ERR_INVALID, "%s: unknown activation %d", what, a->activation);
+  const bool glu = a->activation == PK_ACT_GLU_CONV;
+  const pk_conv_args* cv = a->conv;
+  if (glu) {
+    if (!cv) return fail(PK_ERR_INVALID, "%s: PK_ACT_GLU_CONV needs conv", what);
+    if (cv->kernel != kTaps || cv->chunk < 1 || cv->chunk > 16)
+      return fail(PK_ERR_UNSUPPORTED, "%s: convolution of %d taps over %d frames (built: %d taps, up to 16 frames)", what,
+                  cv->kernel, cv->chunk, kTaps);
+    if (a->n != 2 * (int64_t)cv->d_model || cv->batch < 0 || a->rows != (int64_t)cv->batch * cv->chunk)
+      return fail(PK_ERR_INVALID, "%s: rows %d x n %d are not conv's %d streams x %d frames x 2 x %d", what, a->rows, a->n,
+                  cv->batch, cv->chunk, cv->d_model);
+    if (cv->num_slots <= 0 || cv->num_layers <= 0 || cv->layer < 0 || cv->layer >= cv->num_layers ||
+        (!cv->slots && cv->batch > cv->num_slots))
+      return fail(PK_ERR_INVALID, "%s: layer %d / layers %d / slots %d / batch %d out of range", what, cv->layer,
+                  cv->num_layers, cv->num_slots, cv->batch);
+  }
   if (a->rows == 0) return PK_OK;
   const void* ptrs[4] = {a->x, a->weight, a->out, a->bias ? a->bias : a->weight};
   for (const void* q : ptrs) {
     if (!q) return fail(PK_ERR_INVALID, "%s: a tensor pointer is NULL", what);
     if (!aligned16(q)) return fail(PK_ERR_INVALID, "%s: tensors must be 16-byte aligned", what);
   }
+  if (glu) {
+    const void* need[3] = {cv->cache, cv->dw_weight, cv->dw_bias ? cv->dw_bias : cv->dw_weight};
+    for (const void* q : need) {
+      if (!q) return fail(PK_ERR_INVALID, "%s: a tensor pointer is NULL", what);
+      if (!aligned16(q)) return fail(PK_ERR_INVALID, "%s: tensors must be 16-byte aligned", what);
+    }
+  }
   if (!row_ok(a->rows, a->x_stride, a->k) || !row_ok(a->n, a->weight_stride, a->k) ||
-      !row_ok(a->rows, a->out_stride, a->n))
+      !row_ok(a->rows, a->out_stride, glu ? a->n / 2 : a->n))
     return fail(PK_ERR_INVALID, "%s: row strides must be multiples of 8 elements, at least the row, and a tensor below "
                 "2^31 elements", what);
   LinK<ST> k{};
@@ -728,10 +1009,26 @@ int linear_typed(const pk_linear_args* a, hipStream_t s) {
   k.M = a->rows;
   k.N = a->n;
   k.K = a->k;
+  if (glu) {
+    k.y = static_cast<float*>(a->out);
+    k.y_s = a->out_stride;
+    k.cache = static_cast<ST*>(cv->cache);
+    k.slots = cv->slots;
+    k.pad = cv->pad_mask;
+    k.lengths = cv->lengths;
+    k.len_scalar = cv->length_scalar;
+    k.dw = static_cast<const ST*>(cv->dw_weight);
+    k.dwb = static_cast<const ST*>(cv->dw_bias);
+    k.num_slots = cv->num_slots;
+    k.num_layers = cv->num_layers;
+    k.layer = cv->layer;
+    k.T = cv->chunk;
+    k.batch = cv->batch;
+  }
   if (a->prologue != PK_PRO_NONE) {
-    if (a->prologue < PK_PRO_NONE || a->prologue > PK_PRO_RESIDUAL_NORM2)
+    if (a->prologue < PK_PRO_NONE || a->prologue > PK_PRO_NORM_SILU)
       return fail(PK_ERR_INVALID, "%s: unknown prologue %d", what, a->prologue);
-    const bool res = a->prologue != PK_PRO_NORM, two = a->prologue == PK_PRO_RESIDUAL_NORM2;
+    const bool res = a->prologue == PK_PRO_RESIDUAL_NORM || a->prologue == PK_PRO_RESIDUAL_NORM2, two = a->prologue == PK_PRO_RESIDUAL_NORM2;
     const void* need[7] = {a->ln_weight, a->ln_bias, a->x, res ? a->branch : a->x, res ? a->residual_out : a->x,
                            two ? a->ln0_weight : a->x, two ? a->ln0_bias : a->x};
     for (const void* q : need) {
@@ -759,22 +1056,43 @@ int linear_typed(const pk_linear_args* a, hipStream_t s) {
   }
   DeviceGuard dg(a->device);
   if (!dg.ok) return fail(PK_ERR_HIP, "%s: cannot select device %d", what, a->device);
+  const int cus = cu_count();
   if (a->prologue != PK_PRO_NONE) {
-    const int bn = norm_form(k.M, k.N, k.K, cu_count());
+    const int bn = norm_form(k.M, k.N, k.K, cus, glu ? k.T : 1);
+    const bool silu = a->activation == PK_ACT_SILU, none = a->activation == PK_ACT_NONE;
+    if (a->prologue == PK_PRO_NORM_SILU) {
+      if (!none || (k.K != 512 && k.K != 1024)) return fail(PK_ERR_UNSUPPORTED, "%s: PK_PRO_NORM_SILU is built for k 512 and 1024 without activation", what);
+      k.xf = static_cast<const float*>(a->x);
+      if (bn) return launch_norm_k<ST, kProNormSilu, kEpiNone>(k, bn, s);
+      if (!a->residual_out || !aligned16(a->residual_out) || !row_ok(k.M, a->residual_out_stride, k.K))
+        return fail(PK_ERR_INVALID, "%s: PK_PRO_NORM_SILU on this many rows needs residual_out", what);
+      ST* const h = static_cast<ST*>(a->residual_out);
+      const dim3 grid((unsigned)((k.M + 3) / 4));
+      if (k.K == 512)
+        hipLaunchKernelGGL((norm_silu_kernel<ST, 1>), grid, dim3(256), 0, s, k.xf, k.x_s, k.lnw, k.lnb, k.eps, h, a->residual_out_stride, k.M);
+      else
+        hipLaunchKernelGGL((norm_silu_kernel<ST, 2>), grid, dim3(256), 0, s, k.xf, k.x_s, k.lnw, k.lnb, k.eps, h, a->residual_out_stride, k.M);
+      const int rc = check_launch(what);
+      if (rc != PK_OK) return rc;
+      k.x = h;
+      k.x_s = a->residual_out_stride;
+      return launch_form<ST, kEpiNone>(k, best_form(k.M, k.N, k.K, cus), s);
+    }
     if (!bn) return fail(PK_ERR_UNSUPPORTED, "%s: %d rows of %d -> %d are past the norm form (pk_linear_takes_norm)", what, k.M, k.K, k.N);
-    const bool silu = a->activation == PK_ACT_SILU;
     switch (a->prologue) {
       case PK_PRO_NORM:
         if (!silu) return fail(PK_ERR_UNSUPPORTED, "%s: PK_PRO_NORM is built with SiLU", what);
         return launch_norm_k<ST, kProNorm, kEpiSilu>(k, bn, s);
       case PK_PRO_RESIDUAL_NORM:
+        if (glu) return launch_norm_k<ST, kProResNorm, kEpiConv>(k, bn, s);
         return silu ? launch_norm_k<ST, kProResNorm, kEpiSilu>(k, bn, s) : launch_norm_k<ST, kProResNorm, kEpiNone>(k, bn, s);
       default:
         if (!silu) return fail(PK_ERR_UNSUPPORTED, "%s: PK_PRO_RESIDUAL_NORM2 is built with SiLU", what);
         return launch_norm_k<ST, kProResNorm2, kEpiSilu>(k, bn, s);
     }
   }
-  const int form = best_form(k.M, k.N, k.K, cu_count());
+  if (glu) return launch_conv_form(k, cus, s);
+  const int form = best_form(k.M, k.N, k.K, cus);
   if (a->activation == PK_ACT_SILU) return launch_form<ST, kEpiSilu>(k, form, s);
   return launch_form<ST, kEpiNone>(k, form, s);
 }
@@ -791,8 +1109,8 @@ int linear_any(const pk_linear_args* a, hipStream_t s) {
 }  // namespace
 }  // namespace pk
 
-extern "C" int pk_linear_takes_norm(int32_t rows, int32_t n, int32_t k) {
-  return rows > 0 && n > 0 && pk::norm_form(rows, n, k, pk::cu_count()) > 0 ? 1 : 0;
+extern "C" int pk_linear_takes_norm(int32_t rows, int32_t n, int32_t k, int32_t chunk) {
+  return rows > 0 && n > 0 && chunk > 0 && pk::norm_form(rows, n, k, pk::cu_count(), chunk) > 0 ? 1 : 0;
 }
 
 extern "C" int pk_linear(const pk_linear_args* args, int32_t count, void* stream) {

@@ -30,11 +30,13 @@ PK_ERR_STATE = -5
 
 ACT_NONE = 0
 ACT_SILU = 1
+ACT_GLU_CONV = 2
 
 PRO_NONE = 0
 PRO_NORM = 1
 PRO_RESIDUAL_NORM = 2
 PRO_RESIDUAL_NORM2 = 3
+PRO_NORM_SILU = 4
 
 PCM_S16 = 0
 PCM_F32 = 1
@@ -234,6 +236,7 @@ class LinearArgs(ctypes.Structure):
         ("ln0_eps", ctypes.c_float),
         ("residual_out", c_void_p),
         ("residual_out_stride", c_int64),
+        ("conv", POINTER(ConvArgs)),
     ]
 
 
@@ -365,7 +368,7 @@ SIGNATURES = {
     "pk_streaming_mask": (c_int, [POINTER(MaskArgs), c_void_p]),
     "pk_conv_step": (c_int, [POINTER(ConvArgs), c_void_p]),
     "pk_residual_norm": (c_int, [POINTER(ResNormArgs), c_void_p]),
-    "pk_linear_takes_norm": (c_int, [c_int32, c_int32, c_int32]),
+    "pk_linear_takes_norm": (c_int, [c_int32, c_int32, c_int32, c_int32]),
     "pk_linear": (c_int, [POINTER(LinearArgs), c_int32, c_void_p]),
     "pk_fe_step": (c_int, [POINTER(FeArgs), c_void_p]),
     "pk_subsample": (c_int, [POINTER(SubArgs), c_void_p]),

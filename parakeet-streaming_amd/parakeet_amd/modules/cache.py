@@ -363,6 +363,17 @@ class ModelCache:
             eps=eps,
         )
 
+    def glu_conv(self, layer_idx: int, x, branch, norm, weight, bias, dw_weight, dw_bias, pad_mask):
+        """``ops.glu_conv`` on this batch's conv state of a layer."""
+        if x.shape[0] != self.batch_size:
+            raise ValueError(f"batch {x.shape[0]} != cache rows {self.batch_size}")
+        if not 0 <= layer_idx < self.num_layers:
+            raise IndexError(f"layer {layer_idx} out of range [0, {self.num_layers})")
+        return ops.glu_conv(
+            x, branch, norm, weight, bias, dw_weight, dw_bias, self.conv_frames, layer_idx,
+            None if self._prefix else self._slots_i32, pad_mask,
+        )
+
     # ------------------------------------------------------------------ reset
     def reset(self) -> None:
         """All slots empty (parakeet/modules/cache.py:55-58)."""

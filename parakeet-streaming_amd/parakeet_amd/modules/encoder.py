@@ -203,11 +203,14 @@ class ConformerLayer(nn.Module):
             x, self.norm_self_att, attn.qkv.weight, attn.qkv.bias, branch=ops.module_linear(h, ff1.linear2), alpha=0.5, in_place=own
         )
         a = attn.attend(qkv, pos_emb, attn_mask, cache)
-        r, h = ops.norm_linear(
-            r, self.norm_conv, conv.pointwise_conv1.weight.squeeze(-1), conv.pointwise_conv1.bias, branch=a, in_place=True
-        )
-        c, conv_cache = conv.after_pointwise1(h, pad_mask=pad_mask, cache=cache.conv_ref(self.layer_idx))
-        cache.update_conv_cache(self.layer_idx, conv_cache)
+        p1, p2, dw, bn = conv.pointwise_conv1, conv.pointwise_conv2, conv.depthwise_conv, conv.batch_norm
+        w1, w2 = p1.weight.squeeze(-1), p2.weight.squeeze(-1)
+        if ops.glu_conv_applies(r, w1, p1.bias, w2, p2.bias, dw, bn) and cache.conv_frames.dtype == r.dtype:
+            r, y = cache.glu_conv(self.layer_idx, r, a, self.norm_conv, w1, p1.bias, dw.weight, dw.bias, pad_mask)
+            c = ops.norm_silu_linear(y, bn, w2, p2.bias)
+        else:
+            r, h = ops.norm_linear(r, self.norm_conv, w1, p1.bias, branch=a, in_place=True)
+            c, _ = conv.after_pointwise1(h, pad_mask=pad_mask, cache=cache.conv_ref(self.layer_idx))
         r, h = ops.norm_linear(r, self.norm_feed_forward2, ff2.linear1.weight, ff2.linear1.bias, branch=c, silu=True, in_place=True)
         return ops.Pending(r, ops.module_linear(h, ff2.linear2), self.norm_out, 0.5)
 

@@ -701,7 +701,7 @@ def norm_linear(
     n, k = weight.shape
     dev, dt = first.device, first.dtype
     rows = first.numel() // k
-    if not (lib().pk_linear_takes_norm(rows, n, k) and (silu or branch is not None) and layer_applies(dt, dev, rows, weight, bias, silu)):
+    if not (lib().pk_linear_takes_norm(rows, n, k, 1) and (silu or branch is not None) and layer_applies(dt, dev, rows, weight, bias, silu)):
         if pend is not None:
             r, h = residual_norm2(pend, norm)
         elif branch is not None:
@@ -733,6 +733,97 @@ def norm_linear(
             a.prologue, a.alpha = _lib.PRO_RESIDUAL_NORM, alpha
     check(lib().pk_linear(ctypes.byref(a), 1, _stream(dev)), "pk_linear")
     return r, out
+
+
+def glu_conv_applies(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, w2: torch.Tensor, b2: torch.Tensor | None, dw: torch.nn.Module, norm: torch.nn.Module) -> bool:
+    """Whether :func:`glu_conv` and :func:`norm_silu_linear` take a convolution
+    module's step on x [B, T, D] (its layer accepted by the caller's checks)."""
+    B, T, D = x.shape
+    w = dw.weight
+    return (
+        D in (512, 1024)
+        and 1 <= T <= 16
+        and tuple(w.shape) == (D, 1, 9)
+        and w.dtype == x.dtype
+        and w.device == x.device
+        and w.is_contiguous()
+        and w.data_ptr() % 16 == 0
+        and (dw.bias is None or (dw.bias.dtype == x.dtype and dw.bias.is_contiguous() and dw.bias.data_ptr() % 16 == 0))
+        and norm_applies(norm, x)
+        and weight.shape[0] == 2 * D
+        and layer_applies(x.dtype, x.device, B * T, weight, bias)
+        and layer_applies(x.dtype, x.device, B * T, w2, b2)
+    )
+
+
+def glu_conv(
+    x: torch.Tensor,
+    branch: torch.Tensor,
+    norm: torch.nn.LayerNorm,
+    weight: torch.Tensor,
+    bias: torch.Tensor | None,
+    dw_weight: torch.Tensor,
+    dw_bias: torch.Tensor | None,
+    conv_cache: torch.Tensor,
+    layer: int,
+    slots: torch.Tensor | None,
+    pad_mask: torch.Tensor | None,
+) -> tuple[torch.Tensor, torch.Tensor]:
+    """``r = x + branch`` and the convolution module up to its LayerNorm
+    (convolution.py:37-47,150-155): pointwise convolution of ``norm(r)``, GLU,
+    causal depthwise convolution with ``conv_cache`` [slots, layers, 8, D] updated
+    in place.  Returns r (x itself where the update is a launch of its own) and
+    the convolution's fp32 output [B, T, D]."""
+    B, T, D = x.shape
+    rows, dev, dt = B * T, x.device, x.dtype
+    fused = bool(lib().pk_linear_takes_norm(rows, 2 * D, D, T))
+    y = torch.empty((B, T, D), dtype=torch.float32, device=dev)
+    a, c = LinearArgs(), ConvArgs()
+    if fused:
+        x, branch = _aligned_rows(x), _aligned_rows(branch)
+        r = torch.empty_like(x)
+        _linear_args(a, _DTYPES[dt], dev, x, rows, weight, bias, y, False)
+        a.prologue, a.alpha = _lib.PRO_RESIDUAL_NORM, 1.0
+        a.branch, a.branch_stride = branch.data_ptr(), D
+        a.residual_out, a.residual_out_stride = r.data_ptr(), D
+        a.ln_weight, a.ln_bias, a.ln_eps = _ln(norm)
+    else:
+        r, h = residual_norm(x, branch, norm.weight, norm.bias, eps=norm.eps, in_place=True)
+        _linear_args(a, _DTYPES[dt], dev, h, rows, weight, bias, y, False)
+    a.activation, a.out_stride = _lib.ACT_GLU_CONV, D
+    c.batch, c.chunk, c.d_model, c.kernel = B, T, D, 9
+    c.cache, c.num_slots, c.num_layers, c.layer = conv_cache.data_ptr(), conv_cache.shape[0], conv_cache.shape[1], int(layer)
+    c.slots = slots.data_ptr() if slots is not None else None
+    if pad_mask is not None:
+        if pad_mask.dtype not in (torch.bool, torch.uint8) or tuple(pad_mask.shape) != (B, T):
+            raise ValueError(f"pad_mask must be bool/uint8 [{B}, {T}]")
+        pad_mask = pad_mask.contiguous()
+        if pad_mask.device != dev:
+            raise ValueError("pad_mask on a different device")
+        c.pad_mask = pad_mask.data_ptr()
+    else:
+        c.length_scalar = T
+    c.dw_weight, c.dw_bias = dw_weight.data_ptr(), dw_bias.data_ptr() if dw_bias is not None else None
+    a.conv = ctypes.pointer(c)
+    check(lib().pk_linear(ctypes.byref(a), 1, _stream(dev)), "pk_linear")
+    return r, y
+
+
+def norm_silu_linear(y: torch.Tensor, norm: torch.nn.LayerNorm, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
+    """``linear(SiLU(norm(y)))`` of fp32 y [..., D] in the weight's dtype
+    (convolution.py:156-158)."""
+    n, k = weight.shape
+    rows, dev, dt = y.numel() // k, y.device, weight.dtype
+    out = torch.empty((*y.shape[:-1], n), dtype=dt, device=dev)
+    a = LinearArgs()
+    _linear_args(a, _DTYPES[dt], dev, y, rows, weight, bias, out, False)
+    a.prologue = _lib.PRO_NORM_SILU
+    a.ln_weight, a.ln_bias, a.ln_eps = _ln(norm)
+    if not lib().pk_linear_takes_norm(rows, n, k, 1):
+        h = torch.empty((rows, k), dtype=dt, device=dev)
+        a.residual_out, a.residual_out_stride = h.data_ptr(), k
+    check(lib().pk_linear(ctypes.byref(a), 1, _stream(dev)), "pk_linear")
+    return out
 
 
 def feed_forward(x: torch.Tensor, w1: torch.Tensor, b1: torch.Tensor | None, w2: torch.Tensor, b2: torch.Tensor | None) -> torch.Tensor:

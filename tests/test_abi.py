@@ -241,3 +241,28 @@ def test_linear_args_validated_before_launch():
     a.dtype, a.rows = _lib.DTYPE_BF16, 0  # nothing to do: no pointer is read
     assert L.pk_linear(ctypes.byref(a), 1, None) == _lib.PK_OK
     assert L.pk_linear(ctypes.byref(a), 0, None) == _lib.PK_OK
+    buf = ctypes.create_string_buffer(64)
+    addr = (ctypes.addressof(buf) + 15) & ~15  # aligned, never dereferenced on a failed check
+    a.rows, a.n, a.activation = 4, 1024, _lib.ACT_GLU_CONV
+    a.x = a.weight = a.out = addr
+    assert L.pk_linear(ctypes.byref(a), 1, None) == _lib.PK_ERR_INVALID  # no convolution
+    c = _lib.ConvArgs()
+    c.batch, c.chunk, c.d_model, c.kernel, c.num_slots, c.num_layers = 2, 2, 512, 7, 4, 1
+    a.conv = ctypes.pointer(c)
+    assert L.pk_linear(ctypes.byref(a), 1, None) == _lib.PK_ERR_UNSUPPORTED  # 7 taps
+    c.kernel, c.chunk, c.batch = 9, 17, 1
+    assert L.pk_linear(ctypes.byref(a), 1, None) == _lib.PK_ERR_UNSUPPORTED  # 17 frames
+    c.chunk, c.batch = 2, 3  # 6 frames of 4 rows
+    assert L.pk_linear(ctypes.byref(a), 1, None) == _lib.PK_ERR_INVALID
+    c.batch, c.layer = 2, 1  # layer out of range
+    assert L.pk_linear(ctypes.byref(a), 1, None) == _lib.PK_ERR_INVALID
+    c.layer = 0
+    assert L.pk_linear(ctypes.byref(a), 1, None) == _lib.PK_ERR_INVALID  # NULL cache
+    a.activation, a.n, a.prologue = _lib.ACT_NONE, 512, 7
+    assert L.pk_linear(ctypes.byref(a), 1, None) == _lib.PK_ERR_INVALID  # unknown prologue
+    a.prologue = _lib.PRO_RESIDUAL_NORM
+    assert L.pk_linear(ctypes.byref(a), 1, None) == _lib.PK_ERR_INVALID  # NULL branch
+    a.branch = a.ln_weight = a.ln_bias = a.residual_out = addr
+    a.branch_stride = a.residual_out_stride = 512
+    assert L.pk_linear(ctypes.byref(a), 1, None) == _lib.PK_ERR_INVALID  # residual_out is x
+    assert "must not be x" in _lib.last_error()

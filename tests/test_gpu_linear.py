@@ -210,3 +210,62 @@ def test_encoder_fused_layers_match_module_by_module(cuda, streams):
                 h.remove()
             for t in (b, c):  # three layers of independent fp16 roundings
                 assert float((t.float() - a.float()).norm() / a.float().norm()) <= 4e-3
+
+
+# streams of 1, 2, 3, 14 and 16 frames: several streams a tile and a remainder, a
+# tile of 16 rows not filled; few rows (the norm form) and the tile forms
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,T,D", [(1, 2, 512), (5, 3, 512), (70, 2, 512), (40, 1, 512), (7, 14, 1024), (3, 16, 512), (33, 2, 1024),
+                                   (60, 14, 1024), (300, 2, 512), (700, 3, 512), (1025, 2, 512), (900, 1, 1024)])
+def test_glu_conv_matches_its_parts(cuda, dtype, B, T, D):
+    """pk_linear with the depthwise convolution, then with the norm and SiLU,
+    against float64 and pk_conv_step over two steps: shuffled slots, one padded
+    frame.  The cache holds GLU outputs rounded once (fused: from fp32 values and
+    gates; parts: from values rounded first), so the two agree within the
+    roundings of value and gate: 3 roundings of max(1, |value|)."""
+    print(f"\n[glu-conv] {dtype} B={B} T={T} D={D}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(B * 31 + T)
+    Ly, layer, S, eps = 2, 1, B + 3, EPS[dtype]
+    w1 = (torch.randn(2 * D, D, generator=g, device=cuda) / math.sqrt(D)).to(dtype)
+    b1 = (0.1 * torch.randn(2 * D, generator=g, device=cuda)).to(dtype)
+    w2 = (torch.randn(D, D, generator=g, device=cuda) / math.sqrt(D)).to(dtype)
+    dw = (torch.randn(D, 1, 9, generator=g, device=cuda) / 3).to(dtype)
+    db = (0.1 * torch.randn(D, generator=g, device=cuda)).to(dtype)
+    norm, bn = _norm(D, dtype, cuda, g), _norm(D, dtype, cuda, g)
+    slots = torch.randperm(S, generator=g, device=cuda)[:B].to(torch.int32)
+    cache = torch.randn(S, Ly, 8, D, generator=g, device=cuda).to(dtype)
+    pad = torch.zeros(B, T, dtype=torch.bool, device=cuda)
+    pad[B // 2, T - 1] = True
+    for step in range(2):
+        x = torch.randn(B, T, D, generator=g, device=cuda).to(dtype)
+        br = torch.randn(B, T, D, generator=g, device=cuda).to(dtype)
+        mine, parts = cache.clone(), cache.clone()
+        want_r = x + br
+        r, y = ops.glu_conv(x.clone(), br, norm, w1, b1, dw, db, mine, layer, slots, pad)
+        assert torch.equal(r, want_r) and y.dtype == torch.float32
+        # float64 from this step's cache and the module's own roundings of the norm
+        h = F.layer_norm(want_r.double(), (D,), norm.weight.double(), norm.bias.double(), norm.eps)
+        v, ga = (h.to(dtype).double() @ w1.double().T + b1.double()).chunk(2, -1)
+        glu = (v * torch.sigmoid(ga)).masked_fill(pad[..., None], 0.0)
+        win = torch.cat([cache[slots.long(), layer].double(), glu], 1)
+        ref = sum(win[:, k : k + T] * dw[:, 0, k].double() for k in range(9)) + db.double()
+        assert float((y.double() - ref).norm() / ref.norm()) <= 2 * eps
+        new = mine[slots.long(), layer]
+        assert bool(((new.double() - win[:, -8:]).abs() <= 3 * eps * win[:, -8:].abs().clamp(min=1.0)).all())
+        others = torch.ones(S, dtype=torch.bool, device=cuda)
+        others[slots.long()] = False
+        assert torch.equal(mine[others], cache[others]) and torch.equal(mine[:, 0], cache[:, 0])
+        if T < 8:  # rows that only move keep their bits
+            assert torch.equal(new[:, : 8 - T], cache[slots.long(), layer][:, T:])
+        assert bool((new[B // 2, -1] == 0).all())
+        # against the separate launches
+        _, hh = ops.residual_norm(x, br, norm.weight, norm.bias, eps=norm.eps)
+        z = ops.conv_step(ops.linear(hh, w1, b1), parts, dw, bn.weight, bn.bias, layer=layer, slots=slots, pad_mask=pad, dw_bias=db, eps=bn.eps)
+        out = ops.norm_silu_linear(y, bn, w2, None)
+        sep = ops.linear(z, w2, None)
+        exact = F.silu(F.layer_norm(ref, (D,), bn.weight.double(), bn.bias.double(), bn.eps)) @ w2.double().T
+        e_new, e_old = (float((t.double() - exact).norm() / exact.norm()) for t in (out, sep))
+        print(f"  error against float64: fused {e_new:.2e}, parts {e_old:.2e}", flush=True)
+        assert e_new <= 1.05 * e_old + 0.1 * eps
+        cache = mine
