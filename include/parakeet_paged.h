@@ -410,7 +410,7 @@ typedef struct pk_linear_args {
   const pk_conv_args* conv;
 } pk_linear_args;
 /* 1 if pk_linear takes a prologue with a residual or PK_PRO_NORM for this layer on
- * the current device; chunk: PK_ACT_GLU_CONV's frames a stream, else 1 */
+ * the current device; chunk: PK_ACT_GLU_CONV's frames a stream, else 0 */
 int pk_linear_takes_norm(int32_t rows, int32_t n, int32_t k, int32_t chunk);
 int pk_linear(const pk_linear_args* args, int32_t count, void* stream);
 

@@ -3,9 +3,7 @@
 //
 //   out = act( x W^T + bias )
 //
-//   lin_row_kernel   a few rows: 16 x 16 outputs a workgroup, K split over its
-//                    waves, both operands straight from memory into registers
-//   lin_tile_kernel  16 x 32 to 256 x 256 outputs a workgroup, both operands
+//   lin_tile_kernel  16 x 16 to 256 x 256 outputs a workgroup, both operands
 //                    staged in LDS by buffer loads
 //   lin_norm_kernel  few rows, with the residual update and LayerNorm (or two)
 //                    that make x in the same launch (encoder.py:58-81)
@@ -83,6 +81,7 @@ struct LinK {
   const ST* dw;   // [D][kTaps]
   const ST* dwb;  // [D] or nullptr
   int32_t num_slots, num_layers, layer, T, batch;
+  int32_t per;  // streams a tile
 };
 
 template <typename ST>
@@ -104,112 +103,23 @@ __device__ static inline float epi_act(float v) {
   return v;
 }
 
-// Tile (m, n) of workgroup i: workgroup i runs on XCD i % 8.  xm > 0: the XCDs
-// take an xm x 8/xm grid of equal blocks of tiles (the host picks xm so that a
+// Tile (m, n) of a workgroup: workgroups go to the XCDs in turn in launch order.
+// xm > 0: grid (8, row tiles, column tiles of an XCD): the XCDs take an xm x 8/xm
+// grid of equal blocks of tiles (the host picks xm, a power of two, so that a
 // block's rows and weight columns together are fewest: what each XCD's L2
-// fetches); xm == 0 (the tiles do not divide): contiguous runs, rows fastest.
-__device__ static inline void xcd_tile(int i, int total, int mtiles, int xm, int& m, int& n) {
-  const int x = i & 7, j = i >> 3;
+// fetches).  xm == 0 (the tiles do not divide): grid (tiles), contiguous runs of
+// them an XCD, rows fastest.
+__device__ static inline void xcd_tile(int mtiles, int xm, int& m, int& n) {
   if (xm > 0) {
-    const int ml = mtiles / xm, nl = total / mtiles / (8 / xm);
-    m = (x % xm) * ml + j % ml;
-    n = (x / xm) * nl + j / ml;
+    const int x = blockIdx.x, lg = xm == 1 ? 0 : xm == 2 ? 1 : xm == 4 ? 2 : 3;
+    m = (x & (xm - 1)) * gridDim.y + blockIdx.y;
+    n = (x >> lg) * gridDim.z + blockIdx.z;
     return;
   }
-  const int q = total >> 3, r = total & 7;
-  const int t = x * q + min(x, r) + j;
+  const int total = gridDim.x, x = blockIdx.x & 7, j = blockIdx.x >> 3;
+  const int t = x * (total >> 3) + min(x, total & 7) + j;
   m = t % mtiles;
   n = t / mtiles;
-}
-
-// Bound by latency: the launch, one round trip to memory and the waves' sum; 16
-// rows x 512 -> 512 outputs takes 3.4 us in a graph (2.6 us of it the launch and
-// the round trip) against 4.2 for torch's library GEMM, 60 rows 3.4 against 6.1.
-// An operand read touches 16 rows x 64 bytes, half of each 128-byte line, which
-// limits a CU to about 37 GB/s: larger tiles take lin_tile_kernel.
-//
-// One workgroup: 16*MT rows x 16*NT outputs; wave w multiplies columns
-// [w K/NW, (w+1) K/NW) of both operands and the waves' partial sums are added
-// in LDS in wave order.  W is the product's A operand (its rows the 16 M rows)
-// and x the B operand, so a lane ends with 4 consecutive outputs of one row.
-template <typename ST, int MT, int NT, int NW, int EPI>
-__global__ void __launch_bounds__(64 * NW) lin_row_kernel(const LinK<ST> p) {
-#pragma clang fp contract(off)
-  constexpr int ROWS = 16 * MT;
-  constexpr int kRed = NW * MT * NT * 64 * 16;
-  __shared__ __align__(16) unsigned char smem[kRed];
-
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int l16 = lane & 15, kg = lane >> 4;
-  int mt_i, nt_i;
-  xcd_tile(blockIdx.x, gridDim.x, p.mtiles, p.xm, mt_i, nt_i);
-  const int row0 = mt_i * ROWS, n0 = nt_i * 16 * NT;
-
-  f32x4_t acc[MT][NT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int n = 0; n < NT; ++n) acc[m][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  constexpr int UK = 4;  // 32-column steps a chunk
-  const int kw = p.K / NW;
-  const ST* wp[NT];
-  const ST* xp[MT];
-#pragma unroll
-  for (int n = 0; n < NT; ++n) wp[n] = p.w + (int64_t)(n0 + 16 * n + l16) * p.w_s + wave * kw + kg * 8;
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-    xp[m] = p.x + (int64_t)min(row0 + 16 * m + l16, p.M - 1) * p.x_s + wave * kw + kg * 8;
-  u32x4 wf[2][UK][NT], xf[2][UK][MT];
-  auto load = [&](int b, int k) {
-#pragma unroll
-    for (int u = 0; u < UK; ++u) {
-#pragma unroll
-      for (int n = 0; n < NT; ++n) wf[b][u][n] = ld16(wp[n] + k + 32 * u);
-#pragma unroll
-      for (int m = 0; m < MT; ++m) xf[b][u][m] = ld16(xp[m] + k + 32 * u);
-    }
-  };
-  auto mul = [&](int b) {
-#pragma unroll
-    for (int u = 0; u < UK; ++u)
-#pragma unroll
-      for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int n = 0; n < NT; ++n) acc[m][n] = MmaL<ST>::k32(wf[b][u][n], xf[b][u][m], acc[m][n]);
-  };
-  // two chunks in registers: the next one's loads are in flight during a chunk's products
-  load(0, 0);
-  for (int k = 0; k < kw; k += 64 * UK) {
-    if (k + 32 * UK < kw) load(1, k + 32 * UK);
-    __builtin_amdgcn_sched_barrier(0);
-    mul(0);
-    if (k + 64 * UK < kw) load(0, k + 64 * UK);
-    __builtin_amdgcn_sched_barrier(0);
-    if (k + 32 * UK < kw) mul(1);
-  }
-  f32x4_t* const red = reinterpret_cast<f32x4_t*>(smem);  // [NW][MT*NT][64]
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int n = 0; n < NT; ++n) red[((wave * MT + m) * NT + n) * 64 + lane] = acc[m][n];
-  __syncthreads();
-  for (int i = threadIdx.x; i < MT * NT * 64; i += 64 * NW) {
-    f32x4_t s = red[i];
-#pragma unroll
-    for (int w = 1; w < NW; ++w) s += red[w * MT * NT * 64 + i];
-    const int il = i & 63, t = i >> 6;
-    const int row = row0 + 16 * (t / NT) + (il & 15);
-    const int n = n0 + 16 * (t % NT) + 4 * (il >> 4);
-    float f[4] = {s.x, s.y, s.z, s.w};
-    if (p.bias) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) f[e] += from_st(p.bias[n + e]);
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) f[e] = epi_act<EPI>(f[e]);
-    if (row < p.M) *reinterpret_cast<u32x2*>(p.out + (int64_t)row * p.out_s + n) = pack4<ST>(f);
-  }
 }
 
 // `bytes` readable from base; a read past them gives zeros
@@ -312,7 +222,7 @@ __device__ static inline ST* conv_cache(const LinK<ST>& p, int b, int c) {
 }
 template <typename ST, int CB>
 __device__ static inline void conv_load(const LinK<ST>& p, int i, int mt_i, int c0, ConvItem& it) {
-  const int per = p.rpt / p.T;
+  const int per = p.per;
   const int s = i / (CB / 2), c = c0 + (i % (CB / 2)) * 2, b = mt_i * per + s;
   if (s >= per || b >= p.batch) return;
   const uint32_t* tp = reinterpret_cast<const uint32_t*>(p.dw + (int64_t)c * kTaps);  // c even: 4-byte aligned
@@ -376,7 +286,7 @@ __device__ static inline void store_conv(const LinK<ST>& p, unsigned char* smem,
     }
   }
   __syncthreads();
-  const int per = p.rpt / p.T;
+  const int per = p.per;
   for (int i = threadIdx.x; i < per * (CB / 2); i += NTH) {
     const int s = i / (CB / 2), cl = (i % (CB / 2)) * 2, c = c0 + cl, b = mt_i * per + s;
     if (b >= p.batch) break;  // streams ascend
@@ -433,10 +343,13 @@ __device__ static inline int w_row(int nt_i, int n, int N) {
 // low three bits, so the 16 rows of an operand read fall on distinct banks.
 // Small tiles split K over the waves (WK): each staged byte is then read from LDS
 // once or twice, and the sum over the waves costs one exchange at the end.
-// Bound by: latency up to about one tile a CU (128 x 512 -> 2048 with SiLU 4.5 us,
+// Bound by: latency up to about one tile a CU (128 x 512 -> 2048 with SiLU 4.2 us,
 // torch's GEMM and SiLU 10.2); LDS reads on the large forms (128 x 128 tiles take
 // 0.53 us a stage, of which 0.41 remain with the loads left out and 0.27 with the
-// products left out).  840 x 1024 -> 4096 with SiLU 13.6 us (518 TFLOP/s) against
+// products left out).  An operand read straight from memory (16 rows x 64 bytes
+// an instruction, half of each 128-byte line) moved 37 GB/s a CU against about 100
+// through LDS: 16 rows x 2048 -> 512 6.1 us so, 4.4 staged (torch's GEMM 7.9).
+// 840 x 1024 -> 4096 with SiLU 13.6 us (518 TFLOP/s) against
 // 21.3, 840 x 4096 -> 1024 17.1 against 19.5 for torch's.
 template <typename ST, int BM, int BN, int WM, int WN, int WK, int BK, int S, int EPI>
 __global__ void __launch_bounds__(64 * WM * WN * WK) lin_tile_kernel(const LinK<ST> p) {
@@ -459,7 +372,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) lin_tile_kernel(const LinK<
   const int l16 = lane & 15, kg = lane >> 4;
   const int wk = wave / (WM * WN), wm = (wave / WN) % WM, wn = wave % WN;
   int mt_i, nt_i;
-  xcd_tile(blockIdx.x, gridDim.x, p.mtiles, p.xm, mt_i, nt_i);
+  xcd_tile(p.mtiles, p.xm, mt_i, nt_i);
   const int row0 = mt_i * p.rpt, n0 = nt_i * BN;
 
   // chunk c of a stage: row c / CH of [x rows ; w rows], LDS position c % CH
@@ -570,7 +483,7 @@ __global__ void __launch_bounds__(64 * WN * WK) lin_norm_kernel(const LinK<ST> p
   const int l16 = lane & 15, kg = lane >> 4;
   const int wk = wave / WN, wn = wave % WN;
   int mt_i, nt_i;
-  xcd_tile(blockIdx.x, gridDim.x, p.mtiles, p.xm, mt_i, nt_i);
+  xcd_tile(p.mtiles, p.xm, mt_i, nt_i);
   const int row0 = mt_i * p.rpt, n0 = nt_i * BN;
 
   const __amdgpu_buffer_rsrc_t rw = bytes_rsrc(p.w, (uint32_t)((p.N - 1) * p.w_s + p.K) * 2u);
@@ -808,10 +721,14 @@ int xcd_split(int mtiles, int ntiles, int bm, int bn) {
 
 template <typename ST>
 dim3 tile_grid(LinK<ST>& k, int bm, int bn) {
-  k.rpt = k.T > 0 ? bm / k.T * k.T : bm;
+  k.per = k.T > 0 ? bm / k.T : 0;
+  k.rpt = k.T > 0 ? k.per * k.T : bm;
   k.mtiles = (k.M + k.rpt - 1) / k.rpt;
-  k.xm = xcd_split(k.mtiles, k.N / bn, bm, bn);
-  return dim3((unsigned)(k.mtiles * (k.N / bn)));
+  const int nt = k.N / bn;
+  k.xm = xcd_split(k.mtiles, nt, bm, bn);
+  if (k.xm > 0 && k.mtiles / k.xm <= 65535) return dim3(8u, (unsigned)(k.mtiles / k.xm), (unsigned)(nt / (8 / k.xm)));
+  k.xm = 0;
+  return dim3((unsigned)(k.mtiles * nt));
 }
 
 template <typename ST, int BM, int BN, int WM, int WN, int WK, int BK, int S, int EPI>
@@ -821,38 +738,35 @@ int launch_tile(LinK<ST> k, hipStream_t s) {
   return check_launch("pk_linear");
 }
 
-template <typename ST, int MT, int NT, int NW, int EPI>
-int launch_row(LinK<ST> k, hipStream_t s) {
-  const dim3 grid = tile_grid(k, 16 * MT, 16 * NT);
-  hipLaunchKernelGGL((lin_row_kernel<ST, MT, NT, NW, EPI>), grid, dim3(64 * NW), 0, s, k);
-  return check_launch("pk_linear");
-}
-
 // The forms without a prologue and what a launch of each takes, fitted to launches
 // in a graph with cold weights (K 512 - 4096, 16 - 3584 rows, bf16): `a` us plus `s`
-// us a 1024 columns for workgroups that are alone on their CU, 0.8 s for each
-// further one resident with it (`occ` fit), and again a - 2 for each further
-// round.  Small tiles read more bytes an output but put more CUs on a short
-// launch; the large ones are bound by LDS reads (a 64x32 wave tile reads 6 KB
-// for 8 products).  The cheapest by this model is launched; at the measured
-// shapes it is the fastest form or within 5% of it.
+// us a 1024 columns for workgroups that are alone on their CU, `m` of the latter
+// for each further one resident with it (`occ` fit), and again a - 2 for each
+// further round.  Small tiles read more bytes an output but put more CUs on a
+// short launch, and few long stages (up to 512 columns) wait for fewer barriers;
+// the large ones are bound by LDS reads (a 64x32 wave tile reads 6 KB for 8
+// products).  The cheapest by this model is launched; at the measured shapes it
+// is the fastest form or within 6% of it.
 struct Form {
   int bm, bn, kmul, occ;
-  float a, s;
+  float a, s, m;
 };
 constexpr Form kForms[] = {
-    {16, 16, 512, 4, 2.6f, 1.75f},    // lin_row_kernel
-    {16, 32, 256, 1, 3.45f, 0.97f},   //
-    {16, 32, 128, 2, 3.1f, 1.43f},    //
-    {32, 32, 128, 1, 3.0f, 1.9f},     //
-    {32, 32, 256, 1, 3.75f, 1.36f},   //
-    {32, 64, 128, 1, 3.3f, 2.6f},     //
-    {32, 64, 128, 1, 4.0f, 2.03f},    //
-    {64, 64, 64, 2, 3.75f, 3.35f},    //
-    {64, 128, 64, 2, 4.2f, 5.5f},     //
-    {128, 128, 64, 1, 5.0f, 8.5f},    //
-    {128, 128, 64, 2, 5.7f, 9.1f},    //
-    {256, 256, 64, 1, 10.0f, 28.0f},  //
+    {16, 16, 128, 4, 2.8f, 1.2f, 0.25f},   // 0
+    {16, 16, 512, 1, 3.0f, 0.7f, 0.f},     // 1
+    {16, 16, 256, 2, 2.95f, 0.85f, 0.5f},  // 2
+    {16, 32, 128, 3, 3.05f, 1.37f, 0.5f},  // 3
+    {16, 32, 512, 1, 3.5f, 0.88f, 0.f},    // 4
+    {32, 32, 128, 1, 3.05f, 1.95f, 0.f},   // 5
+    {32, 32, 128, 2, 3.45f, 1.75f, 0.6f},  // 6
+    {32, 32, 256, 1, 3.75f, 1.5f, 0.f},    // 7
+    {32, 64, 128, 2, 3.6f, 2.25f, 0.95f},  // 8
+    {32, 64, 256, 1, 4.05f, 2.0f, 0.f},    // 9
+    {64, 64, 64, 2, 3.75f, 3.35f, 0.8f},   // 10
+    {64, 128, 64, 2, 4.2f, 5.5f, 0.8f},    // 11
+    {128, 128, 64, 1, 5.0f, 8.5f, 0.f},    // 12
+    {128, 128, 64, 2, 5.7f, 9.1f, 0.8f},   // 13
+    {256, 256, 64, 1, 10.0f, 28.0f, 0.f},  // 14
 };
 constexpr int kNumForms = sizeof(kForms) / sizeof(kForms[0]);
 
@@ -863,7 +777,7 @@ float form_cost(const Form& f, int64_t M, int64_t N, int64_t K, int cus, int T =
   const int64_t tiles = (M + rpt - 1) / rpt * (N / f.bn);
   const int64_t per = (tiles + cus - 1) / cus, rounds = (per + f.occ - 1) / f.occ;
   const float c = f.s * (float)K / 1024.f;
-  return f.a + (float)(rounds - 1) * (f.a - 2.f) + (float)rounds * c + 0.8f * c * (float)(per - rounds);
+  return f.a + (float)(rounds - 1) * (f.a - 2.f) + (float)rounds * c + f.m * c * (float)(per - rounds);
 }
 
 int best_form(int64_t M, int64_t N, int64_t K, int cus) {
@@ -882,17 +796,20 @@ int best_form(int64_t M, int64_t N, int64_t K, int cus) {
 template <typename ST, int EPI>
 int launch_form(const LinK<ST>& k, int form, hipStream_t s) {
   switch (form) {
-    case 0: return launch_row<ST, 1, 1, 4, EPI>(k, s);
-    case 1: return launch_tile<ST, 16, 32, 1, 1, 8, 256, 5, EPI>(k, s);
-    case 2: return launch_tile<ST, 16, 32, 1, 1, 4, 128, 6, EPI>(k, s);
-    case 3: return launch_tile<ST, 32, 32, 2, 2, 2, 128, 6, EPI>(k, s);
-    case 4: return launch_tile<ST, 32, 32, 1, 1, 8, 256, 4, EPI>(k, s);
-    case 5: return launch_tile<ST, 32, 64, 2, 2, 2, 128, 5, EPI>(k, s);
-    case 6: return launch_tile<ST, 32, 64, 1, 2, 4, 128, 5, EPI>(k, s);
-    case 7: return launch_tile<ST, 64, 64, 2, 2, 2, 64, 4, EPI>(k, s);
-    case 8: return launch_tile<ST, 64, 128, 2, 4, 1, 64, 3, EPI>(k, s);
-    case 9: return launch_tile<ST, 128, 128, 2, 4, 1, 64, 4, EPI>(k, s);
-    case 10: return launch_tile<ST, 128, 128, 2, 2, 1, 64, 2, EPI>(k, s);
+    case 0: return launch_tile<ST, 16, 16, 1, 1, 4, 128, 4, EPI>(k, s);
+    case 1: return launch_tile<ST, 16, 16, 1, 1, 8, 512, 4, EPI>(k, s);
+    case 2: return launch_tile<ST, 16, 16, 1, 1, 4, 256, 4, EPI>(k, s);
+    case 3: return launch_tile<ST, 16, 32, 1, 1, 4, 128, 4, EPI>(k, s);
+    case 4: return launch_tile<ST, 16, 32, 1, 1, 8, 512, 3, EPI>(k, s);
+    case 5: return launch_tile<ST, 32, 32, 2, 2, 2, 128, 6, EPI>(k, s);
+    case 6: return launch_tile<ST, 32, 32, 1, 1, 4, 128, 4, EPI>(k, s);
+    case 7: return launch_tile<ST, 32, 32, 1, 1, 8, 256, 4, EPI>(k, s);
+    case 8: return launch_tile<ST, 32, 64, 1, 2, 4, 128, 3, EPI>(k, s);
+    case 9: return launch_tile<ST, 32, 64, 1, 2, 4, 256, 3, EPI>(k, s);
+    case 10: return launch_tile<ST, 64, 64, 2, 2, 2, 64, 4, EPI>(k, s);
+    case 11: return launch_tile<ST, 64, 128, 2, 4, 1, 64, 3, EPI>(k, s);
+    case 12: return launch_tile<ST, 128, 128, 2, 4, 1, 64, 4, EPI>(k, s);
+    case 13: return launch_tile<ST, 128, 128, 2, 2, 1, 64, 2, EPI>(k, s);
     default: return launch_tile<ST, 256, 256, 2, 4, 1, 64, 2, EPI>(k, s);
   }
 }
@@ -907,22 +824,26 @@ int launch_norm(LinK<ST> k, hipStream_t s) {
 // Outputs a workgroup of the norm form: the fewest that give no CU a second
 // tile (each tile normalises its rows again), 0 if none does.  In a graph, residual
 // update + norm + 512 -> 2048 with SiLU against pk_residual_norm and pk_linear: 16
-// rows (32 outputs) 5.0 us against 5.9, 128 rows (64) 5.3 against 6.9, 256 rows
-// (128) 6.1 against 7.7, 512 rows (128, two tiles a CU) 8.2 against 8.7; 1024 ->
-// 4096: 16 rows 7.3 against 7.6, 120 rows 8.9 against 9.6, 256 rows 12.7 against 11.2.
-int norm_form(int64_t M, int64_t N, int64_t K, int cus, int T = 1) {
+// rows (16 outputs) 4.1 us against 6.1, 64 rows (32) 4.5 against 6.7, 128 rows (64)
+// 5.1 against 7.0, 256 rows (128) 5.9 against 7.8; 1024 -> 4096: 16 rows (16) 6.2
+// against 7.8, 64 rows (64) 7.3 against 8.6, 120 rows (128) 8.4 against 9.7, 256
+// rows 12.7 against 11.2.  T: frames a stream of the convolution's tiles, 0 for none.
+int norm_form(int64_t M, int64_t N, int64_t K, int cus, int T) {
   if ((K != 512 && K != 1024) || T > 16) return 0;
-  const int rpt = 16 / T * T;
-  for (int bn = 32; bn <= 128; bn *= 2)
+  const int rpt = T > 0 ? 16 / T * T : 16;
+  for (int bn = T > 0 ? 32 : 16; bn <= 128; bn *= 2)
     if (N % bn == 0 && (M + rpt - 1) / rpt * (N / bn) <= cus) return bn;
   return 0;
 }
 
 template <typename ST, int KV, int PRO, int EPI>
 int launch_norm_form(const LinK<ST>& k, int bn, hipStream_t s) {
-  if (bn == 32) return launch_norm<ST, KV, 32, 1, 8, 256, 2, PRO, EPI>(k, s);
+  if constexpr (EPI != kEpiConv) {
+    if (bn == 16) return launch_norm<ST, KV, 16, 1, 8, 512, 2, PRO, EPI>(k, s);
+  }
+  if (bn == 32) return launch_norm<ST, KV, 32, 1, 8, 512, 2, PRO, EPI>(k, s);
   if (bn == 64) return launch_norm<ST, KV, 64, 2, 4, 128, 3, PRO, EPI>(k, s);
-  return launch_norm<ST, KV, 128, 4, 2, 64, 4, PRO, EPI>(k, s);
+  return launch_norm<ST, KV, 128, 4, 2, 128, 3, PRO, EPI>(k, s);
 }
 
 template <typename ST, int PRO, int EPI>
@@ -934,7 +855,7 @@ int launch_norm_k(const LinK<ST>& k, int bn, hipStream_t s) {
 // kEpiConv without a prologue: the tile forms whose waves hold values and gates
 template <typename ST>
 int launch_conv_form(const LinK<ST>& k, int cus, hipStream_t s) {
-  constexpr int forms[] = {6, 7, 8, 10};
+  constexpr int forms[] = {8, 10, 11, 13};
   int best = -1;
   float cost = 0.f;
   for (int f : forms) {
@@ -945,10 +866,10 @@ int launch_conv_form(const LinK<ST>& k, int cus, hipStream_t s) {
     }
   }
   switch (best) {
-    case 6: return launch_tile<ST, 32, 64, 1, 2, 4, 128, 5, kEpiConv>(k, s);
-    case 7: return launch_tile<ST, 64, 64, 2, 2, 2, 64, 4, kEpiConv>(k, s);
-    case 8: return launch_tile<ST, 64, 128, 2, 4, 1, 64, 3, kEpiConv>(k, s);
-    case 10: return launch_tile<ST, 128, 128, 2, 2, 1, 64, 2, kEpiConv>(k, s);
+    case 8: return launch_tile<ST, 32, 64, 1, 2, 4, 128, 3, kEpiConv>(k, s);
+    case 10: return launch_tile<ST, 64, 64, 2, 2, 2, 64, 4, kEpiConv>(k, s);
+    case 11: return launch_tile<ST, 64, 128, 2, 4, 1, 64, 3, kEpiConv>(k, s);
+    case 13: return launch_tile<ST, 128, 128, 2, 2, 1, 64, 2, kEpiConv>(k, s);
     default: return fail(PK_ERR_UNSUPPORTED, "pk_linear: no form for %d -> %d with the convolution", k.K, k.N);
   }
 }
@@ -1058,7 +979,7 @@ int linear_typed(const pk_linear_args* a, hipStream_t s) {
   if (!dg.ok) return fail(PK_ERR_HIP, "%s: cannot select device %d", what, a->device);
   const int cus = cu_count();
   if (a->prologue != PK_PRO_NONE) {
-    const int bn = norm_form(k.M, k.N, k.K, cus, glu ? k.T : 1);
+    const int bn = norm_form(k.M, k.N, k.K, cus, k.T);
     const bool silu = a->activation == PK_ACT_SILU, none = a->activation == PK_ACT_NONE;
     if (a->prologue == PK_PRO_NORM_SILU) {
       if (!none || (k.K != 512 && k.K != 1024)) return fail(PK_ERR_UNSUPPORTED, "%s: PK_PRO_NORM_SILU is built for k 512 and 1024 without activation", what);
@@ -1110,7 +1031,7 @@ int linear_any(const pk_linear_args* a, hipStream_t s) {
 }  // namespace pk
 
 extern "C" int pk_linear_takes_norm(int32_t rows, int32_t n, int32_t k, int32_t chunk) {
-  return rows > 0 && n > 0 && chunk > 0 && pk::norm_form(rows, n, k, pk::cu_count(), chunk) > 0 ? 1 : 0;
+  return rows > 0 && n > 0 && chunk >= 0 && pk::norm_form(rows, n, k, pk::cu_count(), chunk) > 0 ? 1 : 0;
 }
 
 extern "C" int pk_linear(const pk_linear_args* args, int32_t count, void* stream) {

@@ -173,7 +173,8 @@ __device__ static inline void st16_stream(ST* p, const u32x4 v) {
 // ---------------------------------------------------------------------------
 // lane-group all-reduce (sum) over G consecutive lanes with DPP row ops:
 // quad_perm [1,0,3,2], quad_perm [2,3,0,1], row_half_mirror, row_mirror, then
-// cross-row shuffles for groups wider than a DPP row.
+// row swaps between two registers (permlane16/32_swap: no trip through LDS as a
+// shuffle takes) for groups wider than a DPP row: lane l adds lane l ^ 16, l ^ 32.
 
 template <int CTRL>
 __device__ static inline float dpp_f(float v) {
@@ -187,8 +188,16 @@ __device__ static inline float group_sum(float v) {
   if constexpr (G >= 4) v += dpp_f<0x4E>(v);
   if constexpr (G >= 8) v += dpp_f<0x141>(v);
   if constexpr (G >= 16) v += dpp_f<0x140>(v);
-  if constexpr (G >= 32) v += __shfl_xor(v, 16);
-  if constexpr (G >= 64) v += __shfl_xor(v, 32);
+  if constexpr (G >= 32) {
+    const uint32_t u = __float_as_uint(v);
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+  if constexpr (G >= 64) {
+    const uint32_t u = __float_as_uint(v);
+    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
   return v;
 }
 

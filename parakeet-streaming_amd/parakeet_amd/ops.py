@@ -701,7 +701,7 @@ def norm_linear(
     n, k = weight.shape
     dev, dt = first.device, first.dtype
     rows = first.numel() // k
-    if not (lib().pk_linear_takes_norm(rows, n, k, 1) and (silu or branch is not None) and layer_applies(dt, dev, rows, weight, bias, silu)):
+    if not (lib().pk_linear_takes_norm(rows, n, k, 0) and (silu or branch is not None) and layer_applies(dt, dev, rows, weight, bias, silu)):
         if pend is not None:
             r, h = residual_norm2(pend, norm)
         elif branch is not None:
@@ -819,7 +819,7 @@ def norm_silu_linear(y: torch.Tensor, norm: torch.nn.LayerNorm, weight: torch.Te
     _linear_args(a, _DTYPES[dt], dev, y, rows, weight, bias, out, False)
     a.prologue = _lib.PRO_NORM_SILU
     a.ln_weight, a.ln_bias, a.ln_eps = _ln(norm)
-    if not lib().pk_linear_takes_norm(rows, n, k, 1):
+    if not lib().pk_linear_takes_norm(rows, n, k, 0):
         h = torch.empty((rows, k), dtype=dt, device=dev)
         a.residual_out, a.residual_out_stride = h.data_ptr(), k
     check(lib().pk_linear(ctypes.byref(a), 1, _stream(dev)), "pk_linear")
