@@ -557,6 +557,53 @@ typedef struct pk_sub_args {
 int pk_subsample(const pk_sub_args* args, void* stream);
 
 /* ---------------------------------------------------------------------------
+ * pk_fe_plan -- host only: one push of every stream of a batch through the frame
+ * counters (feature_extractor.py:97-151, model_runner.py:198-234), and the
+ * records pk_fe_step and pk_subsample read.
+ * In/out, per slot: total (samples pushed), emitted (frames), offset (samples
+ * trimmed), cached (pre-encode cache frames), has_cache, last_window [2] (first
+ * frame and rows of the last emitting push's window); noise_id per slot.
+ * In, per stream: slots (distinct, else PK_ERR_STATE), n_new, final_flag.
+ * Out, per stream: fe; start, n_frames, n_out, out_row; sub holds the sub_batch
+ * streams with kept outputs, in order.  Out: max_new, max_frames, max_out and
+ * out_rows (the sum of n_out).  PK_ERR_EXHAUSTED: a push past ring_size samples
+ * or mel_rows frames; a refused call changes no counter.
+ */
+typedef struct pk_fe_plan_args {
+  int32_t batch;
+  int32_t num_slots;
+  int32_t n_fft;
+  int32_t win_length;
+  int32_t hop;
+  int32_t cache_size;
+  int32_t drop;
+  int64_t ring_size;
+  int64_t mel_rows;
+  int64_t* total;
+  int64_t* emitted;
+  int64_t* offset;
+  int64_t* cached;
+  uint8_t* has_cache;
+  int64_t* last_window;
+  const uint32_t* noise_id;
+  const int64_t* slots;
+  const int64_t* n_new;
+  const uint8_t* final_flag;
+  pk_fe_stream* fe;
+  pk_sub_stream* sub;
+  int64_t* start;
+  int64_t* n_frames;
+  int64_t* n_out;
+  int64_t* out_row;
+  int64_t max_new;
+  int64_t max_frames;
+  int64_t max_out;
+  int64_t out_rows;
+  int32_t sub_batch;
+} pk_fe_plan_args;
+int pk_fe_plan(pk_fe_plan_args* args);
+
+/* ---------------------------------------------------------------------------
  * pk_rnnt_greedy_step -- one greedy RNNT decoding step for a batch of streams
  * whose predictor state (LSTM h and c of every layer, and the predictor's joint
  * projection) lives on the device in slots.  For each encoder frame t <

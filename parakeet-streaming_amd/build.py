@@ -71,7 +71,7 @@ def build(verbose: bool = False) -> Path:
         _run([HIPCC, *HIP_FLAGS, *inc, "-x", "hip", "-c", str(CSRC / name), "-o", str(obj)], verbose)
         objs.append(obj)
 
-    for name in ("page_pool.cpp", "pk_common.cpp"):
+    for name in ("page_pool.cpp", "frontend_plan.cpp", "pk_common.cpp"):
         obj = BUILD_DIR / (Path(name).stem + ".o")
         _run([CXX, *CXX_FLAGS, *inc, "-c", str(CSRC / name), "-o", str(obj)], verbose)
         objs.append(obj)

@@ -360,6 +360,20 @@ class RnntArgs(ctypes.Structure):
     ]
 
 
+class FePlanArgs(ctypes.Structure):
+    _fields_ = (
+        [(n, c_int32) for n in ("batch", "num_slots", "n_fft", "win_length", "hop", "cache_size", "drop")]
+        + [(n, c_int64) for n in ("ring_size", "mel_rows")]
+        + [
+            (n, c_void_p)
+            for n in ("total", "emitted", "offset", "cached", "has_cache", "last_window", "noise_id", "slots", "n_new",
+                      "final_flag", "fe", "sub", "start", "n_frames", "n_out", "out_row")
+        ]
+        + [(n, c_int64) for n in ("max_new", "max_frames", "max_out", "out_rows")]
+        + [("sub_batch", c_int32)]
+    )
+
+
 # name -> (restype, argtypes); exactly the functions include/parakeet_paged.h declares
 SIGNATURES = {
     "pk_kv_append": (c_int, [POINTER(KvAppendArgs), c_void_p]),
@@ -371,6 +385,7 @@ SIGNATURES = {
     "pk_linear_takes_norm": (c_int, [c_int32, c_int32, c_int32, c_int32]),
     "pk_linear": (c_int, [POINTER(LinearArgs), c_int32, c_void_p]),
     "pk_fe_step": (c_int, [POINTER(FeArgs), c_void_p]),
+    "pk_fe_plan": (c_int, [POINTER(FePlanArgs)]),
     "pk_subsample": (c_int, [POINTER(SubArgs), c_void_p]),
     "pk_rnnt_workspace_bytes": (c_int64, [c_int32, c_int32, c_int32, c_int32, c_int32]),
     "pk_rnnt_greedy_step": (c_int, [POINTER(RnntArgs), c_void_p]),

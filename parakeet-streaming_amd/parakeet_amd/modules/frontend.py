@@ -20,6 +20,7 @@ There is no CPU path: without the HIP library the calls raise.
 
 from __future__ import annotations
 
+import ctypes
 import math
 
 import numpy as np
@@ -28,6 +29,7 @@ from torch import Tensor, nn
 from torch.nn import functional as F
 
 from .. import ops
+from .._lib import PK_ERR_EXHAUSTED, PK_ERR_STATE, FePlanArgs, check, last_error, lib
 
 # 32-byte per-stream records read by the kernels (include/parakeet_paged.h)
 FE_STREAM = np.dtype(
@@ -89,6 +91,10 @@ class _Staging:
         if self.used[i]:
             self.events[i].synchronize()
         return i, self.bufs[i]
+
+    def last(self) -> torch.Tensor:
+        """The buffer taken last."""
+        return self.bufs[(self.i - 1) % len(self.bufs)]
 
     def upload(self, i: int, dst: Tensor, nbytes: int) -> None:
         dst[:nbytes].copy_(self.bufs[i][:nbytes], non_blocking=True)
@@ -255,7 +261,11 @@ class ConvSubsampling(nn.Module):
         self.out = nn.Linear(C * self.final_freq_dim, hidden_size, bias=True)
 
     def conv_weights(self) -> dict:
-        return {f"conv.{i}.{n}": getattr(self.conv[i], n) for i in (0, 2, 3, 5, 6) for n in ("weight", "bias")}
+        w = {}
+        for i, m in enumerate(self.conv):
+            if isinstance(m, nn.Conv2d):
+                w[f"conv.{i}.weight"], w[f"conv.{i}.bias"] = m.weight, m.bias
+        return w
 
     def stack(self, feats: Tensor, records: np.ndarray, ring: bool, out_rows: int, max_out: int) -> Tensor:
         """The convolution stack over ``records`` (SUB_STREAM) -> [out_rows, C*F3]."""
@@ -423,53 +433,73 @@ class PreEncoder:
         self._next_noise += 1
 
     # ------------------------------------------------------------ one step
+    def _plan(self, slots: np.ndarray, n_new: np.ndarray, final: np.ndarray, records: np.ndarray):
+        """One push of every stream through the counters (StreamCounters.plan) and
+        its records into ``records`` (the feature records, then the subsampling
+        ones), in one native call; returns the call's arguments and the per-stream
+        (start, n_frames, n_out, out_row)."""
+        B, c = len(slots), self.counters
+        for name, dt in (("total", np.int64), ("emitted", np.int64), ("offset", np.int64), ("cached", np.int64),
+                         ("has_cache", np.bool_), ("last_window", np.int64)):
+            v = getattr(c, name)
+            if v.dtype != dt or len(v) < self.num_slots or not v.flags.c_contiguous:
+                raise ValueError(f"counters.{name} must be contiguous {np.dtype(dt)} over {self.num_slots} slots")
+        noise = np.ascontiguousarray(self.noise_id, dtype=np.uint32)
+        if len(noise) < self.num_slots:
+            raise ValueError(f"noise_id must hold {self.num_slots} slots")
+        out = np.empty((4, B), dtype=np.int64)
+        a = FePlanArgs()
+        a.batch, a.num_slots = B, self.num_slots
+        a.n_fft, a.win_length, a.hop = c.n_fft, c.win, c.hop
+        a.cache_size, a.drop, a.ring_size, a.mel_rows = c.cache_size, c.drop, c.ring_size, c.mel_rows
+        a.total, a.emitted, a.offset = c.total.ctypes.data, c.emitted.ctypes.data, c.offset.ctypes.data
+        a.cached, a.has_cache, a.last_window = c.cached.ctypes.data, c.has_cache.ctypes.data, c.last_window.ctypes.data
+        a.noise_id, a.slots, a.n_new, a.final_flag = noise.ctypes.data, slots.ctypes.data, n_new.ctypes.data, final.ctypes.data
+        a.fe = records.ctypes.data
+        a.sub = a.fe + 32 * B
+        a.start = out.ctypes.data
+        a.n_frames, a.n_out, a.out_row = a.start + 8 * B, a.start + 16 * B, a.start + 24 * B
+        rc = lib().pk_fe_plan(ctypes.byref(a))
+        if rc == PK_ERR_STATE:
+            raise ValueError(last_error())
+        if rc == PK_ERR_EXHAUSTED:
+            raise RuntimeError(last_error())
+        check(rc, "pk_fe_plan")
+        return a, out
+
     def _features(self, slots, samples, n_new, final):
+        """The feature half of a step: the push's plan as StreamCounters.plan
+        returns it, the streams with kept outputs and their first rows."""
+        plan, (start, n_frames, n_out, out_row) = self._push(slots, samples, n_new, final)
+        rec = self._stage.last().numpy()
+        fe, sub = rec[: 32 * plan.batch].view(FE_STREAM), rec[32 * plan.batch : 32 * (plan.batch + plan.sub_batch)].view(SUB_STREAM)
+        emit = n_frames > 0
+        rows = np.where(emit, self.counters.last_window[fe["slot"], 1], 0)
+        sel = np.nonzero(n_out > 0)[0]
+        drop = np.zeros(plan.batch, dtype=np.int64)
+        drop[sel] = sub["drop"]
+        return (fe["sample_base"].copy(), start, n_frames, rows - n_frames, rows, drop, n_out, emit), sel, out_row
+
+    def _push(self, slots, samples, n_new, final):
         slots = np.ascontiguousarray(slots, dtype=np.int64)
         B = len(slots)
         if B > self.max_batch:
             raise ValueError(f"batch {B} exceeds max_batch {self.max_batch}")
-        if len(np.unique(slots)) != B or (B and (slots.min() < 0 or slots.max() >= self.num_slots)):
-            raise ValueError("slots must be distinct and in range")
-        n_new = np.broadcast_to(np.asarray(n_new, dtype=np.int64), (B,)).copy()
-        final = np.broadcast_to(np.asarray(final, dtype=bool), (B,)).copy()
-        plan = self.counters.plan(slots, n_new, final)
-        total0, start, n_frames, c, W, drop, n_out, emit = plan
+        n_new = np.array(np.broadcast_to(np.asarray(n_new, dtype=np.int64), (B,)))
+        final = np.array(np.broadcast_to(np.asarray(final, dtype=bool), (B,)))
         i, buf = self._stage.take()
-        fe_rec = buf[: 32 * B].numpy().view(FE_STREAM)
-        fe_rec["slot"] = slots
-        fe_rec["n_new"] = n_new
-        fe_rec["sample_base"] = total0
-        fe_rec["frame0"] = np.where(emit, start, 0)
-        fe_rec["n_frames"] = n_frames
-        fe_rec["noise_id"] = self.noise_id[slots]
-        fe_rec["reserved"] = 0
-        sel = np.nonzero(n_out > 0)[0]
-        sub_rec = buf[32 * B : 32 * (B + len(sel))].numpy().view(SUB_STREAM)
-        out_row = np.zeros(B, dtype=np.int64)
-        out_row[sel] = np.concatenate([[0], np.cumsum(n_out[sel])[:-1]]) if len(sel) else []
-        sub_rec["slot"] = slots[sel]
-        sub_rec["row0"] = (start - c)[sel]
-        sub_rec["rows"] = W[sel]
-        sub_rec["length"] = W[sel]
-        sub_rec["drop"] = drop[sel]
-        sub_rec["n_out"] = n_out[sel]
-        sub_rec["out_row"] = out_row[sel]
-        sub_rec["reserved"] = 0
-        nbytes = 32 * (B + len(sel))
-        self._stage.upload(i, self.hdr, nbytes)
-        max_new = int(n_new.max()) if B else 0
-        max_frames = int(n_frames.max()) if B else 0
-        if B and (max_new or max_frames):
+        plan, out = self._plan(slots, n_new, final, buf.numpy())
+        self._stage.upload(i, self.hdr, 32 * (B + plan.sub_batch))
+        if B and (plan.max_new or plan.max_frames):
             ops.fe_step(self.hdr[: 32 * B], B, samples, self.sample_ring, self.mel_ring, self.tables,
-                        dither=self.fe.dither, seed=self.fe.seed, max_new=max_new, max_frames=max_frames)
-        return plan, sel, out_row
+                        dither=self.fe.dither, seed=self.fe.seed, max_new=plan.max_new, max_frames=plan.max_frames)
+        return plan, out
 
     def push_features(self, slot: int, samples, final: bool = False):
         """FeatureExtractor.push for one slot: [1, n_mels, n] or None."""
         x = torch.as_tensor(np.asarray(samples, dtype=np.float32)).to(self.device).reshape(1, -1)
         n = int(x.shape[1])
-        plan, _, _ = self._features(np.array([slot]), x if n else None, n, final)
-        _, start, n_frames, *_ = plan
+        _, (start, n_frames, _, _) = self._push(np.array([slot]), x if n else None, n, final)
         if not n_frames[0]:
             return None
         rows = (int(start[0]) + torch.arange(int(n_frames[0]), device=self.device)) & (self.mel_rows - 1)
@@ -485,18 +515,16 @@ class PreEncoder:
         frames are rows[first[b] : first[b] + counts[b]]."""
         if self.sub is None:
             raise RuntimeError("this PreEncoder has no subsampling module")
-        plan, sel, out_row = self._features(slots, samples, n_new, final)
-        n_out = plan[6]
-        R = int(n_out.sum())
+        plan, (_, _, n_out, out_row) = self._push(slots, samples, n_new, final)
+        R = plan.out_rows
         C, F3 = self.sub._conv_channels, self.sub.final_freq_dim
         w = self.sub.out.weight
         if R == 0:
             return torch.empty((0, w.shape[0]), dtype=w.dtype, device=self.device), n_out, out_row
-        B = len(plan[0])
         flat = torch.empty((R, C * F3), dtype=w.dtype, device=self.device)
-        ops.subsample(self.hdr[32 * B :], len(sel), self.mel_ring, True, self.sub.conv_weights(), flat,
-                      max_out=int(n_out.max()))
-        return F.linear(flat, w, self.sub.out.bias), n_out, out_row
+        ops.subsample(self.hdr[32 * plan.batch :], plan.sub_batch, self.mel_ring, True, self.sub.conv_weights(), flat,
+                      max_out=plan.max_out)
+        return ops.functional_linear(flat, w, self.sub.out.bias), n_out, out_row
 
 
 __all__ = ["FeatureExtractor", "ConvSubsampling", "PreEncoder", "StreamCounters", "slaney_mel_filterbank", "stack_len"]

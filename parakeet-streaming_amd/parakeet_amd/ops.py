@@ -44,7 +44,9 @@ def _require_device(*tensors: torch.Tensor) -> torch.device:
 
 
 def _stream(dev: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    # torch.cuda.current_stream(dev).cuda_stream without the Stream object (0.3 us, 4 with it)
+    i = dev.index
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if i is None else i))
 
 
 def _event_handle(ev) -> int:

@@ -266,3 +266,15 @@ def test_linear_args_validated_before_launch():
     a.branch_stride = a.residual_out_stride = 512
     assert L.pk_linear(ctypes.byref(a), 1, None) == _lib.PK_ERR_INVALID  # residual_out is x
     assert "must not be x" in _lib.last_error()
+
+
+def test_front_end_plan_layout_and_null():
+    assert [f[0] for f in _lib.FePlanArgs._fields_] == _struct_fields("pk_fe_plan_args")
+    L = _lib.lib()
+    assert L.pk_fe_plan(None) == _lib.PK_ERR_INVALID
+    a = _lib.FePlanArgs()
+    a.batch, a.num_slots, a.n_fft, a.hop = 1, 1, 512, 160
+    assert L.pk_fe_plan(ctypes.byref(a)) == _lib.PK_ERR_INVALID  # NULL arrays
+    assert "NULL" in _lib.last_error()
+    a.batch = 0
+    assert L.pk_fe_plan(ctypes.byref(a)) == _lib.PK_OK

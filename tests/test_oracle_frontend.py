@@ -330,3 +330,66 @@ def test_stream_counters_reject_what_the_rings_cannot_hold():
     ctr = StreamCounters(2, 512, 400, 160, ring_size=8192, mel_rows=16)
     with pytest.raises(RuntimeError, match="mel ring"):
         ctr.plan(np.array([1]), np.array([4000]), np.array([False]))  # 24 frames in one window
+
+
+def test_native_plan_matches_stream_counters():
+    """pk_fe_plan against StreamCounters.plan over random pushes (empty, short,
+    final, subsets in any order, offsets from several trims): the same returns,
+    records and counters, and the same refusals with no counter changed."""
+    import types
+
+    from parakeet_amd.modules.frontend import FE_STREAM, SUB_STREAM, PreEncoder, StreamCounters
+
+    rng = np.random.default_rng(5)
+    for cache_size, drop, ring, rows in ((9, 2, 8192, 64), (0, 2, 8192, 64), (9, 0, 4096, 32)):
+        S = 9
+        a, b = (StreamCounters(S, 512, 400, 160, cache_size, drop, ring, rows) for _ in range(2))
+        pre = types.SimpleNamespace(counters=b, num_slots=S, noise_id=rng.integers(0, 2**32, S, dtype=np.uint32))
+        for step in range(400):
+            B = int(rng.integers(0, S + 1))
+            slots = rng.permutation(S)[:B].astype(np.int64)
+            n = rng.choice([0, 1, 100, 159, 160, 1440, 2560, 2561, 3999], B).astype(np.int64)
+            final = rng.random(B) < 0.1
+            if step % 50 == 49:
+                s = int(rng.integers(0, S))
+                a.reset(s)
+                b.reset(s)
+            total0 = a.total[slots].copy()
+            rec = np.zeros(64 * max(B, 1), dtype=np.uint8)
+            before = [getattr(b, k).copy() for k in ("total", "emitted", "offset", "cached", "has_cache", "last_window")]
+            try:
+                want = a.plan(slots, n, final)
+            except RuntimeError as e:
+                with pytest.raises(RuntimeError) as got:
+                    PreEncoder._plan(pre, slots, n, final, rec)
+                assert str(got.value) == str(e)
+                for k, v in zip(("total", "emitted", "offset", "cached", "has_cache", "last_window"), before):
+                    assert np.array_equal(getattr(b, k), v)
+                for s in slots:
+                    a.reset(int(s))
+                    b.reset(int(s))
+                continue
+            _, start, n_frames, c, W, dr, n_out, emit = want
+            args, out = PreEncoder._plan(pre, slots, n, final, rec)
+            assert np.array_equal(out[1], n_frames) and np.array_equal(out[2], n_out)
+            assert np.array_equal(out[0][emit], start[emit])
+            for k in ("total", "emitted", "offset", "cached", "has_cache", "last_window"):
+                assert np.array_equal(getattr(a, k), getattr(b, k)), k
+            fe = rec[: 32 * B].view(FE_STREAM)
+            for k, v in (("slot", slots), ("n_new", n), ("sample_base", total0), ("frame0", np.where(emit, start, 0)),
+                         ("n_frames", n_frames), ("noise_id", pre.noise_id[slots]), ("reserved", 0 * n)):
+                assert np.array_equal(fe[k], v), k
+            sel = np.nonzero(n_out > 0)[0]
+            assert args.sub_batch == len(sel) and args.out_rows == n_out.sum()
+            sub = rec[32 * B : 32 * (B + len(sel))].view(SUB_STREAM)
+            first = np.concatenate([[0], np.cumsum(n_out[sel])[:-1]]) if len(sel) else np.zeros(0, np.int64)
+            for k, v in (("slot", slots[sel]), ("row0", (start - c)[sel]), ("rows", W[sel]), ("length", W[sel]), ("drop", dr[sel]),
+                         ("n_out", n_out[sel]), ("out_row", first)):
+                assert np.array_equal(sub[k], v), k
+            assert np.array_equal(out[3][sel], first) and not out[3][n_out == 0].any()
+            if B:
+                assert (args.max_new, args.max_frames, args.max_out) == (n.max(), n_frames.max(), n_out.max())
+        for bad in ([0, 0], [-1], [S]):
+            z = np.array(bad, dtype=np.int64)
+            with pytest.raises(ValueError, match="distinct and in range"):
+                PreEncoder._plan(pre, z, 0 * z + 160, z < -9, np.zeros(128, dtype=np.uint8))
