@@ -186,9 +186,10 @@ class GreedyDecoder:
         if g is not None:
             return g
         dev = self.device
-        W = T * self.max_symbols + T  # per stream: tokens, then counts per frame
+        n_tok = B * T * self.max_symbols
         meta = torch.zeros(2 * B, dtype=torch.int32, device=dev)  # slots | lengths
-        out = torch.zeros((B, W), dtype=torch.int32, device=dev)
+        # one buffer, one copy back: [B, T * max_symbols] tokens, then [B, T] counts
+        out = torch.zeros(n_tok + B * T, dtype=torch.int32, device=dev)
         g = {
             "meta": meta,
             # two pinned upload and two pinned result buffers, used in turn: a call
@@ -204,27 +205,23 @@ class GreedyDecoder:
             "enc": torch.zeros((B, T, D), dtype=self.dtype, device=dev),
             "e": torch.empty((B, T, self.joint), dtype=self.dtype, device=dev),
             "out": out,
-            "out_h": [torch.zeros((B, W), dtype=torch.int32, pin_memory=True) for _ in range(2)],
-            "tokens": out[:, : T * self.max_symbols],
-            "counts": out[:, T * self.max_symbols :],
+            "out_h": [torch.zeros(out.shape, dtype=torch.int32, pin_memory=True) for _ in range(2)],
+            "tokens": out[:n_tok].view(B, T * self.max_symbols),
+            "counts": out[n_tok:].view(B, T),
         }
         a = self._args(g["slots"], prime=False)
         a.enc_proj, a.enc_stride_b, a.enc_stride_t = g["e"].data_ptr(), g["e"].stride(0), g["e"].stride(1)
         a.lengths, a.max_frames = g["lens"].data_ptr(), T
         a.tokens, a.frame_counts = g["tokens"].data_ptr(), g["counts"].data_ptr()
-        # rows of `out` hold T*max_symbols tokens then T counts: the kernels index
-        # tokens with row length T*max_symbols and counts with row length T, so
-        # they get their own buffers and the graph copies them into `out`
-        g["tok_buf"] = torch.empty((B, T * self.max_symbols), dtype=torch.int32, device=dev)
-        g["cnt_buf"] = torch.empty((B, T), dtype=torch.int32, device=dev)
-        a.tokens, a.frame_counts = g["tok_buf"].data_ptr(), g["cnt_buf"].data_ptr()
         g["args"] = a
+        native = ops.layer_applies(self.dtype, dev, B * T, self.w_enc, self.b_enc) and self.dtype != torch.float32
 
         def run():
-            torch.addmm(self.b_enc, g["enc"].view(B * T, D), self.w_enc.t(), out=g["e"].view(B * T, self.joint))
+            if native:
+                ops.linear(g["enc"].view(B * T, D), self.w_enc, self.b_enc, out=g["e"].view(B * T, self.joint))
+            else:
+                torch.addmm(self.b_enc, g["enc"].view(B * T, D), self.w_enc.t(), out=g["e"].view(B * T, self.joint))
             check(lib().pk_rnnt_greedy_step(ctypes.byref(a), ops._stream(dev)), "pk_rnnt_greedy_step")
-            g["tokens"].copy_(g["tok_buf"])
-            g["counts"].copy_(g["cnt_buf"])
 
         side = torch.cuda.Stream(dev)
         side.wait_stream(torch.cuda.current_stream(dev))
@@ -396,10 +393,10 @@ class PendingTokens:
     def result(self):
         if self._out is None:
             self._event.synchronize()
-            o = self._buf.numpy()
+            o, B = self._buf.numpy(), len(self._lens)
             # the buffer is reused two calls later: the lazy result keeps its own copy
-            self._out = GreedyDecoder._split(o[:, : self._n_tok].copy(), o[:, self._n_tok :], self._lens,
-                                             self._frame_tokens)
+            self._out = GreedyDecoder._split(o[: B * self._n_tok].reshape(B, self._n_tok).copy(),
+                                             o[B * self._n_tok :].reshape(B, -1), self._lens, self._frame_tokens)
             self._buf = None
         return self._out
 

@@ -624,12 +624,17 @@ def _aligned_rows(x: torch.Tensor) -> torch.Tensor:
     return x if x.data_ptr() % 16 == 0 else x.clone()
 
 
-def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None, *, silu: bool = False) -> torch.Tensor:
+def linear(
+    x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None, *, silu: bool = False, out: torch.Tensor | None = None
+) -> torch.Tensor:
     """``x @ weight.T + bias``, and SiLU of it, in one launch, for layers that
     :func:`linear_applies` accepts (feedforward.py:20-26, attention.py:92,122)."""
     x = _aligned_rows(x)
     n, k = weight.shape
-    out = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
+    if out is None:
+        out = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
+    elif tuple(out.shape) != (*x.shape[:-1], n) or out.dtype != x.dtype or out.device != x.device or not out.is_contiguous():
+        raise ValueError(f"out must be contiguous {(*x.shape[:-1], n)} of {x.dtype} on {x.device}")
     a = LinearArgs()
     _linear_args(a, _DTYPES[x.dtype], x.device, x, x.numel() // k, weight, bias, out, silu)
     check(lib().pk_linear(ctypes.byref(a), 1, _stream(x.device)), "pk_linear")
