@@ -643,6 +643,12 @@ int pk_fe_plan(pk_fe_plan_args* args);
  *              launches run over that list instead of every 16-stream tile that
  *              holds one such stream (one more small launch per iteration, which
  *              decides and builds the list).  Outputs are the same either way.
+ * packed     : 1 if w_ih, w_hh, w_pred and w_out hold their rows in matrix-core
+ *              operand order (16-bit types: k-steps of 32 columns, chunks of 8;
+ *              fp32: 16 and 4): [rows / 16][K / k-step][4][16][chunk], element
+ *              (t, s, g, r, e) = W[16 t + r][k-step s + chunk g + e]; w_out's rows
+ *              padded to a multiple of 64.  A load of 16 rows is then 1 KB in a
+ *              row.  0: the plain layouts above.  Outputs are the same.
  * workspace  : device bytes, at least pk_rnnt_workspace_bytes(...), 16-aligned.
  * One dtype for every floating tensor; fp32 accumulation.  hidden must be 640
  * (both reference models, config.py:19-21); joint a multiple of 64, <= 1024.
@@ -681,6 +687,7 @@ typedef struct pk_rnnt_args {
   int32_t* tokens;
   int32_t* frame_counts;
   void* workspace;
+  int32_t packed;
 } pk_rnnt_args;
 int64_t pk_rnnt_workspace_bytes(int32_t dtype, int32_t batch, int32_t vocab1, int32_t layers, int32_t hidden);
 int pk_rnnt_greedy_step(const pk_rnnt_args* args, void* stream);

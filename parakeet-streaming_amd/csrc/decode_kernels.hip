@@ -103,6 +103,7 @@ struct DecK {
   int32_t* acount;  // [2]
   int32_t compact;
   int32_t it;
+  int32_t packed;  // w_ih, w_hh, w_pred, w_out in operand order (pk_rnnt_args)
 };
 
 // stream state words in the workspace
@@ -136,21 +137,28 @@ struct KChunk {
 };
 
 // The wave's 16 weight rows (A, from global memory) against 16 columns held in
-// LDS (B), over nk k-steps of 4*VEC elements.  Rows are read from `wa` for
-// k-steps [0, ka) and from `wb` (at k-step - ka) after it; the LDS column runs
-// contiguously over all nk k-steps.  Weights move in chunks of CH k-steps whose
+// LDS (B), over nk k-steps of 4*VEC elements.  Weights move in chunks of CH k-steps whose
 // loads are all issued before the chunk's first MFMA (the index clamped, so
 // every load is valid): a wave waits for one L2 round trip per CH k-steps rather
 // than one per k-step.  The k-steps accumulate in order, as a plain loop would.
-template <typename ST, int CH>
-__device__ static inline void load_chunk(u32x4 (&w)[CH], const ST* wa, const ST* wb, int ka, int nk, int k0, int lg) {
+struct WRows {
+  const void* p;  // the lane's chunk of k-step 0
+  int step;       // elements from a k-step to the next
+};
+// The lane's view of 16 weight rows from row `row0` of [rows][K]: plain, its row's
+// chunks (an instruction touches 16 rows x 64 bytes, half of each 128-byte line);
+// packed, a k-step's 64 lanes are 1 KB in a row.
+template <typename ST>
+__device__ static inline WRows w_rows(const void* w, bool packed, int64_t row0, int64_t last, int K, int lr, int lg) {
   constexpr int VEC = 16 / sizeof(ST);
+  if (packed) return WRows{(const ST*)w + row0 * K + (lg * 16 + lr) * VEC, 64 * VEC};
+  const int64_t row = row0 + lr < last ? row0 + lr : last;
+  return WRows{(const ST*)w + row * K + VEC * lg, 4 * VEC};
+}
+template <typename ST, int CH>
+__device__ static inline void load_chunk(u32x4 (&w)[CH], const WRows& r, int nk, int k0) {
 #pragma unroll
-  for (int u = 0; u < CH; ++u) {
-    const int kk = min(k0 + u, nk - 1);
-    const ST* src = kk < ka ? wa + kk * 4 * VEC : wb + (kk - ka) * 4 * VEC;
-    w[u] = ld16(src + VEC * lg);
-  }
+  for (int u = 0; u < CH; ++u) w[u] = ld16((const ST*)r.p + min(k0 + u, nk - 1) * r.step);
 }
 
 template <typename ST, int CH>
@@ -162,31 +170,17 @@ __device__ static inline f32x4_t mma_chunk(const u32x4 (&w)[CH], const ST* col, 
   return d;
 }
 
-// d += the product, with the first chunk's weights already loaded into w0 (its
-// loads issued early, so their round trip overlaps the caller's other loads).
+// d += the product, with the first two chunks' weights already loaded into w0 and
+// w1 (issued early, so their round trip overlaps the caller's other loads).
 template <typename ST, int CH>
-__device__ static inline f32x4_t mma_rows(const u32x4 (&w0)[CH], const ST* wa, const ST* wb, int ka, int nk,
-                                          const ST* col, int lg, f32x4_t d) {
+__device__ static inline f32x4_t mma_rows2(const u32x4 (&w0)[CH], const u32x4 (&w1)[CH], const WRows& r, int nk, const ST* col,
+                                           int lg, f32x4_t d) {
   d = mma_chunk<ST>(w0, col, 0, nk, lg, d);
-  for (int k0 = CH; k0 < nk; k0 += CH) {
-    u32x4 w[CH];
-    load_chunk<ST>(w, wa, wb, ka, nk, k0, lg);
-    __builtin_amdgcn_sched_barrier(0);  // the chunk's loads all issue before its first MFMA
-    d = mma_chunk<ST>(w, col, k0, nk, lg, d);
-  }
-  return d;
-}
-
-// The same with the first two chunks already loaded (w1: k-steps CH .. 2 CH).
-template <typename ST, int CH>
-__device__ static inline f32x4_t mma_rows2(const u32x4 (&w0)[CH], const u32x4 (&w1)[CH], const ST* wa,
-                                           const ST* wb, int ka, int nk, const ST* col, int lg, f32x4_t d) {
-  d = mma_chunk<ST>(w0, col, 0, nk, lg, d);
-  d = mma_chunk<ST>(w1, col, CH, nk, lg, d);
+  if (CH < nk) d = mma_chunk<ST>(w1, col, CH, nk, lg, d);
   for (int k0 = 2 * CH; k0 < nk; k0 += CH) {
     u32x4 w[CH];
-    load_chunk<ST>(w, wa, wb, ka, nk, k0, lg);
-    __builtin_amdgcn_sched_barrier(0);
+    load_chunk<ST>(w, r, nk, k0);
+    __builtin_amdgcn_sched_barrier(0);  // the chunk's loads all issue before its first MFMA
     d = mma_chunk<ST>(w, col, k0, nk, lg, d);
   }
   return d;
@@ -247,9 +241,9 @@ __global__ void __launch_bounds__(kJointWaves * 64) joint_kernel(const DecK p) {
   // address valid for any entry, then masked), the second weight chunk behind
   const int J = p.J, nch = J / VEC, ks = J / (4 * VEC);
   const int r0 = vt * kVT + wave * 16;
-  const ST* wrow = (const ST*)p.w_out + (int64_t)min(r0 + lr, p.V1 - 1) * J;
+  const WRows wrow = w_rows<ST>(p.w_out, p.packed, r0, p.V1 - 1, J, lr, lg);
   u32x4 w0[KChunk<ST>::CH], w1[KChunk<ST>::CH];
-  load_chunk<ST>(w0, wrow, wrow, ks, ks, 0, lg);
+  load_chunk<ST>(w0, wrow, ks, 0);
   float bias[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) bias[i] = from_st(((const ST*)p.b_out)[min(r0 + 4 * lg + i, p.V1 - 1)]);
@@ -264,7 +258,7 @@ __global__ void __launch_bounds__(kJointWaves * 64) joint_kernel(const DecK p) {
       qr[j] = ld16(qr_src + cc);
     }
   }
-  load_chunk<ST>(w1, wrow, wrow, ks, ks, KChunk<ST>::CH, lg);
+  load_chunk<ST>(w1, wrow, ks, KChunk<ST>::CH);
   if (c == 0) bid_s[k] = b;
 #pragma unroll
   for (int j = 0; j < CPT; ++j) {
@@ -285,7 +279,7 @@ __global__ void __launch_bounds__(kJointWaves * 64) joint_kernel(const DecK p) {
   }
   __syncthreads();
   // logits of rows r0 .. r0 + 15 for the 16 streams
-  const f32x4_t d = mma_rows2<ST>(w0, w1, wrow, wrow, ks, ks, &hid[lr][0], lg, f32x4_t{0.f, 0.f, 0.f, 0.f});
+  const f32x4_t d = mma_rows2<ST>(w0, w1, wrow, ks, &hid[lr][0], lg, f32x4_t{0.f, 0.f, 0.f, 0.f});
   // lane holds rows 4*lg + i (of the wave's 16) for stream lr
   float best = -INFINITY;
   int bidx = 0x7fffffff;
@@ -587,11 +581,11 @@ __global__ void __launch_bounds__(512) lstm_kernel(const DecK p) {  // LstmCfg::
     }
   }
   // the wave's weight rows: gate gi, units u0 .. u0 + 15, first chunk
-  const int64_t row = (int64_t)layer * 4 * H + gi * H + u0 + lr;
+  const int64_t row = (int64_t)layer * 4 * H + gi * H + u0;
   constexpr int ks = H / (4 * VEC);
-  const ST* wrow = (const ST*)(part ? p.w_hh : p.w_ih) + row * H;
+  const WRows wrow = w_rows<ST>(part ? p.w_hh : p.w_ih, p.packed, row, row + 15, H, lr, lg);
   u32x4 w0[CH];
-  load_chunk<ST>(w0, wrow, wrow, ks, ks, 0, lg);
+  load_chunk<ST>(w0, wrow, ks, 0);
   __builtin_amdgcn_sched_barrier(0);
   u32x4 v[NE][CPT];
   u32x4 w1[CH];   // the second weight chunk
@@ -605,7 +599,7 @@ __global__ void __launch_bounds__(512) lstm_kernel(const DecK p) {  // LstmCfg::
     // the second weight chunk, then x: the embedding row of the token (layer 0)
     // or the layer below's new h; loads from addresses valid for any entry,
     // then masked
-    load_chunk<ST>(w1, wrow, wrow, ks, ks, CH, lg);
+    load_chunk<ST>(w1, wrow, ks, CH);
 #pragma unroll
     for (int e = 0; e < NE; ++e) {
       const ST* src = layer == 0 ? (const ST*)p.embed + (int64_t)max(tk[e], 0) * H
@@ -654,12 +648,12 @@ __global__ void __launch_bounds__(512) lstm_kernel(const DecK p) {  // LstmCfg::
   // gate gi rows for the streams, 16 a column tile: the input part's k-steps,
   // then the recurrent part's from those sums (its second chunk loading
   // meanwhile); lane: units u0 + 4 lg + i, stream 16 ct + lr
-  if (part == 1) load_chunk<ST>(w1, wrow, wrow, ks, ks, CH, lg);
+  if (part == 1) load_chunk<ST>(w1, wrow, ks, CH);
   if (part == 0) {
 #pragma unroll
     for (int ct = 0; ct < NE; ++ct) {
       const f32x4_t d =
-          mma_rows2<ST>(w0, w1, wrow, wrow, ks, ks, &xs[16 * ct + lr][0], lg, f32x4_t{0.f, 0.f, 0.f, 0.f});
+          mma_rows2<ST>(w0, w1, wrow, ks, &xs[16 * ct + lr][0], lg, f32x4_t{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
       for (int i = 0; i < 4; ++i) gsm[gi][16 * ct + lr][4 * lg + i] = d[i];
     }
@@ -671,7 +665,7 @@ __global__ void __launch_bounds__(512) lstm_kernel(const DecK p) {  // LstmCfg::
       f32x4_t d;
 #pragma unroll
       for (int i = 0; i < 4; ++i) d[i] = gsm[gi][16 * ct + lr][4 * lg + i];
-      d = mma_rows2<ST>(w0, w1, wrow, wrow, ks, ks, &hs[16 * ct + lr][0], lg, d);
+      d = mma_rows2<ST>(w0, w1, wrow, ks, &hs[16 * ct + lr][0], lg, d);
 #pragma unroll
       for (int i = 0; i < 4; ++i) gsm[gi][16 * ct + lr][4 * lg + i] = d[i];
     }
@@ -737,9 +731,9 @@ __global__ void __launch_bounds__(kPredWaves * 64) pred_kernel(const DecK p) {
   constexpr int ks = H / (4 * VEC);
   const int jw = j0 + wave * 16;
   const bool wave_live = jw < J;  // uniform per wave
-  const ST* wrow = (const ST*)p.w_pred + (int64_t)min(jw + lr, J - 1) * H;
+  const WRows wrow = w_rows<ST>(p.w_pred, p.packed, min(jw, J - 16), J - 1, H, lr, lg);
   u32x4 w0[KChunk<ST>::CH], w1[KChunk<ST>::CH];
-  load_chunk<ST>(w0, wrow, wrow, ks, ks, 0, lg);
+  load_chunk<ST>(w0, wrow, ks, 0);
   float bias[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) bias[i] = from_st(((const ST*)p.b_pred)[min(jw + 4 * lg + i, J - 1)]);
@@ -754,7 +748,7 @@ __global__ void __launch_bounds__(kPredWaves * 64) pred_kernel(const DecK p) {
   const int nq = L * NCH, qs = gridDim.x * TPS;
   const ST* hn_b = (const ST*)p.hn + (int64_t)max(b, 0) * L * H;
   ST* h_s = (ST*)p.h + (int64_t)slot * L * H;
-  load_chunk<ST>(w1, wrow, wrow, ks, ks, KChunk<ST>::CH, lg);
+  load_chunk<ST>(w1, wrow, ks, KChunk<ST>::CH);
   if (c == 0) {
     tok_s[k] = tk;
     slot_s[k] = slot;
@@ -768,7 +762,7 @@ __global__ void __launch_bounds__(kPredWaves * 64) pred_kernel(const DecK p) {
   }
   __syncthreads();
   if (!wave_live) return;  // uniform per wave; no barrier below
-  const f32x4_t d = mma_rows2<ST>(w0, w1, wrow, wrow, ks, ks, &hs[lr][0], lg, f32x4_t{0.f, 0.f, 0.f, 0.f});
+  const f32x4_t d = mma_rows2<ST>(w0, w1, wrow, ks, &hs[lr][0], lg, f32x4_t{0.f, 0.f, 0.f, 0.f});
   // lane: outputs jw + 4 lg + i for stream lr
   if (tok_s[lr] >= 0) {
 #pragma unroll
@@ -826,6 +820,7 @@ static int run_step(const pk_rnnt_args* a, hipStream_t st) {
   k.compact = !a->prime && (a->compact > 0 || (a->compact == 0 && a->batch >= kCompactMinBatch));
   k.h = a->h;
   k.prime = a->prime;
+  k.packed = a->packed;
   const dim3 gj(k.vtiles, (a->batch + 15) / 16);
   // 32 streams a LSTM workgroup (16-bit types only: the fp32 rows of 32 streams
   // do not fit in LDS) in compact mode, where the tiles hold only streams that

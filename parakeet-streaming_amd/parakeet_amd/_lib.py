@@ -357,6 +357,7 @@ class RnntArgs(ctypes.Structure):
         ("tokens", c_void_p),
         ("frame_counts", c_void_p),
         ("workspace", c_void_p),
+        ("packed", c_int32),
     ]
 
 

@@ -95,6 +95,15 @@ class GreedyDecoder:
         self._ws: dict[int, torch.Tensor] = {}
         self._graphs: dict[tuple[int, int, int], dict] = {}
 
+    @staticmethod
+    def _packed(w: Tensor) -> Tensor:
+        """[..., rows, K] weight rows in the kernels' operand order
+        (pk_rnnt_args.packed), rows padded with zeros to a multiple of 64."""
+        w = w.reshape(-1, w.shape[-1])
+        vec = 16 // w.element_size()
+        w = F.pad(w, (0, 0, 0, -w.shape[0] % 64))
+        return w.view(w.shape[0] // 16, 16, w.shape[1] // (4 * vec), 4, vec).permute(0, 2, 3, 1, 4).contiguous()
+
     _WEIGHTS = ("w_ih", "w_hh", "b_ih", "b_hh", "embed", "w_pred", "b_pred", "w_enc", "b_enc", "w_out", "b_out")
 
     def refresh_weights(self) -> None:
@@ -118,13 +127,16 @@ class GreedyDecoder:
                 "w_enc": own(j.enc.weight), "b_enc": own(j.enc.bias),
                 "w_out": own(out.weight), "b_out": own(out.bias),
             }
+            for k in ("w_ih", "w_hh", "w_pred", "w_out"):  # what the kernels read
+                if new[k].shape[-1] % 64 == 0:  # every size they are built for
+                    new[k + "_packed"] = self._packed(new[k])
         if new["w_ih"].shape[2] != self.hidden:
             raise NotImplementedError("the predictor's embedding size must equal its hidden size (config.py:19)")
         for t in new.values():
             if t.dtype != self.dtype or t.device != self.device:
                 raise ValueError("predictor and joiner parameters must share one dtype and device")
         cur = getattr(self, "w_ih", None)
-        same = cur is not None and all(getattr(self, k).shape == v.shape for k, v in new.items())
+        same = cur is not None and all(hasattr(self, k) and getattr(self, k).shape == v.shape for k, v in new.items())
         if same:
             with torch.no_grad():
                 for k, v in new.items():
@@ -151,10 +163,13 @@ class GreedyDecoder:
         a.layers, a.hidden, a.joint, a.vocab1 = self.layers, self.hidden, self.joint, self.vocab1
         a.blank, a.max_symbols, a.prime = self.blank, self.max_symbols, int(prime)
         a.compact = int(self.compact)
-        a.embed, a.w_ih, a.w_hh = self.embed.data_ptr(), self.w_ih.data_ptr(), self.w_hh.data_ptr()
+        packed = all(hasattr(self, k + "_packed") for k in ("w_ih", "w_hh", "w_pred", "w_out"))
+        w_ih, w_hh, w_pred, w_out = (getattr(self, k + "_packed" if packed else k) for k in ("w_ih", "w_hh", "w_pred", "w_out"))
+        a.packed = int(packed)
+        a.embed, a.w_ih, a.w_hh = self.embed.data_ptr(), w_ih.data_ptr(), w_hh.data_ptr()
         a.b_ih, a.b_hh = self.b_ih.data_ptr(), self.b_hh.data_ptr()
-        a.w_pred, a.b_pred = self.w_pred.data_ptr(), self.b_pred.data_ptr()
-        a.w_out, a.b_out = self.w_out.data_ptr(), self.b_out.data_ptr()
+        a.w_pred, a.b_pred = w_pred.data_ptr(), self.b_pred.data_ptr()
+        a.w_out, a.b_out = w_out.data_ptr(), self.b_out.data_ptr()
         a.h, a.c, a.pred_proj = self.h.data_ptr(), self.c.data_ptr(), self.pred_proj.data_ptr()
         a.workspace = self._workspace(a.batch).data_ptr()
         return a

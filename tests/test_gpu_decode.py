@@ -307,3 +307,39 @@ def test_pending_results_match_blocking_calls(cuda):
         assert torch.equal(a.h, b.h) and torch.equal(a.c, b.c) and torch.equal(a.pred_proj, b.pred_proj)
     assert [p.result() for p in pending] == want  # the rest at the end (0, 1 built when their buffer came round)
     assert sum(len(t) for w in want for s_ in w for t in s_) > 5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layers,vocab,streams", [(1, 130, 33), (2, 70, 5), (1, 127, 140), (1, 90, 600)])
+def test_packed_weights_and_listed_tiles_give_the_plain_ones(cuda, dtype, layers, vocab, streams):
+    """Weights in operand order against the plain layouts, and the LSTM's list of
+    updating streams (up to 512 streams) against tiles by batch position (compact
+    mode's forms, which the decoder's own tests check): the same tokens and state
+    bits; a vocabulary that fills no whole tile, streams past one list round."""
+    from parakeet_amd.modules.decoder import GreedyDecoder, Joiner, Predictor
+
+    torch.manual_seed(layers * 100 + vocab)
+    with torch.device(cuda):
+        pred, joint = Predictor(640, 640, layers, vocab), Joiner(512, 640, 640, num_classes=vocab)
+    joint.joint_net[-1].weight.data.mul_(4.0)
+    joint.joint_net[-1].bias.data[vocab] += 1.0
+    pred, joint = pred.to(dtype).eval().requires_grad_(False), joint.to(dtype).eval().requires_grad_(False)
+    x = torch.randn(3, streams, 2, 512, device=cuda).to(dtype)
+    slots = np.random.default_rng(0).permutation(streams)
+    results = []
+    for mode in ("packed", "plain", "compact"):
+        dec = GreedyDecoder(pred, joint, blank_id=vocab, num_slots=streams)
+        if mode == "plain":
+            for k in ("w_ih", "w_hh", "w_pred", "w_out"):
+                delattr(dec, k + "_packed")
+        if mode == "compact":
+            dec.compact = 1
+        dec.reset_slot(slots)
+        toks = [[list(t) for t in dec.decode(slots, x[i], lengths=None if i else [1 + (b % 2) for b in range(streams)])] for i in range(3)]
+        results.append((toks, dec.h.clone(), dec.c.clone(), dec.pred_proj.clone()))
+    assert sum(len(t) for step in results[0][0] for t in step) > 0
+    for other in results[1:]:
+        assert other[0] == results[0][0]
+        for a, b in zip(results[0][1:], other[1:]):
+            assert torch.equal(a, b)
