@@ -114,7 +114,10 @@ constexpr int kBand = 32;  // filterbank weights per band staged in LDS
 // twiddles, window and filterbank then serves 16 frames), which stages the
 // samples of 16 frames and so takes hops up to kFeHopWide
 constexpr int kFeHopWide = 192;
-constexpr int kFeWideRounds = 8;  // workgroups a CU from which the 4-frames-a-wave form is used
+// the 4-frames-a-wave form is used from 3 such workgroups per 2 CUs: at 80 mels 256
+// streams (1 a CU) take 16.3 us with one frame a wave and 19.5 with four, 512
+// streams (2 a CU) 26.2 and 22.9; 60 streams x 112 frames (1.64 a CU) 24.4 and 22.3
+constexpr int kFeWideTwice = 3;
 template <int FPW>
 struct FeGeom {
   static constexpr int HOP = FPW == 1 ? kMaxHop : kFeHopWide;
@@ -191,6 +194,13 @@ __global__ void __launch_bounds__(64 * kFeWaves) fe_kernel(const FeK p) {
   const int64_t g0 = span0 >> 2;  // floor, span0 may be negative
 #pragma unroll
   for (int u = 0; u < kXsPer; ++u) {
+    // the span is the frames' reach, usually well under the staging's size: a
+    // round of groups past it loads nothing (uniform)
+    if (4 * u * 64 * kFeWaves >= span + 4) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) xr[u][e] = 0.f;
+      continue;
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int64_t g = 4 * (g0 + tid + u * 64 * kFeWaves) + e;
@@ -213,7 +223,6 @@ __global__ void __launch_bounds__(64 * kFeWaves) fe_kernel(const FeK p) {
   for (int u = 0; u < kXsPer; ++u) {
     const int64_t j = g0 + tid + u * 64 * kFeWaves;
     const int64_t i0 = 4 * j - span0;  // xs index of the group's first sample
-    // the span is the frames' reach, usually well under the staging's size
     if (i0 + 3 >= 0 && i0 < span) {
       float z[4] = {0.f, 0.f, 0.f, 0.f};
       if (p.dither != 0.f && 4 * j + 3 >= 0 && 4 * j < total) dither_normal4(j, s.noise_id, p.seed_lo, p.seed_hi, z);
@@ -233,14 +242,17 @@ __global__ void __launch_bounds__(64 * kFeWaves) fe_kernel(const FeK p) {
     const int m = i / kBand, k = rng_s[m].x + i % kBand;
     fr[u] = (m < p.n_mels && k < rng_s[m].y) ? p.fb[(int64_t)m * kBins + k] : 0.f;
   }
+  // tw[m] is tw2[2 m] for the first half circle and its negative for the second:
+  // one sincospif a thread instead of two (with the skipped rounds above 10.6 ->
+  // 9.6 us at 128 streams x 16 frames, 26.0 -> 24.4 at 60 x 112)
   for (int m = tid; m < kBins; m += blockDim.x) {
     float sn, cs;
-    if (m < kCplx) {
-      sincospif((float)m / 128.0f, &sn, &cs);
-      tw[m] = make_float2(cs, -sn);
-    }
     sincospif((float)m / 256.0f, &sn, &cs);
     tw2[m] = make_float2(cs, -sn);
+    if (m < kCplx && (m & 1) == 0) {
+      tw[m >> 1] = make_float2(cs, -sn);
+      tw[(m >> 1) + kCplx / 2] = make_float2(-cs, sn);
+    }
   }
 #pragma unroll
   for (int u = 0; u < kFbPer; ++u) {
@@ -1499,7 +1511,7 @@ extern "C" int pk_fe_step(const pk_fe_args* a, void* stream) {
   // such workgroups (and the hop fits their sample staging), one otherwise
   const int wide_frames = 4 * kFeWaves;
   const int64_t gx4 = a->max_frames > 0 ? (a->max_frames + wide_frames - 1) / wide_frames : 1;
-  const bool wide = a->hop <= kFeHopWide && gx4 * a->batch >= (int64_t)kFeWideRounds * cu_count();
+  const bool wide = a->hop <= kFeHopWide && 2 * gx4 * a->batch >= (int64_t)kFeWideTwice * cu_count();
   const int gx = a->max_frames > 0 ? (a->max_frames + (wide ? wide_frames : kFeWaves) - 1) / (wide ? wide_frames : kFeWaves) : 1;
   // the streams in launches of at most kMaxGridYZ (the grid's y extent)
   const size_t pcm_bytes = a->pcm_dtype == PK_PCM_S16 ? 2 : 4;
