@@ -209,6 +209,11 @@ typedef struct pk_attn_args {
   int64_t pos_stride_b; /* elements between streams' position tables; 0: one table for all */
 } pk_attn_args;
 int pk_paged_relpos_attn(const pk_attn_args* args, void* stream);
+/* pk_paged_relpos_attn for `count` layers whose calls are independent of each
+ * other (none reads or appends what another writes; different layers of a pool),
+ * in one launch where they differ in their tensors and layer alone and no call
+ * asks for events, else one by one.  One dtype and device.  The same outputs. */
+int pk_paged_relpos_attn_layers(const pk_attn_args* args, int32_t count, void* stream);
 
 /* ---------------------------------------------------------------------------
  * pk_streaming_mask -- device-side construction of the streaming attention and

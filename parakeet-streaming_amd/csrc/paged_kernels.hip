@@ -15,7 +15,9 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
 
+#include <algorithm>
 #include <cstdint>
+#include <cstring>
 #include <type_traits>
 
 #include "pk_common.h"
@@ -92,6 +94,47 @@ struct AttnK {
   const int32_t* nact;  // streams 0..*nact-1 are live (nullptr: all B)
   float scale;          // log2(e) / sqrt(head_dim)
 };
+
+// A launch over several layers' independent calls (grid z): what differs between
+// them, in the kernel's arguments.
+constexpr int kMaxLaunchLayers = 32;
+template <typename ST>
+struct AttnLayer {
+  const ST *q, *kn, *vn, *bu, *bv;
+  ST *kp, *vp, *out;
+};
+template <typename ST>
+struct AttnLayersK {
+  AttnK<ST> k;
+  AttnLayer<ST> l[kMaxLaunchLayers];
+};
+template <typename ST>
+__device__ static inline const AttnK<ST>& layer_args(const AttnK<ST>& k) {
+  return k;
+}
+template <typename ST>
+__device__ static inline AttnK<ST> layer_args(const AttnLayersK<ST>& a) {
+  AttnK<ST> k = a.k;
+  const AttnLayer<ST>& l = a.l[blockIdx.z];
+  k.q = l.q;
+  k.kn = l.kn;
+  k.vn = l.vn;
+  k.bu = l.bu;
+  k.bv = l.bv;
+  k.kp = l.kp;
+  k.vp = l.vp;
+  k.out = l.out;
+  return k;
+}
+// the two-query kernel's query pair: grid z (several layers: the only pair)
+template <typename ST>
+__device__ static inline int query_pair(const AttnK<ST>&) {
+  return blockIdx.z;
+}
+template <typename ST>
+__device__ static inline int query_pair(const AttnLayersK<ST>&) {
+  return 0;
+}
 
 // Streaming-mask state of one stream (encoder.py:186-212), 32-bit.  The key and
 // query chunk indices are floor((key_start + x) / C) = ks_q + (ks_r + x) / C with
@@ -577,8 +620,9 @@ __device__ static inline __amdgpu_buffer_rsrc_t rows_rsrc(const void* base, int 
 // Pages hold 64-byte column blocks ([page][block][page_size][32 elements]),
 // so one k-step load of a 16-slot tile reads 16 rows x 64 bytes of one block:
 // 1 KB of contiguous memory when the 16 slots share a page.
-template <typename ST, int DK, int NT, int MODE, bool MULTI, bool STREAM, int NW>
-__global__ void __launch_bounds__(64 * NW) relpos_attn_mfma_kernel(const AttnK<ST> p) {
+template <typename ST, int DK, int NT, int MODE, bool MULTI, bool STREAM, int NW, typename P>
+__global__ void __launch_bounds__(64 * NW) relpos_attn_mfma_kernel(const P arg) {
+  const AttnK<ST> p = layer_args(arg);
   constexpr int SPLIT = DK / 64;
   static_assert(NW == 4 || NW == 2, "waves a workgroup");
   constexpr int SPW = NW / SPLIT;  // streams per workgroup
@@ -634,7 +678,7 @@ __global__ void __launch_bounds__(64 * NW) relpos_attn_mfma_kernel(const AttnK<S
   const int w0 = sw * SPLIT;    // first wave of this stream
   const int sb = blockIdx.x;  // stream block
   const int h = blockIdx.y;
-  const int i0 = blockIdx.z * TQ;
+  const int i0 = query_pair(arg) * TQ;
   const int nq = min(TQ, p.T - i0);
   const int b_raw = sb * SPW + sw;
   const int b = min(b_raw, p.B - 1);  // loads stay inside the batch arrays
@@ -845,7 +889,7 @@ __global__ void __launch_bounds__(64 * NW) relpos_attn_mfma_kernel(const AttnK<S
     l_run[ii] = 0.f;
   }
   uint8_t* vl = v_lds[wave];
-  const bool do_append = p.append && blockIdx.z == 0 && active && paged;
+  const bool do_append = p.append && i0 == 0 && active && paged;
 
   // MULTI: windows longer than one pass (the single-pass form is straight-line
   // code, with nothing carried around a loop)
@@ -1193,8 +1237,9 @@ __device__ static inline float row_bcast(float v) {
 //   * the fused append stores the frame rows into their pages (K after the K
 //     products, V after P.V).
 // 4 waves a SIMD: at most 128 registers a lane and 40 KB of LDS a workgroup.
-template <typename ST, int DK, int MODE, bool STREAM>
-__global__ void __launch_bounds__(256, 4) relpos_attn_chunk_kernel(const AttnK<ST> p) {
+template <typename ST, int DK, int MODE, bool STREAM, typename P>
+__global__ void __launch_bounds__(256, 4) relpos_attn_chunk_kernel(const P arg) {
+  const AttnK<ST> p = layer_args(arg);
   constexpr int NW = 4;
   constexpr int NTH = 64 * NW;
   constexpr int KS = DK / 32;       // 16x16x32 k-steps over the head
@@ -1892,17 +1937,35 @@ void pick_tiling(int Lk, int rlw, int hint, int waves, int* NR, int* tiles) {
 // rows.
 constexpr int kMfmaTiles = 5;
 
+// several layers' calls in one launch (state mask only): count of them, their pointers
+template <typename ST>
+struct LayerSet {
+  int n = 1;
+  AttnLayer<ST> l[kMaxLaunchLayers];
+};
+
 template <typename ST, int DK, int MODE, bool MULTI, bool STREAM, int NW>
-int launch_attn_mfma_t(const pk_attn_args* a, const AttnK<ST>& k, hipStream_t s) {
+int launch_attn_mfma_t(const pk_attn_args* a, const AttnK<ST>& k, const LayerSet<ST>* ls, hipStream_t s) {
   constexpr int SPW = NW / (DK / 64);  // streams per workgroup
+  if constexpr (MODE == 2) {
+    if (ls) {
+      AttnLayersK<ST> kl;
+      kl.k = k;
+      std::copy(ls->l, ls->l + ls->n, kl.l);
+      const dim3 grid((unsigned)((a->batch + SPW - 1) / SPW), (unsigned)a->num_heads, (unsigned)ls->n);
+      hipLaunchKernelGGL((relpos_attn_mfma_kernel<ST, DK, kMfmaTiles, MODE, MULTI, STREAM, NW, AttnLayersK<ST>>), grid,
+                         dim3(64u * NW), 0, s, kl);
+      return check_launch("pk_paged_relpos_attn_layers");
+    }
+  }
   dim3 grid((unsigned)((a->batch + SPW - 1) / SPW), (unsigned)a->num_heads,
             (unsigned)((a->chunk + 1) / 2));
   dim3 block(64u * NW);
   if (a->start_event || a->stop_event) {
-    hipExtLaunchKernelGGL(relpos_attn_mfma_kernel<ST, DK, kMfmaTiles, MODE, MULTI, STREAM, NW>, grid, block,
+    hipExtLaunchKernelGGL((relpos_attn_mfma_kernel<ST, DK, kMfmaTiles, MODE, MULTI, STREAM, NW, AttnK<ST>>), grid, block,
                           0u, s, (hipEvent_t)a->start_event, (hipEvent_t)a->stop_event, 0u, k);
   } else {
-    hipLaunchKernelGGL((relpos_attn_mfma_kernel<ST, DK, kMfmaTiles, MODE, MULTI, STREAM, NW>), grid, block, 0,
+    hipLaunchKernelGGL((relpos_attn_mfma_kernel<ST, DK, kMfmaTiles, MODE, MULTI, STREAM, NW, AttnK<ST>>), grid, block, 0,
                        s, k);
   }
   return check_launch("pk_paged_relpos_attn");
@@ -1914,13 +1977,13 @@ int launch_attn_mfma_t(const pk_attn_args* a, const AttnK<ST>& k, hipStream_t s)
 // with a CU's worth or more they are slower (230 streams of the large model:
 // 13.6-14.1 -> 14.7-15.0 us), and small grids never take the streaming policy
 template <typename ST, int DK, int MODE, bool MULTI, bool STREAM>
-int launch_attn_mfma_nw(const pk_attn_args* a, const AttnK<ST>& k, hipStream_t s) {
+int launch_attn_mfma_nw(const pk_attn_args* a, const AttnK<ST>& k, const LayerSet<ST>* ls, hipStream_t s) {
   if constexpr (!STREAM) {
     const int64_t wgs4 = (int64_t)((a->batch + 4 / (DK / 64) - 1) / (4 / (DK / 64))) * a->num_heads *
-                         ((a->chunk + 1) / 2);
-    if (wgs4 < cu_count()) return launch_attn_mfma_t<ST, DK, MODE, MULTI, STREAM, 2>(a, k, s);
+                         ((a->chunk + 1) / 2) * (ls ? ls->n : 1);
+    if (wgs4 < cu_count()) return launch_attn_mfma_t<ST, DK, MODE, MULTI, STREAM, 2>(a, k, ls, s);
   }
-  return launch_attn_mfma_t<ST, DK, MODE, MULTI, STREAM, 4>(a, k, s);
+  return launch_attn_mfma_t<ST, DK, MODE, MULTI, STREAM, 4>(a, k, ls, s);
 }
 
 // Page rows are read with the streaming cache policy once a step's windows
@@ -1933,29 +1996,29 @@ int launch_attn_mfma_nw(const pk_attn_args* a, const AttnK<ST>& k, hipStream_t s
 constexpr int64_t kStreamingBytes = 192ll << 20;
 
 template <typename ST, int DK, int MODE, bool STREAM>
-int launch_attn_mfma_ms(const pk_attn_args* a, const AttnK<ST>& k, hipStream_t s) {
+int launch_attn_mfma_ms(const pk_attn_args* a, const AttnK<ST>& k, const LayerSet<ST>* ls, hipStream_t s) {
   // the single-pass form holds at most 16 * kMfmaTiles - 1 keys (its staged
   // position rows stop at 16 * kMfmaTiles)
-  if (k.tiles > 1 || k.Lk > 16 * kMfmaTiles - 1) return launch_attn_mfma_nw<ST, DK, MODE, true, STREAM>(a, k, s);
-  return launch_attn_mfma_nw<ST, DK, MODE, false, STREAM>(a, k, s);
+  if (k.tiles > 1 || k.Lk > 16 * kMfmaTiles - 1) return launch_attn_mfma_nw<ST, DK, MODE, true, STREAM>(a, k, ls, s);
+  return launch_attn_mfma_nw<ST, DK, MODE, false, STREAM>(a, k, ls, s);
 }
 
 template <typename ST, int DK, int MODE>
-int launch_attn_mfma_mode(const pk_attn_args* a, const AttnK<ST>& k, hipStream_t s) {
+int launch_attn_mfma_mode(const pk_attn_args* a, const AttnK<ST>& k, const LayerSet<ST>* ls, hipStream_t s) {
   const int64_t layers = a->pages.num_layers > 1 ? a->pages.num_layers : 1;
   const int64_t window_bytes = (int64_t)a->batch * k.Lk * a->num_heads * DK * (int64_t)sizeof(ST) * 2 * layers;
   const bool stream = k.pg.rows != nullptr && window_bytes > kStreamingBytes;
-  if (stream) return launch_attn_mfma_ms<ST, DK, MODE, true>(a, k, s);
-  return launch_attn_mfma_ms<ST, DK, MODE, false>(a, k, s);
+  if (stream) return launch_attn_mfma_ms<ST, DK, MODE, true>(a, k, ls, s);
+  return launch_attn_mfma_ms<ST, DK, MODE, false>(a, k, ls, s);
 }
 
 template <typename ST, int DK>
-int launch_attn_mfma(const pk_attn_args* a, AttnK<ST>& k, hipStream_t s) {
+int launch_attn_mfma(const pk_attn_args* a, AttnK<ST>& k, const LayerSet<ST>* ls, hipStream_t s) {
   constexpr int KT = 16 * kMfmaTiles;  // window columns per pass
   k.tiles = (k.Lk + KT - 1) / KT;
-  if (k.mask) return launch_attn_mfma_mode<ST, DK, 1>(a, k, s);
-  if (k.st_proc) return launch_attn_mfma_mode<ST, DK, 2>(a, k, s);
-  return launch_attn_mfma_mode<ST, DK, 0>(a, k, s);
+  if (k.mask) return launch_attn_mfma_mode<ST, DK, 1>(a, k, ls, s);
+  if (k.st_proc) return launch_attn_mfma_mode<ST, DK, 2>(a, k, ls, s);
+  return launch_attn_mfma_mode<ST, DK, 0>(a, k, ls, s);
 }
 
 // Whole-chunk matrix-core path: workgroups of 2 streams x one head, the
@@ -1964,36 +2027,47 @@ constexpr int kChunkMaxT = 14;      // query operand rows 0..13 (14: u, 15: v)
 constexpr int kChunkMaxWindow = 96;  // 2 waves x 3 tiles of 16 window columns
 
 template <typename ST, int DK, int MODE, bool STREAM>
-int launch_attn_chunk_t(const pk_attn_args* a, const AttnK<ST>& k, hipStream_t s) {
+int launch_attn_chunk_t(const pk_attn_args* a, const AttnK<ST>& k, const LayerSet<ST>* ls, hipStream_t s) {
+  if constexpr (MODE == 2) {
+    if (ls) {
+      AttnLayersK<ST> kl;
+      kl.k = k;
+      std::copy(ls->l, ls->l + ls->n, kl.l);
+      const dim3 grid((unsigned)((a->batch + 1) / 2), (unsigned)a->num_heads, (unsigned)ls->n);
+      hipLaunchKernelGGL((relpos_attn_chunk_kernel<ST, DK, MODE, STREAM, AttnLayersK<ST>>), grid, dim3(256u), 0, s, kl);
+      return check_launch("pk_paged_relpos_attn_layers");
+    }
+  }
   dim3 grid((unsigned)((a->batch + 1) / 2), (unsigned)a->num_heads);
   dim3 block(256u);
   if (a->start_event || a->stop_event) {
-    hipExtLaunchKernelGGL(relpos_attn_chunk_kernel<ST, DK, MODE, STREAM>, grid, block, 0u, s,
+    hipExtLaunchKernelGGL((relpos_attn_chunk_kernel<ST, DK, MODE, STREAM, AttnK<ST>>), grid, block, 0u, s,
                           (hipEvent_t)a->start_event, (hipEvent_t)a->stop_event, 0u, k);
   } else {
-    hipLaunchKernelGGL((relpos_attn_chunk_kernel<ST, DK, MODE, STREAM>), grid, block, 0, s, k);
+    hipLaunchKernelGGL((relpos_attn_chunk_kernel<ST, DK, MODE, STREAM, AttnK<ST>>), grid, block, 0, s, k);
   }
   return check_launch("pk_paged_relpos_attn");
 }
 
 template <typename ST, int DK, int MODE>
-int launch_attn_chunk_mode(const pk_attn_args* a, const AttnK<ST>& k, hipStream_t s) {
+int launch_attn_chunk_mode(const pk_attn_args* a, const AttnK<ST>& k, const LayerSet<ST>* ls, hipStream_t s) {
   const int64_t layers = a->pages.num_layers > 1 ? a->pages.num_layers : 1;
   const int64_t window_bytes = (int64_t)a->batch * k.Lk * a->num_heads * DK * (int64_t)sizeof(ST) * 2 * layers;
-  if (k.pg.rows != nullptr && window_bytes > kStreamingBytes) return launch_attn_chunk_t<ST, DK, MODE, true>(a, k, s);
-  return launch_attn_chunk_t<ST, DK, MODE, false>(a, k, s);
+  if (k.pg.rows != nullptr && window_bytes > kStreamingBytes) return launch_attn_chunk_t<ST, DK, MODE, true>(a, k, ls, s);
+  return launch_attn_chunk_t<ST, DK, MODE, false>(a, k, ls, s);
 }
 
 template <typename ST, int DK>
-int launch_attn_chunk(const pk_attn_args* a, AttnK<ST>& k, hipStream_t s) {
+int launch_attn_chunk(const pk_attn_args* a, AttnK<ST>& k, const LayerSet<ST>* ls, hipStream_t s) {
   k.tiles = 1;
-  if (k.mask) return launch_attn_chunk_mode<ST, DK, 1>(a, k, s);
-  if (k.st_proc) return launch_attn_chunk_mode<ST, DK, 2>(a, k, s);
-  return launch_attn_chunk_mode<ST, DK, 0>(a, k, s);
+  if (k.mask) return launch_attn_chunk_mode<ST, DK, 1>(a, k, ls, s);
+  if (k.st_proc) return launch_attn_chunk_mode<ST, DK, 2>(a, k, ls, s);
+  return launch_attn_chunk_mode<ST, DK, 0>(a, k, ls, s);
 }
 
+// the checked arguments of a call, as the kernels take them (batch > 0)
 template <typename ST>
-int attn_typed(const pk_attn_args* a, hipStream_t s) {
+int attn_build(const pk_attn_args* a, AttnK<ST>& k) {
   constexpr int VEC = Tr<ST>::VEC;
   const char* what = "pk_paged_relpos_attn";
   const int DK = a->head_dim;
@@ -2005,7 +2079,7 @@ int attn_typed(const pk_attn_args* a, hipStream_t s) {
     return fail(PK_ERR_INVALID, "%s: need chunk > 0 and left >= 0", what);
   const int Lk = a->left + a->chunk;
   if (a->batch < 0) return fail(PK_ERR_INVALID, "%s: batch must be >= 0", what);
-  if (a->batch == 0) return PK_OK;
+  if (a->batch == 0) return PK_OK;  // nothing is launched
   if (a->pos_rows < Lk + a->chunk - 1)
     return fail(PK_ERR_INVALID, "%s: pos has %d rows, needs >= window + chunk - 1 = %d", what,
                 a->pos_rows, Lk + a->chunk - 1);
@@ -2025,7 +2099,6 @@ int attn_typed(const pk_attn_args* a, hipStream_t s) {
   if ((int64_t)a->batch * a->num_heads > 0x7fffffffLL)
     return fail(PK_ERR_INVALID, "%s: batch * heads too large", what);
 
-  AttnK<ST> k{};
   k.q = static_cast<const ST*>(a->query);
   k.kn = static_cast<const ST*>(a->key);
   k.vn = static_cast<const ST*>(a->value);
@@ -2092,6 +2165,18 @@ int attn_typed(const pk_attn_args* a, hipStream_t s) {
 
   if (a->num_heads > 65535 || a->chunk > 2 * 65535)
     return fail(PK_ERR_INVALID, "%s: num_heads or chunk exceeds the launch grid", what);
+  return PK_OK;
+}
+
+// ls: the layers of a launch over several (else nullptr); k is the first's.  Takes
+// a launch over several only with a matrix-core kernel and one query pair: else
+// PK_ERR_UNSUPPORTED, and the caller launches them one by one.
+template <typename ST>
+int attn_dispatch(const pk_attn_args* a, AttnK<ST>& k, const LayerSet<ST>* ls, hipStream_t s) {
+  constexpr int VEC = Tr<ST>::VEC;
+  const char* what = "pk_paged_relpos_attn";
+  const int DK = a->head_dim, D = a->num_heads * DK, Lk = a->left + a->chunk;
+  const bool need_pages = a->left > 0 || a->append;
   if constexpr (!std::is_same<ST, float>::value) {
     // the matrix-core kernel addresses rows through buffer resources: row
     // strides up to kMaxBufferStride bytes and fewer than 2^32 pool rows
@@ -2114,21 +2199,22 @@ int attn_typed(const pk_attn_args* a, hipStream_t s) {
       if (!chunk_ok)
         return fail(PK_ERR_UNSUPPORTED, "%s: the whole-chunk kernel needs chunk <= %d, window <= %d, one position table",
                     what, kChunkMaxT, kChunkMaxWindow);
-      if (DK == 64) return launch_attn_chunk<ST, 64>(a, k, s);
-      return launch_attn_chunk<ST, 128>(a, k, s);
+      if (DK == 64) return launch_attn_chunk<ST, 64>(a, k, ls, s);
+      return launch_attn_chunk<ST, 128>(a, k, ls, s);
     }
     if (a->rows_per_lane == 0 && chunk_ok && a->chunk >= 3) {
-      if (DK == 64) return launch_attn_chunk<ST, 64>(a, k, s);
-      return launch_attn_chunk<ST, 128>(a, k, s);
+      if (DK == 64) return launch_attn_chunk<ST, 64>(a, k, ls, s);
+      return launch_attn_chunk<ST, 128>(a, k, ls, s);
     }
-    if ((a->rows_per_lane == 0 || a->rows_per_lane == -1) && mfma_ok && a->chunk <= 16) {
-      if (DK == 64) return launch_attn_mfma<ST, 64>(a, k, s);
-      return launch_attn_mfma<ST, 128>(a, k, s);
+    if ((a->rows_per_lane == 0 || a->rows_per_lane == -1) && mfma_ok && a->chunk <= 16 && !(ls && a->chunk > 2)) {
+      if (DK == 64) return launch_attn_mfma<ST, 64>(a, k, ls, s);
+      return launch_attn_mfma<ST, 128>(a, k, ls, s);
     }
     if (a->rows_per_lane < 0)
       return fail(PK_ERR_UNSUPPORTED, "%s: rows_per_lane %d asks for a matrix-core kernel this call cannot take", what,
                   a->rows_per_lane);
   }
+  if (ls) return PK_ERR_UNSUPPORTED;
   const int G = DK / VEC;
   const int rlw = 64 / G;
   const int TQ = pick_tq(a->chunk);
@@ -2145,6 +2231,64 @@ int attn_typed(const pk_attn_args* a, hipStream_t s) {
   k.tiles = tiles;
   if (DK == 64) return launch_attn_tq<ST, 64>(a, k, TQ, NR, waves, s);
   return launch_attn_tq<ST, 128>(a, k, TQ, NR, waves, s);
+}
+
+template <typename ST>
+int attn_typed(const pk_attn_args* a, hipStream_t s) {
+  AttnK<ST> k{};
+  const int rc = attn_build(a, k);
+  if (rc != PK_OK || a->batch == 0) return rc;
+  return attn_dispatch<ST>(a, k, nullptr, s);
+}
+
+// `n` layers' calls: launches over up to kMaxLaunchLayers of them where they differ
+// in their tensors and layer alone, else one by one.  One grid over the layers has
+// no launch gap and no idle tail between them: 24 layers x 230 streams of the large
+// model 380 -> 298 us (2 frames) and 547 -> 428 us (14 frames); for few streams
+// the launches themselves were the time (17 layers of a few streams 101 -> 36 us).
+template <typename ST>
+int attn_layers_typed(const pk_attn_args* a, int n, hipStream_t s) {
+  for (int i = 0; i < n;) {
+    AttnK<ST> k{};
+    int rc = attn_build(a + i, k);
+    if (rc != PK_OK) return rc;
+    if (a[i].batch == 0) {
+      ++i;
+      continue;
+    }
+    LayerSet<ST> ls;
+    ls.n = 0;
+    const bool plain = k.st_proc && !k.mask && k.pg.rows && !a[i].start_event && !a[i].stop_event && a[i].rows_per_lane == 0;
+    for (int j = i; plain && j < n && ls.n < kMaxLaunchLayers; ++j) {
+      // what may differ, taken from the first; layers ascend, so no two share pages
+      pk_attn_args c = a[j];
+      if (j > i && c.layer <= a[j - 1].layer) break;
+      c.layer = a[i].layer;
+      c.query = a[i].query;
+      c.key = a[i].key;
+      c.value = a[i].value;
+      c.bias_u = a[i].bias_u;
+      c.bias_v = a[i].bias_v;
+      c.out = a[i].out;
+      if (std::memcmp(&c, a + i, sizeof(c)) != 0) break;
+      AttnK<ST> kj{};
+      rc = attn_build(a + j, kj);
+      if (rc != PK_OK) return rc;
+      ls.l[ls.n++] = AttnLayer<ST>{kj.q, kj.kn, kj.vn, kj.bu, kj.bv, kj.kp, kj.vp, kj.out};
+    }
+    if (ls.n > 1) {
+      rc = attn_dispatch<ST>(a + i, k, &ls, s);
+      if (rc == PK_OK) {
+        i += ls.n;
+        continue;
+      }
+      if (rc != PK_ERR_UNSUPPORTED) return rc;
+    }
+    rc = attn_dispatch<ST>(a + i, k, nullptr, s);
+    if (rc != PK_OK) return rc;
+    ++i;
+  }
+  return PK_OK;
 }
 
 template <typename ST>
@@ -2204,6 +2348,25 @@ int pk_paged_relpos_attn(const pk_attn_args* a, void* stream) {
     case PK_DTYPE_F16: return pk::attn_typed<_Float16>(a, s);
     case PK_DTYPE_BF16: return pk::attn_typed<pk::bf16_t>(a, s);
     default: return pk::fail(PK_ERR_INVALID, "pk_paged_relpos_attn: unknown dtype %d", a->dtype);
+  }
+}
+
+int pk_paged_relpos_attn_layers(const pk_attn_args* a, int32_t count, void* stream) {
+  pk::clear_error();
+  if (!a) return pk::fail(PK_ERR_INVALID, "pk_paged_relpos_attn_layers: args is NULL");
+  if (count < 0) return pk::fail(PK_ERR_INVALID, "pk_paged_relpos_attn_layers: count %d < 0", count);
+  for (int32_t i = 1; i < count; ++i)
+    if (a[i].dtype != a[0].dtype || a[i].device != a[0].device)
+      return pk::fail(PK_ERR_INVALID, "pk_paged_relpos_attn_layers: calls of several dtypes or devices");
+  if (count == 0) return PK_OK;
+  pk::DeviceGuard dg(a->device);
+  if (!dg.ok) return pk::fail(PK_ERR_HIP, "pk_paged_relpos_attn_layers: cannot select device %d", a->device);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  switch (a->dtype) {
+    case PK_DTYPE_F32: return pk::attn_layers_typed<float>(a, count, s);
+    case PK_DTYPE_F16: return pk::attn_layers_typed<_Float16>(a, count, s);
+    case PK_DTYPE_BF16: return pk::attn_layers_typed<pk::bf16_t>(a, count, s);
+    default: return pk::fail(PK_ERR_INVALID, "pk_paged_relpos_attn_layers: unknown dtype %d", a->dtype);
   }
 }
 

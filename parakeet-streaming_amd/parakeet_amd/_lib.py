@@ -380,6 +380,7 @@ SIGNATURES = {
     "pk_kv_append": (c_int, [POINTER(KvAppendArgs), c_void_p]),
     "pk_kv_gather": (c_int, [POINTER(KvGatherArgs), c_void_p]),
     "pk_paged_relpos_attn": (c_int, [POINTER(AttnArgs), c_void_p]),
+    "pk_paged_relpos_attn_layers": (c_int, [POINTER(AttnArgs), c_int32, c_void_p]),
     "pk_streaming_mask": (c_int, [POINTER(MaskArgs), c_void_p]),
     "pk_conv_step": (c_int, [POINTER(ConvArgs), c_void_p]),
     "pk_residual_norm": (c_int, [POINTER(ResNormArgs), c_void_p]),

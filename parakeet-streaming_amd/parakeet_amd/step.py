@@ -87,7 +87,7 @@ class AttentionStep:
         self._stage_ev = [torch.cuda.Event() for _ in range(depth)]
         self._stage_used = [False] * depth
         self._stage_i = 0
-        self._args = [self._attn_args(layer, rows_per_lane) for layer in range(Ly)]
+        self._args = (AttnArgs * Ly)(*[self._attn_args(layer, rows_per_lane) for layer in range(Ly)])
         self._stream = ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
         self.batch = 0
         self.graph: torch.cuda.CUDAGraph | None = None
@@ -173,25 +173,24 @@ class AttentionStep:
         return B
 
     def run(self, events=None) -> None:
-        """All layers' fused append + attention for the batch opened last, one
-        launch per layer sized to the batch.  ``events``: optional per-layer
-        (start, stop) pairs timing each kernel."""
+        """All layers' fused append + attention for the batch opened last, sized
+        to it: one launch over every layer (their inputs and pages are each
+        layer's own), or with ``events``, optional per-layer (start, stop) pairs
+        timing each kernel, one per layer."""
         B = self.batch
         if B == 0:
             return
-        L = lib()
+        self._set_args(B, None, events)
+        check(lib().pk_paged_relpos_attn_layers(self._args, len(self._args), self._stream), "pk_paged_relpos_attn_layers")
+
+    def _set_args(self, batch: int, live: int | None, events=None) -> None:
         for layer, a in enumerate(self._args):
-            a.batch = B
-            a.live_streams = None
-            if events is not None:
-                a.start_event, a.stop_event = events[layer]
-            else:
-                a.start_event = a.stop_event = None
-            check(L.pk_paged_relpos_attn(ctypes.byref(a), self._stream), "pk_paged_relpos_attn")
+            a.batch, a.live_streams = batch, live
+            a.start_event, a.stop_event = events[layer] if events is not None else (None, None)
 
     def capture(self) -> None:
-        """Records every layer's launch in a HIP graph: the launches cover all
-        slots and read the live count from the device, so one recording serves
+        """Records the launch over every layer in a HIP graph: it covers all
+        slots and reads the live count from the device, so one recording serves
         every batch size.  The recording holds no memset and no allocation."""
         L = lib()
         g = torch.cuda.CUDAGraph()
@@ -199,11 +198,8 @@ class AttentionStep:
         side.wait_stream(torch.cuda.current_stream(self.device))
         with torch.cuda.graph(g, stream=side):
             stream = ctypes.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)
-            for a in self._args:
-                a.batch = self.num_slots
-                a.live_streams = self.live.data_ptr()
-                a.start_event = a.stop_event = None
-                check(L.pk_paged_relpos_attn(ctypes.byref(a), stream), "pk_paged_relpos_attn")
+            self._set_args(self.num_slots, self.live.data_ptr())
+            check(L.pk_paged_relpos_attn_layers(self._args, len(self._args), stream), "pk_paged_relpos_attn_layers")
         torch.cuda.current_stream(self.device).wait_stream(side)
         self.graph = g
 

@@ -278,3 +278,16 @@ def test_front_end_plan_layout_and_null():
     assert "NULL" in _lib.last_error()
     a.batch = 0
     assert L.pk_fe_plan(ctypes.byref(a)) == _lib.PK_OK
+
+
+def test_attention_layers_args_validated_before_launch():
+    L = _lib.lib()
+    assert L.pk_paged_relpos_attn_layers(None, 1, None) == _lib.PK_ERR_INVALID
+    a = (_lib.AttnArgs * 2)()
+    assert L.pk_paged_relpos_attn_layers(a, -1, None) == _lib.PK_ERR_INVALID
+    assert L.pk_paged_relpos_attn_layers(a, 0, None) == _lib.PK_OK
+    a[0].dtype, a[1].dtype = _lib.DTYPE_F16, _lib.DTYPE_BF16
+    assert L.pk_paged_relpos_attn_layers(a, 2, None) == _lib.PK_ERR_INVALID  # two dtypes
+    a[0].dtype, a[1].device = _lib.DTYPE_BF16, 1
+    assert L.pk_paged_relpos_attn_layers(a, 2, None) == _lib.PK_ERR_INVALID  # two devices
+    assert "several" in _lib.last_error()

@@ -120,3 +120,46 @@ def test_step_graph_replays_match_oracle(cuda, shape):
     replays the test's own eager work runs (uploads, gathers, copies back,
     synchronizations) and every replay is checked against the oracle."""
     _run(cuda, shape, slots=6, steps=30, seed=8, graph=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("streams,layers,d,right", [(1, 3, 512, 1), (5, 33, 512, 0), (37, 4, 512, 1), (9, 5, 1024, 13), (130, 3, 1024, 1), (3, 2, 512, 6)])
+def test_layers_in_one_launch_match_layer_by_layer(cuda, dtype, streams, layers, d, right):
+    """pk_paged_relpos_attn_layers (AttentionStep's launch over every layer; past 32
+    layers two launches, fp32 one by one) against one launch a layer: outputs and
+    pages bit for bit, over steps that evict, with streams of several ages, and
+    replayed from a graph over a smaller batch."""
+    import numpy as np
+
+    from parakeet_amd import synth
+    from parakeet_amd.step import AttentionStep
+
+    T, left = right + 1, 20
+    shape = synth.Shape("layers", layers, d, 8, left=left, right=right, dtype=dtype)
+    g = torch.Generator(device="cuda").manual_seed(streams + layers)
+    pos = torch.randn(2 * (left + T) - 1, d, generator=g, device=cuda).to(dtype)
+    bu, bv = ([torch.randn(8, d // 8, generator=g, device=cuda).to(dtype) for _ in range(layers)] for _ in range(2))
+    qkv = [torch.zeros(streams, T, 3 * d, dtype=dtype, device=cuda) for _ in range(layers)]
+    steps = [AttentionStep(shape, streams, torch.device("cuda", 0), qkv, pos, bu, bv) for _ in range(3)]
+    for st in steps:
+        st.k_pages.zero_()
+        st.v_pages.zero_()
+    rng = np.random.default_rng(0)
+    ev = [tuple(torch.cuda.Event(enable_timing=True) for _ in range(2)) for _ in range(layers)]
+    for a, b in ev:
+        a.record()
+        b.record()
+    for i in range(left // T + 4):
+        n = streams if i % 3 else max(1, streams // 2)
+        slots = np.sort(rng.permutation(streams)[:n]).astype(np.int32)
+        for x in qkv:
+            x.copy_(torch.randn(x.shape, generator=g, device=cuda).to(dtype))
+        steps[0].step(slots)
+        steps[1].step(slots, events=[(a.cuda_event, b.cuda_event) for a, b in ev])  # one launch a layer
+        steps[2].step(slots, graph=True)
+        torch.cuda.synchronize()
+        for other in steps[1:]:
+            assert torch.equal(steps[0].k_pages, other.k_pages) and torch.equal(steps[0].v_pages, other.v_pages)
+            for a, b in zip(steps[0].out, other.out):
+                assert torch.equal(a[:n], b[:n])
