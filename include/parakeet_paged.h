@@ -642,7 +642,7 @@ int pk_fe_plan(pk_fe_plan_args* args);
  * lengths    : int32 [batch] frames of each stream (<= max_frames).
  * tokens     : int32 [batch][max_frames * max_symbols] out: the emitted tokens;
  *              frame_counts: int32 [batch][max_frames] out: tokens per frame.
- * compact    : 0 (by batch size: from 1024 streams), 1 or -1.  Compact mode
+ * compact    : 0 (by batch size: from 512 streams), 1 or -1.  Compact mode
  *              keeps, per iteration, a device list of the streams that emitted a
  *              token: the next symbol's joint and the LSTM and projection
  *              launches run over that list instead of every 16-stream tile that

@@ -8,7 +8,11 @@
 //   conv_chunk_kernel the same step with a chunk's frames in parallel (chunks of
 //                     3 or more frames at small batches); same bits
 //   resnorm_kernel    a Conformer layer's residual update and the LayerNorm
-//                     that reads it (parakeet/modules/encoder.py:58-81)
+//                     that reads it (parakeet/modules/encoder.py:58-81); at a
+//                     layer's end also the next layer's first LayerNorm
+//
+// The encoder's layers take conv_step_kernel / conv_chunk_kernel where the linear
+// kernels do not hold the convolution (fp32, kernels other than 9, chunks over 16).
 //
 // conv_step_kernel: one workgroup per stream.  Lane l of the workgroup owns the channels
 // [l*VEC, (l+1)*VEC) -- one 16-byte chunk, 8 fp16/bf16 or 4 fp32 channels -- so

@@ -73,8 +73,12 @@ struct MmaR<float> {
 constexpr int kVT = 64;                // vocabulary rows per joint workgroup
 constexpr int kJointWaves = kVT / 16;  // a wave per 16 rows
 constexpr int kPredWaves = 2;          // pred_proj columns per workgroup: 16 a wave
-constexpr int kCompactMinBatch = 1024;  // compact mode by default from this batch
-constexpr int kGatherMax = 512;  // streams whose decisions every LSTM workgroup may take itself
+// compact mode by default from this batch.  us a 2-frame step of the small model in
+// fp16, tile by tile and compact, at 1.7 | 0.3 | 0.02 tokens a frame: 256 streams 309
+// 315 | 276 291 | 217 228, 512 streams 431 356 | 377 332 | 299 314, 1000 streams 616
+// 473 | 548 364 | 400 345; the large model's 14 frames at 512 streams 3627 2540 | 2990
+// 2350 | 2039 2120
+constexpr int kCompactMinBatch = 512;
 constexpr int kMaxDim = 1024;  // hidden / joint sizes held in LDS
 // per-stream words of the step workspace: flag, token, emitted count, pad
 constexpr int kWsHead = 4;
@@ -447,14 +451,7 @@ struct LstmCfg {
 // flight beside the decision and the embedding rows of the input part.  The
 // recurrent part continues each gate's MFMA chain from the input part's sums,
 // so the k-steps run in the order of one chain over K = [x ; h].
-// GATHER (the host takes it up to kGatherMax streams out of compact mode): every
-// workgroup takes all streams' decisions (layers above: reads their recorded
-// tokens) and lists the ones that update, in order; tile y holds entries y SPW ..
-// of that list, so the streams that update fill the fewest workgroups and the
-// rest return.  By batch position, nearly every tile of 16 held some stream that
-// updated, and at 128 streams 320 workgroups on 256 CUs ran at every symbol: 13.3 us
-// a launch against 10.3 (and 10.8 for 160 of 32 streams at a first symbol).
-template <typename ST, int SPW, bool GATHER>
+template <typename ST, int SPW>
 __global__ void __launch_bounds__(512) lstm_kernel(const DecK p) {  // LstmCfg::WAVES x 64
 #pragma clang fp contract(off)
   typedef LstmCfg<ST, SPW> Cfg;
@@ -481,104 +478,61 @@ __global__ void __launch_bounds__(512) lstm_kernel(const DecK p) {  // LstmCfg::
   // 0 records it.
   const int pt = tid & 255, k = pt >> 4, c = pt & 15;
   int tk[NE], b[NE], slot[NE];
-  [[maybe_unused]] bool act[NE];
-  [[maybe_unused]] bool rec = false;
-  if constexpr (GATHER) {
-    __shared__ int32_t lb_s[kGatherMax], lt_s[kGatherMax];  // the list: stream, token
-    __shared__ int32_t wn_s[Cfg::WAVES];
-    const int c4 = tid & 3;  // 4 lanes a stream
-    int n = 0;
-    for (int r0 = 0; r0 < p.batch; r0 += 128) {
-      const int sb = r0 + (tid >> 2);
-      int t = -1;
-      if (sb < p.batch) {  // uniform per lane group
-        if (layer == 0) {
-          bool a;
-          t = decide_finish<4>(p, sb, c4, decide_load<4>(p, sb, c4), &a);
-          if (blockIdx.x == 0 && blockIdx.y == 0 && c4 == 0) record(p, sb, a, t);
-        } else if ((uint32_t)p.slots[sb] < (uint32_t)p.num_slots) {
-          t = ws_of(p, sb)[1];
-        }
-      }
-      const uint64_t m = __ballot(t >= 0 && c4 == 0);
-      if (lane == 0) wn_s[wave] = __popcll(m);
-      __syncthreads();
-      int at = n;
-      for (int w = 0; w < Cfg::WAVES; ++w) {
-        if (w < wave) at += wn_s[w];
-        n += wn_s[w];
-      }
-      if (t >= 0 && c4 == 0) {
-        at += __popcll(m & ((1ull << lane) - 1));
-        lb_s[at] = sb;
-        lt_s[at] = t;
-      }
-      __syncthreads();  // the list, and wn_s before the next round
-    }
-    if (b0 >= n) return;  // uniform
+  bool act[NE];
+  const bool deciding = layer == 0 && !p.compact && !p.prime;
+  DecideLoads<16> dl[NE];
 #pragma unroll
-    for (int e = 0; e < NE; ++e) {
-      const int i = b0 + k + 16 * e;
-      b[e] = i < n ? lb_s[i] : -1;
-      tk[e] = i < n ? lt_s[i] : -1;
-      slot[e] = i < n ? p.slots[lb_s[i]] : 0;  // a stream with a token has a valid slot
-    }
-  } else {
-    const bool deciding = layer == 0 && !p.compact && !p.prime;
-    DecideLoads<16> dl[NE];
+  for (int e = 0; e < NE; ++e) {
+    tk[e] = -1;
+    act[e] = false;
+    if (deciding && part == 0) dl[e] = decide_load<16>(p, min(b0 + k + 16 * e, p.batch - 1), c);
+  }
+  // lane c of every 16-lane group reads whether entries c + 16 e may update
+  // (deciding: they are active), so each wave holds all entries: a tile with
+  // none returns before any weight or row load, with no barrier (every wave
+  // sees the same words); entry k + 16 e's stream, token and slot come from
+  // lane k of the thread's group
+  int bq[NE], tq[NE], sq[NE];
+  bool may = false;
 #pragma unroll
-    for (int e = 0; e < NE; ++e) {
-      tk[e] = -1;
-      act[e] = false;
-      if (deciding && part == 0) dl[e] = decide_load<16>(p, min(b0 + k + 16 * e, p.batch - 1), c);
+  for (int e = 0; e < NE; ++e) {
+    const int q = b0 + (lane & 15) + 16 * e;
+    bq[e] = listed ? listed_stream(p, p.it & 1, q) : (q < p.batch ? q : -1);
+    tq[e] = -1;  // deciding: 0 if active
+    sq[e] = 0;
+    if (bq[e] >= 0) {
+      const StreamWords w = stream_words(p, bq[e]);
+      const bool sok = (uint32_t)w.slot < (uint32_t)p.num_slots;
+      sq[e] = sok ? w.slot : 0;
+      if (deciding) tq[e] = active_from(p, w) ? 0 : -1;
+      else if (p.prime) tq[e] = sok ? p.blank : -1;
+      else tq[e] = ws_of(p, bq[e])[1];
     }
-    // lane c of every 16-lane group reads whether entries c + 16 e may update
-    // (deciding: they are active), so each wave holds all entries: a tile with
-    // none returns before any weight or row load, with no barrier (every wave
-    // sees the same words); entry k + 16 e's stream, token and slot come from
-    // lane k of the thread's group
-    int bq[NE], tq[NE], sq[NE];
-    bool may = false;
+    may |= tq[e] >= 0;
+  }
+  const int kl = (lane & 48) | k;  // the lane holding entry k; every lane takes part in the shuffles
 #pragma unroll
-    for (int e = 0; e < NE; ++e) {
-      const int q = b0 + (lane & 15) + 16 * e;
-      bq[e] = listed ? listed_stream(p, p.it & 1, q) : (q < p.batch ? q : -1);
-      tq[e] = -1;  // deciding: 0 if active
-      sq[e] = 0;
-      if (bq[e] >= 0) {
-        const StreamWords w = stream_words(p, bq[e]);
-        const bool sok = (uint32_t)w.slot < (uint32_t)p.num_slots;
-        sq[e] = sok ? w.slot : 0;
-        if (deciding) tq[e] = active_from(p, w) ? 0 : -1;
-        else if (p.prime) tq[e] = sok ? p.blank : -1;
-        else tq[e] = ws_of(p, bq[e])[1];
-      }
-      may |= tq[e] >= 0;
-    }
-    const int kl = (lane & 48) | k;  // the lane holding entry k; every lane takes part in the shuffles
+  for (int e = 0; e < NE; ++e) {
+    b[e] = __shfl(bq[e], kl);
+    slot[e] = __shfl(sq[e], kl);
+    const int t = __shfl(tq[e], kl);
+    if (!deciding) tk[e] = t;
+  }
+  if (deciding && part == 0) {
 #pragma unroll
-    for (int e = 0; e < NE; ++e) {
-      b[e] = __shfl(bq[e], kl);
-      slot[e] = __shfl(sq[e], kl);
-      const int t = __shfl(tq[e], kl);
-      if (!deciding) tk[e] = t;
-    }
-    if (deciding && part == 0) {
+    for (int e = 0; e < NE; ++e)
+      if (b[e] >= 0) tk[e] = decide_finish<16>(p, b[e], c, dl[e], &act[e]);
+  }
+  const bool rec = deciding && part == 0 && blockIdx.x == 0 && c == 0;
+  if (__ballot(may) == 0) {
+    // no stream of the tile is active: column 0 still records every decision
+    // (no token, and the frame's counters at its first symbol)
+    if (rec) {
 #pragma unroll
       for (int e = 0; e < NE; ++e)
-        if (b[e] >= 0) tk[e] = decide_finish<16>(p, b[e], c, dl[e], &act[e]);
+        if (b[e] >= 0) record(p, b[e], act[e], tk[e]);
     }
-    rec = deciding && part == 0 && blockIdx.x == 0 && c == 0;
-    if (__ballot(may) == 0) {
-      // no stream of the tile is active: column 0 still records every decision
-      // (no token, and the frame's counters at its first symbol)
-      if (rec) {
-#pragma unroll
-        for (int e = 0; e < NE; ++e)
-          if (b[e] >= 0) record(p, b[e], act[e], tk[e]);
-      }
-      return;
-    }
+    return;
   }
   // the wave's weight rows: gate gi, units u0 .. u0 + 15, first chunk
   const int64_t row = (int64_t)layer * 4 * H + gi * H + u0;
@@ -824,14 +778,12 @@ static int run_step(const pk_rnnt_args* a, hipStream_t st) {
   const dim3 gj(k.vtiles, (a->batch + 15) / 16);
   // 32 streams a LSTM workgroup (16-bit types only: the fp32 rows of 32 streams
   // do not fit in LDS) in compact mode, where the tiles hold only streams that
-  // update and 32 of them read the weights half as often, and otherwise when
-  // every stream may update (a frame's first symbol, or priming) and that
+  // update and 32 of them read the weights half as often, and by batch position
+  // where every stream may update (a frame's first symbol, or priming) if that
   // leaves no CU with two workgroups; else 16: at later symbols the smaller
   // tiles more often have no update and return early
   const int cus = cu_count();
-  // past kGatherMax streams (and priming): by batch position
-  const bool gather = !k.compact && !k.prime && a->batch <= kGatherMax;
-  const bool wide_fits = sizeof(ST) == 2 && !k.compact && !gather &&
+  const bool wide_fits = sizeof(ST) == 2 && !k.compact &&
                          (int64_t)(a->hidden / 16) * ((a->batch + 15) / 16) > cus &&
                          (int64_t)(a->hidden / 16) * ((a->batch + 31) / 32) <= cus;
   const dim3 gl16(a->hidden / 16, (a->batch + 15) / 16), gl32(a->hidden / 16, (a->batch + 31) / 32);
@@ -839,17 +791,13 @@ static int run_step(const pk_rnnt_args* a, hipStream_t st) {
   auto lstm = [&]() {
     for (int l = 0; l < a->layers; ++l) {
       k.layer = l;
-      if (gather) {
-        hipLaunchKernelGGL((lstm_kernel<ST, 16, true>), gl16, dim3(LstmCfg<ST, 16>::WAVES * 64), 0, st, k);
-        continue;
-      }
       if constexpr (sizeof(ST) == 2) {
         if (k.compact || (wide_fits && (k.prime || k.s == 0))) {
-          hipLaunchKernelGGL((lstm_kernel<ST, 32, false>), gl32, dim3(LstmCfg<ST, 32>::WAVES * 64), 0, st, k);
+          hipLaunchKernelGGL((lstm_kernel<ST, 32>), gl32, dim3(LstmCfg<ST, 32>::WAVES * 64), 0, st, k);
           continue;
         }
       }
-      hipLaunchKernelGGL((lstm_kernel<ST, 16, false>), gl16, dim3(LstmCfg<ST, 16>::WAVES * 64), 0, st, k);
+      hipLaunchKernelGGL((lstm_kernel<ST, 16>), gl16, dim3(LstmCfg<ST, 16>::WAVES * 64), 0, st, k);
     }
   };
   auto pred = [&]() { hipLaunchKernelGGL(pred_kernel<ST>, gp, dim3(kPredWaves * 64), 0, st, k); };

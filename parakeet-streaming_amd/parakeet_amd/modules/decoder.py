@@ -72,7 +72,7 @@ class GreedyDecoder:
     def __init__(self, predictor: nn.Module, joiner: nn.Module, blank_id: int, num_slots: int, max_symbols: int = 5):
         self.pred, self.joiner = predictor, joiner
         self.blank, self.max_symbols = int(blank_id), int(max_symbols)
-        # 0: the library compacts each iteration's updating streams from 1024
+        # 0: the library compacts each iteration's updating streams from 512
         # streams on; 1 / -1: always / never (the outputs are the same)
         self.compact = 0
         self.num_slots = S = int(num_slots)

@@ -8,15 +8,18 @@
   (encoder.py:167-227);
 * ``forward`` keeps the layer loop and the state advance (encoder.py:229-267);
   the attention of every layer runs on the paged cache;
-* ``EncoderStepGraph`` replays a recorded step for a fixed batch: the about 20
+* ``EncoderStepGraph`` replays a recorded step for a fixed batch: the 9 to 13
   launches per layer that ``forward`` issues from Python become one HIP graph
   replay, with the host page work and one upload per step left outside it.
 
-The convolution module's GLU / depthwise conv / LayerNorm / SiLU runs as one HIP
-launch with each stream's conv state updated in place (convolution.py:107-162,
-cache.py:47-53); the feed-forward blocks, layer norms and pointwise projections
-are torch modules with the reference's parameter names (encoder.py:11-81,
-feedforward.py:4-26).  ``pre_encode`` is the batched convolution subsampling of
+The parameters are torch modules with the reference's names (encoder.py:11-81,
+feedforward.py:4-26).  In 16 bits without gradients, a layer's products run on
+``pk_linear``: SiLU in the first feed-forward product, the convolution module's
+GLU and depthwise conv in its first pointwise product with each stream's conv
+state updated in place (convolution.py:107-162, cache.py:47-53), its LayerNorm
+and SiLU ahead of the second, and for few rows each residual update and LayerNorm
+in the product that reads it.  Every other case (fp32, gradients, hooks, other
+sizes) runs the modules, with the conv step as one HIP launch.  ``pre_encode`` is the batched convolution subsampling of
 ``modules/frontend.py`` (one HIP launch for the 8x stack), built from the same
 constructor arguments as the reference's (encoder.py:105-112), so a reference
 checkpoint loads strictly and ``ModelRunner`` finds ``encoder.pre_encode``

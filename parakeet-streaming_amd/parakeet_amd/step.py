@@ -10,9 +10,10 @@ directly and for measurement:
      processed_frames / cache_lengths and its block-table rows (the reference
      gathers the state per step with index_select, parakeet/engine/scheduler.py:
      128-170);
-  2. per layer: one kernel -- fused page append + paged rel-pos attention with
-     the streaming mask evaluated in the kernel from the stream state
-     (attention.py:97-121, encoder.py:167-227);
+  2. one launch over every layer's fused page append + paged rel-pos attention,
+     with the streaming mask evaluated in the kernel from the stream state
+     (attention.py:97-121, encoder.py:167-227); one a layer where a launch is
+     timed or the kernel has no such form (fp32);
   3. advance the state scalars (encoder.py:257-260) on the host mirror.
 
 The engine always feeds whole chunks (parakeet/engine/sequence.py:137-146), so

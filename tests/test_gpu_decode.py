@@ -312,11 +312,11 @@ def test_pending_results_match_blocking_calls(cuda):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("layers,vocab,streams", [(1, 130, 33), (2, 70, 5), (1, 127, 140), (1, 90, 600)])
-def test_packed_weights_and_listed_tiles_give_the_plain_ones(cuda, dtype, layers, vocab, streams):
-    """Weights in operand order against the plain layouts, and the LSTM's list of
-    updating streams (up to 512 streams) against tiles by batch position (compact
-    mode's forms, which the decoder's own tests check): the same tokens and state
-    bits; a vocabulary that fills no whole tile, streams past one list round."""
+def test_packed_weights_give_the_plain_ones(cuda, dtype, layers, vocab, streams):
+    """Weights in operand order against the plain layouts, tile by tile and in
+    compact mode, and the mode the library picks by batch size: the same tokens and
+    state bits; a vocabulary that fills no whole tile, batches on both sides of the
+    line for compact mode."""
     from parakeet_amd.modules.decoder import GreedyDecoder, Joiner, Predictor
 
     torch.manual_seed(layers * 100 + vocab)
@@ -328,13 +328,12 @@ def test_packed_weights_and_listed_tiles_give_the_plain_ones(cuda, dtype, layers
     x = torch.randn(3, streams, 2, 512, device=cuda).to(dtype)
     slots = np.random.default_rng(0).permutation(streams)
     results = []
-    for mode in ("packed", "plain", "compact"):
+    for mode in ("packed", "plain", "compact", "by size"):
         dec = GreedyDecoder(pred, joint, blank_id=vocab, num_slots=streams)
         if mode == "plain":
             for k in ("w_ih", "w_hh", "w_pred", "w_out"):
                 delattr(dec, k + "_packed")
-        if mode == "compact":
-            dec.compact = 1
+        dec.compact = {"compact": 1, "by size": 0}.get(mode, -1)
         dec.reset_slot(slots)
         toks = [[list(t) for t in dec.decode(slots, x[i], lengths=None if i else [1 + (b % 2) for b in range(streams)])] for i in range(3)]
         results.append((toks, dec.h.clone(), dec.c.clone(), dec.pred_proj.clone()))
