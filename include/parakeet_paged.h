@@ -322,8 +322,8 @@ int pk_conv_step(const pk_conv_args* args, void* stream);
  * norm_self_att, norm_conv, norm_feed_forward2 and norm_out that read them.
  * residual, branch, residual_out, norm_out: [rows][d_model] of `dtype` with row
  * strides in elements (channels contiguous, 16-byte aligned rows);
- * residual_out may be residual (updated in place), or NULL where nothing reads
- * it; norm_out may be branch; no other overlap.  ln_weight, ln_bias: [d_model].  d_model a multiple of 8
+ * residual_out may be residual (updated in place), or with ln2_weight NULL, where
+ * nothing reads it; norm_out may be branch; no other overlap.  ln_weight, ln_bias: [d_model].  d_model a multiple of 8
  * (fp16/bf16) or 4 (fp32), at most 4096 (fp16/bf16) or 2048 (fp32).
  */
 typedef struct pk_resnorm_args {

@@ -583,7 +583,7 @@ int resnorm_typed(const pk_resnorm_args* a, hipStream_t s) {
   if (!(a->alpha == a->alpha) || a->alpha == INFINITY || a->alpha == -INFINITY)
     return fail(PK_ERR_INVALID, "%s: alpha must be finite", what);
   if (a->rows == 0) return PK_OK;
-  const void* ptrs[6] = {a->residual, a->branch, a->ln_weight, a->ln_bias, a->residual_out ? a->residual_out : a->norm_out, a->norm_out};
+  const void* ptrs[6] = {a->residual, a->branch, a->ln_weight, a->ln_bias, a->residual_out || !a->ln2_weight ? a->residual_out : a->norm_out, a->norm_out};
   for (const void* q : ptrs) {
     if (!q) return fail(PK_ERR_INVALID, "%s: a tensor pointer is NULL", what);
     if (!aligned16(q)) return fail(PK_ERR_INVALID, "%s: tensors must be 16-byte aligned", what);

@@ -1507,8 +1507,8 @@ extern "C" int pk_fe_step(const pk_fe_args* a, void* stream) {
   k.guard = a->log_guard;
   k.seed_lo = (uint32_t)a->seed;
   k.seed_hi = (uint32_t)(a->seed >> 32);
-  // four frames a wave when the batch fills the CUs several times over with
-  // such workgroups (and the hop fits their sample staging), one otherwise
+  // four frames a wave when the batch gives at least 3 such workgroups per 2 CUs
+  // (and the hop fits their sample staging), one otherwise
   const int wide_frames = 4 * kFeWaves;
   const int64_t gx4 = a->max_frames > 0 ? (a->max_frames + wide_frames - 1) / wide_frames : 1;
   const bool wide = a->hop <= kFeHopWide && 2 * gx4 * a->batch >= (int64_t)kFeWideTwice * cu_count();

@@ -174,7 +174,10 @@ class ConformerLayer(nn.Module):
         """Whether :meth:`fused_step` is this layer's step on ``x``: every module
         of it is the class's own (no subclass, hook, replaced forward or active
         dropout that the fused launches would pass by) on one 16-bit dtype, and
-        no gradient is asked for."""
+        no gradient is asked for.  Past the sizes at which the first pointwise
+        product takes the convolution with it, the modules one by one are as fast
+        or faster: 2772 rows x 1024 292 us a layer against 297, 3584 rows 326
+        against 336 (2100 rows, where it does, 269 against 262)."""
         attn, conv = self.self_attn, self.conv
         return (
             isinstance(cache, ModelCache)
@@ -193,6 +196,7 @@ class ConformerLayer(nn.Module):
                 for n in (self.norm_feed_forward1, self.norm_self_att, self.norm_conv, self.norm_feed_forward2, self.norm_out)
             )
             and attn.qkv.weight.dtype == conv.pointwise_conv1.weight.dtype == x.dtype
+            and x.numel() // x.shape[-1] * conv.pointwise_conv1.weight.numel() <= ops._LINEAR_PRODUCTS
         )
 
     def fused_step(self, x, pos_emb: Tensor, pad_mask: Tensor, attn_mask: Tensor, cache: ModelCache) -> ops.Pending:
