@@ -468,6 +468,13 @@ def conv_step(
     return out
 
 
+def _match(residual: torch.Tensor, branch: torch.Tensor) -> None:
+    """What a residual update takes: operands of one shape and dtype."""
+    if residual.shape != branch.shape or residual.dtype != branch.dtype:
+        raise ValueError(f"residual {tuple(residual.shape)} {residual.dtype} and branch "
+                         f"{tuple(branch.shape)} {branch.dtype} must match")
+
+
 def residual_norm(
     residual: torch.Tensor,
     branch: torch.Tensor,
@@ -487,9 +494,7 @@ def residual_norm(
 
     residual, branch: [..., D] of one dtype and shape (``residual`` contiguous
     when ``in_place``); ln_weight, ln_bias: [D] of the same dtype."""
-    if residual.shape != branch.shape or residual.dtype != branch.dtype:
-        raise ValueError(f"residual {tuple(residual.shape)} {residual.dtype} and branch "
-                         f"{tuple(branch.shape)} {branch.dtype} must match")
+    _match(residual, branch)
     D = int(residual.shape[-1])
     dt = residual.dtype
     for name, v in (("ln_weight", ln_weight), ("ln_bias", ln_bias)):
@@ -525,6 +530,8 @@ def residual_norm2(pend: "Pending", norm2: torch.nn.LayerNorm) -> tuple[torch.Te
     """``y = norm(x + alpha * branch)`` of a :class:`Pending` update and
     ``norm2(y)``, in one launch: a layer's norm_out and the next layer's
     norm_feed_forward1 (encoder.py:58-60,80)."""
+    _match(pend.x, pend.branch)
+    _require_device(pend.x, pend.branch)
     x, br = _aligned_rows(pend.x), _aligned_rows(pend.branch)
     D = x.shape[-1]
     y, z = torch.empty_like(x), torch.empty_like(x)
@@ -719,8 +726,11 @@ def norm_linear(
             return r, linear(h, weight, bias, silu=silu)
         y = torch.nn.functional.linear(h, weight, bias)
         return r, torch.nn.functional.silu(y) if silu else y
-    first = _aligned_rows(first)
     br = pend.branch if pend is not None else branch
+    if br is not None:
+        _match(first, br)
+        _require_device(first, br)
+    first = _aligned_rows(first)
     out = torch.empty((*first.shape[:-1], n), dtype=dt, device=dev)
     a = LinearArgs()
     _linear_args(a, _DTYPES[dt], dev, first, rows, weight, bias, out, silu)
@@ -787,6 +797,8 @@ def glu_conv(
     y = torch.empty((B, T, D), dtype=torch.float32, device=dev)
     a, c = LinearArgs(), ConvArgs()
     if fused:
+        _match(x, branch)
+        _require_device(x, branch)
         x, branch = _aligned_rows(x), _aligned_rows(branch)
         r = torch.empty_like(x)
         _linear_args(a, _DTYPES[dt], dev, x, rows, weight, bias, y, False)
