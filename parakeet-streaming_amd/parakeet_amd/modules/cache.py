@@ -363,6 +363,13 @@ class ModelCache:
             eps=eps,
         )
 
+    def takes_glu_conv(self, x: Tensor) -> bool:
+        """Whether :meth:`glu_conv` updates this conv state for x [B, T, D]: the 8
+        rows of 9 taps, of x's width and dtype, on its device (any other state goes
+        to :meth:`conv_step`, which takes it or says what is wrong with it)."""
+        f = self.conv_frames
+        return f.dtype == x.dtype and f.device == x.device and f.is_contiguous() and tuple(f.shape[2:]) == (8, x.shape[-1])
+
     def glu_conv(self, layer_idx: int, x, branch, norm, weight, bias, dw_weight, dw_bias, pad_mask):
         """``ops.glu_conv`` on this batch's conv state of a layer."""
         if x.shape[0] != self.batch_size:

@@ -212,7 +212,7 @@ class ConformerLayer(nn.Module):
         a = attn.attend(qkv, pos_emb, attn_mask, cache)
         p1, p2, dw, bn = conv.pointwise_conv1, conv.pointwise_conv2, conv.depthwise_conv, conv.batch_norm
         w1, w2 = p1.weight.squeeze(-1), p2.weight.squeeze(-1)
-        if ops.glu_conv_applies(r, w1, p1.bias, w2, p2.bias, dw, bn) and cache.conv_frames.dtype == r.dtype:
+        if ops.glu_conv_applies(r, w1, p1.bias, w2, p2.bias, dw, bn) and cache.takes_glu_conv(r):
             r, y = cache.glu_conv(self.layer_idx, r, a, self.norm_conv, w1, p1.bias, dw.weight, dw.bias, pad_mask)
             c = ops.norm_silu_linear(y, bn, w2, p2.bias)
         else:

@@ -383,6 +383,33 @@ def hbm_read_probe(src: torch.Tensor, out: torch.Tensor, workgroups: int = 0, st
           "pk_hbm_read_probe")
 
 
+def _conv_operands(x, cache, dw_weight, vecs, slots, layer: int, B: int, D: int):
+    """What a convolution step reads and writes, checked against x's dtype and
+    device: the state [slots, layers, K-1, D], the taps [D, 1, K] or [D, K],
+    vectors [D] (name, tensor), the slot map.  Returns (taps, slots, layers, K, device)."""
+    dt = x.dtype
+    if cache.dim() != 4 or cache.shape[3] != D or cache.dtype != dt or not cache.is_contiguous():
+        raise ValueError(f"cache must be contiguous [slots, layers, K-1, {D}] of {dt}, got {tuple(cache.shape)} {cache.dtype}")
+    S, Ly, R, _ = (int(v) for v in cache.shape)
+    K = R + 1
+    w = dw_weight.reshape(dw_weight.shape[0], -1) if dw_weight.dim() == 3 else dw_weight
+    if tuple(w.shape) != (D, K) or w.dtype != dt or not w.is_contiguous():
+        raise ValueError(f"dw_weight must be contiguous [{D}, 1, {K}] or [{D}, {K}] of {dt}")
+    for name, v in vecs:
+        if tuple(v.shape) != (D,) or v.dtype != dt or not v.is_contiguous():
+            raise ValueError(f"{name} must be contiguous [{D}] of {dt}")
+    tensors = [x, cache, w] + [v for _, v in vecs]
+    if slots is not None:
+        if slots.dtype != torch.int32 or tuple(slots.shape) != (B,) or not slots.is_contiguous():
+            raise ValueError(f"slots must be contiguous int32 [{B}]")
+        tensors.append(slots)
+    elif B > S:
+        raise ValueError(f"batch {B} exceeds {S} cache slots")
+    if not 0 <= int(layer) < Ly:
+        raise IndexError(f"layer {layer} out of range [0, {Ly})")
+    return w, S, Ly, K, _require_device(*tensors)
+
+
 def conv_step(
     glu_in: torch.Tensor,
     cache: torch.Tensor,
@@ -416,27 +443,8 @@ def conv_step(
     dt = glu_in.dtype
     if glu_in.stride(2) != 1:
         raise ValueError("glu_in: last dimension must be contiguous")
-    if cache.dim() != 4 or cache.shape[3] != D or cache.dtype != dt or not cache.is_contiguous():
-        raise ValueError(f"cache must be contiguous [slots, layers, K-1, {D}] of {dt}, got {tuple(cache.shape)} {cache.dtype}")
-    S, Ly, R, _ = (int(x) for x in cache.shape)
-    K = R + 1
-    w = dw_weight.reshape(dw_weight.shape[0], -1) if dw_weight.dim() == 3 else dw_weight
-    if tuple(w.shape) != (D, K) or w.dtype != dt or not w.is_contiguous():
-        raise ValueError(f"dw_weight must be contiguous [{D}, 1, {K}] or [{D}, {K}] of {dt}")
     vecs = [("ln_weight", ln_weight), ("ln_bias", ln_bias)] + ([("dw_bias", dw_bias)] if dw_bias is not None else [])
-    for name, v in vecs:
-        if tuple(v.shape) != (D,) or v.dtype != dt or not v.is_contiguous():
-            raise ValueError(f"{name} must be contiguous [{D}] of {dt}")
-    tensors = [glu_in, cache, w, ln_weight, ln_bias] + ([dw_bias] if dw_bias is not None else [])
-    if slots is not None:
-        if slots.dtype != torch.int32 or tuple(slots.shape) != (B,) or not slots.is_contiguous():
-            raise ValueError(f"slots must be contiguous int32 [{B}]")
-        tensors.append(slots)
-    elif B > S:
-        raise ValueError(f"batch {B} exceeds {S} cache slots")
-    if not 0 <= int(layer) < Ly:
-        raise IndexError(f"layer {layer} out of range [0, {Ly})")
-    dev = _require_device(*tensors)
+    w, S, Ly, K, dev = _conv_operands(glu_in, cache, dw_weight, vecs, slots, layer, B, D)
     if out is None:
         out = torch.empty((B, T, D), dtype=dt, device=dev)
     _rows3(out, "out", B, T, D, dt)
@@ -765,7 +773,9 @@ def glu_conv_applies(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor |
         and w.device == x.device
         and w.is_contiguous()
         and w.data_ptr() % 16 == 0
-        and (dw.bias is None or (dw.bias.dtype == x.dtype and dw.bias.is_contiguous() and dw.bias.data_ptr() % 16 == 0))
+        and (dw.bias is None or (tuple(dw.bias.shape) == (D,) and dw.bias.dtype == x.dtype and dw.bias.device == x.device
+                                 and dw.bias.is_contiguous() and dw.bias.data_ptr() % 16 == 0))
+        and not (torch.is_grad_enabled() and (w.requires_grad or (dw.bias is not None and dw.bias.requires_grad)))
         and norm_applies(norm, x)
         and weight.shape[0] == 2 * D
         and layer_applies(x.dtype, x.device, B * T, weight, bias)
@@ -792,12 +802,16 @@ def glu_conv(
     in place.  Returns r (x itself where the update is a launch of its own) and
     the convolution's fp32 output [B, T, D]."""
     B, T, D = x.shape
-    rows, dev, dt = B * T, x.device, x.dtype
+    rows, dt = B * T, x.dtype
+    _match(x, branch)
+    vecs = [("dw_bias", dw_bias)] if dw_bias is not None else []
+    taps, S, Ly, K, dev = _conv_operands(x, conv_cache, dw_weight, vecs, slots, layer, B, D)
+    if tuple(weight.shape) != (2 * D, D) or weight.dtype != dt or weight.device != dev:
+        raise ValueError(f"weight must be [{2 * D}, {D}] of {dt} on {dev}")
     fused = bool(lib().pk_linear_takes_norm(rows, 2 * D, D, T))
     y = torch.empty((B, T, D), dtype=torch.float32, device=dev)
     a, c = LinearArgs(), ConvArgs()
     if fused:
-        _match(x, branch)
         _require_device(x, branch)
         x, branch = _aligned_rows(x), _aligned_rows(branch)
         r = torch.empty_like(x)
@@ -810,8 +824,8 @@ def glu_conv(
         r, h = residual_norm(x, branch, norm.weight, norm.bias, eps=norm.eps, in_place=True)
         _linear_args(a, _DTYPES[dt], dev, h, rows, weight, bias, y, False)
     a.activation, a.out_stride = _lib.ACT_GLU_CONV, D
-    c.batch, c.chunk, c.d_model, c.kernel = B, T, D, 9
-    c.cache, c.num_slots, c.num_layers, c.layer = conv_cache.data_ptr(), conv_cache.shape[0], conv_cache.shape[1], int(layer)
+    c.batch, c.chunk, c.d_model, c.kernel = B, T, D, K
+    c.cache, c.num_slots, c.num_layers, c.layer = conv_cache.data_ptr(), S, Ly, int(layer)
     c.slots = slots.data_ptr() if slots is not None else None
     if pad_mask is not None:
         if pad_mask.dtype not in (torch.bool, torch.uint8) or tuple(pad_mask.shape) != (B, T):
@@ -822,7 +836,7 @@ def glu_conv(
         c.pad_mask = pad_mask.data_ptr()
     else:
         c.length_scalar = T
-    c.dw_weight, c.dw_bias = dw_weight.data_ptr(), dw_bias.data_ptr() if dw_bias is not None else None
+    c.dw_weight, c.dw_bias = taps.data_ptr(), dw_bias.data_ptr() if dw_bias is not None else None
     a.conv = ctypes.pointer(c)
     check(lib().pk_linear(ctypes.byref(a), 1, _stream(dev)), "pk_linear")
     return r, y

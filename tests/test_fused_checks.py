@@ -54,3 +54,59 @@ def test_branch_must_match_the_residual(no_launch, entry, branch):
             ops.residual_norm2(ops.Pending(x, br, n, 0.5), n)
         else:
             ops.glu_conv(x, br, n, w, None, _half(512, 1, 9), None, _half(2, 1, 8, 512), 0, None, None)
+
+
+def _conv_args(cache=(2, 1, 8, 512), dw=(512, 1, 9), db=(512,), layer=0, slots=None, weight=(1024, 512)):
+    return (_half(*weight), None, _half(*dw), None if db is None else _half(*db), _half(*cache), layer, slots, None)
+
+
+BAD_CONV = {
+    "a cache of 4 rows": (dict(cache=(2, 1, 4, 512)), ValueError, "dw_weight"),
+    "a cache of 10 rows": (dict(cache=(2, 1, 10, 512)), ValueError, "dw_weight"),
+    "a narrower cache": (dict(cache=(2, 1, 8, 256)), ValueError, "cache must be"),
+    "a cache of 3 dimensions": (dict(cache=(2, 8, 512)), ValueError, "cache must be"),
+    "fewer slots than streams": (dict(cache=(1, 1, 8, 512)), ValueError, "slots"),
+    "a layer past the cache": (dict(layer=1), IndexError, "out of range"),
+    "a slot map of int64": (dict(slots=torch.zeros(2, dtype=torch.int64)), ValueError, "int32"),
+    "a shorter slot map": (dict(slots=torch.zeros(1, dtype=torch.int32)), ValueError, "int32"),
+    "a shorter depthwise bias": (dict(db=(256,)), ValueError, "dw_bias"),
+    "fewer taps": (dict(dw=(512, 1, 5)), ValueError, "dw_weight"),
+    "a narrower product": (dict(weight=(1024, 256)), ValueError, "weight must be"),
+}
+
+
+@pytest.mark.parametrize("what", list(BAD_CONV))
+def test_glu_conv_refuses_a_state_that_does_not_fit(no_launch, monkeypatch, what):
+    """The kernel indexes the state as [slot][layer][8][D]: what conv_step refuses,
+    the launch that replaces it refuses too."""
+    kw, error, match = BAD_CONV[what]
+    monkeypatch.setattr(ops, "_require_device", lambda *t: t[0].device)
+    x = _half(2, 2, 512)
+    with pytest.raises(error, match=match):
+        ops.glu_conv(x, x, _ln(512), *_conv_args(**kw))
+
+
+@pytest.mark.parametrize("shape,dtype,takes", [((2, 1, 8, 512), torch.float16, True), ((2, 1, 4, 512), torch.float16, False),
+                                               ((2, 1, 8, 1024), torch.float16, False), ((2, 1, 8, 512), torch.float32, False)])
+def test_conv_state_of_another_shape_takes_the_conv_step(shape, dtype, takes):
+    from parakeet_amd.modules.cache import ModelCache
+
+    cache = types.SimpleNamespace(conv_frames=torch.zeros(shape, dtype=dtype))
+    assert ModelCache.takes_glu_conv(cache, _half(2, 2, 512)) is takes
+
+
+def test_glu_conv_applies_looks_at_the_depthwise_parameters():
+    w1, w2, n = _half(1024, 512), _half(512, 512), _ln(512)
+    x = _half(2, 2, 512)
+
+    def applies(**kw):
+        dw = nn.Conv1d(512, 512, 9, groups=512).half().requires_grad_(False)
+        for k, v in kw.items():
+            setattr(dw, k, v)
+        return ops.glu_conv_applies(x, w1, None, w2, None, dw, n)
+
+    assert applies() and applies(bias=None)
+    assert not applies(bias=nn.Parameter(_half(256), requires_grad=False))
+    assert not applies(bias=nn.Parameter(torch.zeros(512, device="meta", dtype=torch.float16), requires_grad=False))
+    assert not applies(weight=nn.Parameter(_half(512, 1, 9)))  # a gradient is asked for
+    assert not applies(bias=nn.Parameter(_half(512)))
