@@ -54,7 +54,7 @@ class ConformerFeedForward(nn.Module):
         l1, l2 = self.linear1, self.linear2
         if self._fused() and ops.linear_applies(x, l1.weight, l1.bias, silu=True):
             rows = x.numel() // x.shape[-1]
-            if ops.plain_module(l2, nn.Linear) and ops.layer_applies(x.dtype, x.device, rows, l2.weight, l2.bias):
+            if ops.plain_module(l2, nn.Linear) and l2.weight.shape[1:] == l1.weight.shape[:1] and ops.layer_applies(x.dtype, x.device, rows, l2.weight, l2.bias):
                 return ops.feed_forward(x, l1.weight, l1.bias, l2.weight, l2.bias)
             return l2(ops.linear(x, l1.weight, l1.bias, silu=True))
         return l2(self.dropout(self.activation(l1(x))))

@@ -544,11 +544,11 @@ def residual_norm2(pend: "Pending", norm2: torch.nn.LayerNorm) -> tuple[torch.Te
     D = x.shape[-1]
     y, z = torch.empty_like(x), torch.empty_like(x)
     a = ResNormArgs()
-    a.dtype, a.device = dtype_code(x.dtype), x.device.index
+    a.dtype, a.device = dtype_code(x.dtype), x.device.index or 0
     a.rows, a.d_model, a.alpha = x.numel() // D, D, float(pend.alpha)
     a.residual, a.residual_stride, a.branch, a.branch_stride = x.data_ptr(), D, br.data_ptr(), D
-    a.ln_weight, a.ln_bias, a.ln_eps = _ln(pend.norm)
-    a.ln2_weight, a.ln2_bias, a.ln2_eps = _ln(norm2)
+    a.ln_weight, a.ln_bias, a.ln_eps = _ln(pend.norm, D, x.dtype, x.device)
+    a.ln2_weight, a.ln2_bias, a.ln2_eps = _ln(norm2, D, x.dtype, x.device)
     a.norm_out, a.norm_out_stride, a.norm2_out, a.norm2_out_stride = y.data_ptr(), D, z.data_ptr(), D
     check(lib().pk_residual_norm(ctypes.byref(a), _stream(x.device)), "pk_residual_norm")
     return y, z
@@ -584,6 +584,11 @@ def plain_module(m: torch.nn.Module, cls: type) -> bool:
     )
 
 
+def _plain(t: torch.Tensor) -> bool:
+    """Whether ``t`` is a dense tensor whose memory is its value: no subclass."""
+    return type(t) in (torch.Tensor, torch.nn.Parameter) and t.layout == torch.strided
+
+
 # past this many products torch's library GEMM is at least as fast as pk_linear:
 # 840 x 1024 x 4096 17.3 us against 19.1, 1792 x 1024 x 4096 27.6 against 27.6,
 # 3584 x 1024 x 4096 39.8 against 39.5, 3584 x 3072 x 1024 37 against 27.
@@ -593,9 +598,9 @@ _LINEAR_PRODUCTS = 4_500_000_000
 
 
 def layer_applies(dtype: torch.dtype, device: torch.device, rows: int, weight: torch.Tensor, bias: torch.Tensor | None, silu: bool = False) -> bool:
-    """Whether :func:`linear` takes a layer on ``rows`` rows of ``dtype``, and is
-    the faster way to run it."""
-    if type(weight) not in (torch.Tensor, torch.nn.Parameter) or weight.dtype != dtype or weight.device != device:
+    """Whether :func:`linear` takes a layer on ``rows`` rows of ``dtype`` as wide
+    as the weight, and is the faster way to run it."""
+    if not _plain(weight) or weight.dim() != 2 or weight.dtype != dtype or weight.device != device:
         return False
     n, k = weight.shape
     if n % 64 or k % 256 or n == 0 or k == 0 or rows == 0:
@@ -605,7 +610,10 @@ def layer_applies(dtype: torch.dtype, device: torch.device, rows: int, weight: t
         return False
     if max((n - 1) * ld + k, rows * k, rows * n) >= 1 << 31:
         return False
-    if bias is not None and (bias.dtype != dtype or bias.device != device or not bias.is_contiguous() or bias.data_ptr() % 16):
+    if bias is not None and (
+        not _plain(bias) or tuple(bias.shape) != (n,) or bias.dtype != dtype or bias.device != device
+        or not bias.is_contiguous() or bias.data_ptr() % 16
+    ):
         return False
     if not silu and rows * n * k > _LINEAR_PRODUCTS:
         return False
@@ -618,14 +626,19 @@ def linear_applies(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | N
     if x.dtype not in (torch.float16, torch.bfloat16) or x.device.type != "cuda" or x.dim() == 0:
         return False
     k = x.shape[-1]
-    if weight.dim() != 2 or weight.shape[1] != k or (torch.is_grad_enabled() and x.requires_grad) or _transformed(x):
+    if not _plain(weight) or weight.dim() != 2 or weight.shape[1] != k or (torch.is_grad_enabled() and x.requires_grad) or _transformed(x):
         return False
     return k > 0 and layer_applies(x.dtype, x.device, x.numel() // k, weight, bias, silu)
 
 
-def _linear_args(a: LinearArgs, code: int, dev: torch.device, x: torch.Tensor, rows: int, weight, bias, out, silu: bool) -> None:
+def _linear_args(a: LinearArgs, dt: torch.dtype, dev: torch.device, x: torch.Tensor, rows: int, weight, bias, out, silu: bool) -> None:
     n, k = weight.shape
-    a.dtype, a.device = code, dev.index
+    if k != x.shape[-1] or weight.dtype != dt or weight.device != dev:
+        raise ValueError(f"weight {tuple(weight.shape)} {weight.dtype} on {weight.device} does not take x "
+                         f"{tuple(x.shape)} of {dt} on {dev}")
+    if bias is not None and (tuple(bias.shape) != (n,) or bias.dtype != dt or bias.device != dev):
+        raise ValueError(f"bias must be [{n}] of {dt} on {dev}")
+    a.dtype, a.device = _DTYPES[dt], dev.index or 0
     a.rows, a.n, a.k = rows, n, k
     a.activation = _lib.ACT_SILU if silu else _lib.ACT_NONE
     a.x, a.x_stride = x.data_ptr(), k
@@ -651,7 +664,7 @@ def linear(
     elif tuple(out.shape) != (*x.shape[:-1], n) or out.dtype != x.dtype or out.device != x.device or not out.is_contiguous():
         raise ValueError(f"out must be contiguous {(*x.shape[:-1], n)} of {x.dtype} on {x.device}")
     a = LinearArgs()
-    _linear_args(a, _DTYPES[x.dtype], x.device, x, x.numel() // k, weight, bias, out, silu)
+    _linear_args(a, x.dtype, x.device, x, x.numel() // k, weight, bias, out, silu)
     check(lib().pk_linear(ctypes.byref(a), 1, _stream(x.device)), "pk_linear")
     return out
 
@@ -681,7 +694,10 @@ class Pending:
     alpha: float
 
 
-def _ln(m: torch.nn.LayerNorm):
+def _ln(m: torch.nn.LayerNorm, D: int, dt: torch.dtype, dev: torch.device):
+    for name, v in (("weight", m.weight), ("bias", m.bias)):
+        if tuple(v.shape) != (D,) or v.dtype != dt or v.device != dev or not v.is_contiguous():
+            raise ValueError(f"the LayerNorm's {name} must be contiguous [{D}] of {dt} on {dev}")
     return m.weight.data_ptr(), m.bias.data_ptr(), float(m.eps)
 
 
@@ -692,6 +708,9 @@ def norm_applies(m: torch.nn.Module, x: torch.Tensor) -> bool:
         and m.normalized_shape == (x.shape[-1],)
         and m.weight is not None
         and m.bias is not None
+        and _plain(m.weight)
+        and _plain(m.bias)
+        and m.weight.shape == m.bias.shape == m.normalized_shape
         and m.weight.dtype == x.dtype == m.bias.dtype
         and m.weight.device == x.device == m.bias.device
         and m.weight.is_contiguous()
@@ -723,14 +742,15 @@ def norm_linear(
     n, k = weight.shape
     dev, dt = first.device, first.dtype
     rows = first.numel() // k
-    if not (lib().pk_linear_takes_norm(rows, n, k, 0) and (silu or branch is not None) and layer_applies(dt, dev, rows, weight, bias, silu)):
+    fits = first.shape[-1] == k and layer_applies(dt, dev, rows, weight, bias, silu)
+    if not (fits and lib().pk_linear_takes_norm(rows, n, k, 0) and (silu or branch is not None)):
         if pend is not None:
             r, h = residual_norm2(pend, norm)
         elif branch is not None:
             r, h = residual_norm(x, branch, norm.weight, norm.bias, alpha=alpha, eps=norm.eps, in_place=in_place)
         else:
             r, h = x, norm(x)
-        if layer_applies(dt, dev, rows, weight, bias, silu):
+        if fits:
             return r, linear(h, weight, bias, silu=silu)
         y = torch.nn.functional.linear(h, weight, bias)
         return r, torch.nn.functional.silu(y) if silu else y
@@ -741,8 +761,8 @@ def norm_linear(
     first = _aligned_rows(first)
     out = torch.empty((*first.shape[:-1], n), dtype=dt, device=dev)
     a = LinearArgs()
-    _linear_args(a, _DTYPES[dt], dev, first, rows, weight, bias, out, silu)
-    a.ln_weight, a.ln_bias, a.ln_eps = _ln(norm)
+    _linear_args(a, dt, dev, first, rows, weight, bias, out, silu)
+    a.ln_weight, a.ln_bias, a.ln_eps = _ln(norm, k, dt, dev)
     r = first
     if br is None:
         a.prologue = _lib.PRO_NORM
@@ -753,7 +773,7 @@ def norm_linear(
         a.residual_out, a.residual_out_stride = r.data_ptr(), k
         if pend is not None:
             a.prologue, a.alpha = _lib.PRO_RESIDUAL_NORM2, pend.alpha
-            a.ln0_weight, a.ln0_bias, a.ln0_eps = _ln(pend.norm)
+            a.ln0_weight, a.ln0_bias, a.ln0_eps = _ln(pend.norm, k, dt, dev)
         else:
             a.prologue, a.alpha = _lib.PRO_RESIDUAL_NORM, alpha
     check(lib().pk_linear(ctypes.byref(a), 1, _stream(dev)), "pk_linear")
@@ -768,16 +788,18 @@ def glu_conv_applies(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor |
     return (
         D in (512, 1024)
         and 1 <= T <= 16
+        and _plain(w)
         and tuple(w.shape) == (D, 1, 9)
         and w.dtype == x.dtype
         and w.device == x.device
         and w.is_contiguous()
         and w.data_ptr() % 16 == 0
-        and (dw.bias is None or (tuple(dw.bias.shape) == (D,) and dw.bias.dtype == x.dtype and dw.bias.device == x.device
+        and (dw.bias is None or (_plain(dw.bias) and tuple(dw.bias.shape) == (D,) and dw.bias.dtype == x.dtype and dw.bias.device == x.device
                                  and dw.bias.is_contiguous() and dw.bias.data_ptr() % 16 == 0))
         and not (torch.is_grad_enabled() and (w.requires_grad or (dw.bias is not None and dw.bias.requires_grad)))
         and norm_applies(norm, x)
-        and weight.shape[0] == 2 * D
+        and tuple(weight.shape) == (2 * D, D)
+        and w2.shape[1] == D
         and layer_applies(x.dtype, x.device, B * T, weight, bias)
         and layer_applies(x.dtype, x.device, B * T, w2, b2)
     )
@@ -806,8 +828,8 @@ def glu_conv(
     _match(x, branch)
     vecs = [("dw_bias", dw_bias)] if dw_bias is not None else []
     taps, S, Ly, K, dev = _conv_operands(x, conv_cache, dw_weight, vecs, slots, layer, B, D)
-    if tuple(weight.shape) != (2 * D, D) or weight.dtype != dt or weight.device != dev:
-        raise ValueError(f"weight must be [{2 * D}, {D}] of {dt} on {dev}")
+    if tuple(weight.shape) != (2 * D, D):
+        raise ValueError(f"weight must be [{2 * D}, {D}], got {tuple(weight.shape)}")
     fused = bool(lib().pk_linear_takes_norm(rows, 2 * D, D, T))
     y = torch.empty((B, T, D), dtype=torch.float32, device=dev)
     a, c = LinearArgs(), ConvArgs()
@@ -815,14 +837,14 @@ def glu_conv(
         _require_device(x, branch)
         x, branch = _aligned_rows(x), _aligned_rows(branch)
         r = torch.empty_like(x)
-        _linear_args(a, _DTYPES[dt], dev, x, rows, weight, bias, y, False)
+        _linear_args(a, dt, dev, x, rows, weight, bias, y, False)
         a.prologue, a.alpha = _lib.PRO_RESIDUAL_NORM, 1.0
         a.branch, a.branch_stride = branch.data_ptr(), D
         a.residual_out, a.residual_out_stride = r.data_ptr(), D
-        a.ln_weight, a.ln_bias, a.ln_eps = _ln(norm)
+        a.ln_weight, a.ln_bias, a.ln_eps = _ln(norm, D, dt, dev)
     else:
         r, h = residual_norm(x, branch, norm.weight, norm.bias, eps=norm.eps, in_place=True)
-        _linear_args(a, _DTYPES[dt], dev, h, rows, weight, bias, y, False)
+        _linear_args(a, dt, dev, h, rows, weight, bias, y, False)
     a.activation, a.out_stride = _lib.ACT_GLU_CONV, D
     c.batch, c.chunk, c.d_model, c.kernel = B, T, D, K
     c.cache, c.num_slots, c.num_layers, c.layer = conv_cache.data_ptr(), S, Ly, int(layer)
@@ -845,13 +867,15 @@ def glu_conv(
 def norm_silu_linear(y: torch.Tensor, norm: torch.nn.LayerNorm, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
     """``linear(SiLU(norm(y)))`` of fp32 y [..., D] in the weight's dtype
     (convolution.py:156-158)."""
+    if y.dtype != torch.float32 or not y.is_contiguous():
+        raise ValueError(f"y must be contiguous float32, got {y.dtype}")
     n, k = weight.shape
     rows, dev, dt = y.numel() // k, y.device, weight.dtype
     out = torch.empty((*y.shape[:-1], n), dtype=dt, device=dev)
     a = LinearArgs()
-    _linear_args(a, _DTYPES[dt], dev, y, rows, weight, bias, out, False)
+    _linear_args(a, dt, dev, y, rows, weight, bias, out, False)
     a.prologue = _lib.PRO_NORM_SILU
-    a.ln_weight, a.ln_bias, a.ln_eps = _ln(norm)
+    a.ln_weight, a.ln_bias, a.ln_eps = _ln(norm, k, dt, dev)
     if not lib().pk_linear_takes_norm(rows, n, k, 0):
         h = torch.empty((rows, k), dtype=dt, device=dev)
         a.residual_out, a.residual_out_stride = h.data_ptr(), k
@@ -867,9 +891,8 @@ def feed_forward(x: torch.Tensor, w1: torch.Tensor, b1: torch.Tensor | None, w2:
     h = torch.empty((rows, w1.shape[0]), dtype=x.dtype, device=x.device)
     out = torch.empty((*x.shape[:-1], w2.shape[0]), dtype=x.dtype, device=x.device)
     a = (LinearArgs * 2)()
-    code = _DTYPES[x.dtype]
-    _linear_args(a[0], code, x.device, x, rows, w1, b1, h, True)
-    _linear_args(a[1], code, x.device, h, rows, w2, b2, out, False)
+    _linear_args(a[0], x.dtype, x.device, x, rows, w1, b1, h, True)
+    _linear_args(a[1], x.dtype, x.device, h, rows, w2, b2, out, False)
     check(lib().pk_linear(a, 2, _stream(x.device)), "pk_linear")
     return out
 

@@ -110,3 +110,52 @@ def test_glu_conv_applies_looks_at_the_depthwise_parameters():
     assert not applies(bias=nn.Parameter(torch.zeros(512, device="meta", dtype=torch.float16), requires_grad=False))
     assert not applies(weight=nn.Parameter(_half(512, 1, 9)))  # a gradient is asked for
     assert not applies(bias=nn.Parameter(_half(512)))
+
+
+@pytest.mark.filterwarnings("ignore:Sparse CSR")
+def test_a_parameter_of_another_shape_keeps_torch(no_launch):
+    """What torch's own modules broadcast, refuse or take another way is left to
+    them: biases that are not [n], sparse weights, norms of another width."""
+    w, x = _half(512, 512), _half(2, 2, 512)
+
+    def applies(weight, bias=None):
+        return ops.layer_applies(torch.float16, x.device, 4, weight, bias)
+
+    assert applies(w) and applies(w, _half(512))
+    assert not applies(w, _half(1)) and not applies(w, _half(256)) and not applies(w, _half(1, 512))
+    assert not applies(w.to_sparse_csr()) and not applies(_half(512, 512, 1)) and not applies(_half(512))
+    n = _ln(512)
+    assert ops.norm_applies(n, x)
+    n.weight = nn.Parameter(_half(256), requires_grad=False)
+    assert not ops.norm_applies(n, x)
+    assert not ops.glu_conv_applies(x, _half(1024, 256), None, w, None, nn.Conv1d(512, 512, 9, groups=512).half().requires_grad_(False), _ln(512))
+
+
+def test_products_refuse_operands_that_do_not_fit(no_launch):
+    x, n = _half(2, 2, 512), _ln(512)
+    calls = [
+        lambda: ops.linear(x, _half(512, 1024)),
+        lambda: ops.linear(x, _half(512, 512).bfloat16()),
+        lambda: ops.linear(x, _half(512, 512), _half(256)),
+        lambda: ops.feed_forward(x, _half(1024, 512), None, _half(512, 512), None),
+        lambda: ops.norm_silu_linear(x, n, _half(512, 512), None),
+        lambda: ops.norm_silu_linear(x.float(), _ln(256), _half(512, 512), None),
+        lambda: ops.norm_linear(x, _ln(256), _half(512, 512), None, silu=True),
+    ]
+    for f in calls:
+        with pytest.raises(ValueError):
+            f()
+    with pytest.raises(RuntimeError):  # torch's own
+        ops.norm_linear(x, n, _half(512, 1024), None, silu=True)
+
+
+def test_feed_forward_of_unequal_layers_is_refused_by_torch(monkeypatch):
+    from parakeet_amd.modules.encoder import ConformerFeedForward
+
+    ff = ConformerFeedForward(512, 1024, 0.0).half().eval().requires_grad_(False)
+    ff.linear2 = nn.Linear(2048, 512).half().requires_grad_(False)
+    monkeypatch.setattr(ops, "linear_applies", lambda *a, **k: True)
+    monkeypatch.setattr(ops, "linear", lambda x, w, b, silu=False: torch.nn.functional.silu(torch.nn.functional.linear(x, w, b)))
+    monkeypatch.setattr(ops, "feed_forward", lambda *a: pytest.fail("the launch would read past the hidden rows"))
+    with pytest.raises(RuntimeError):
+        ff(_half(2, 2, 512))
