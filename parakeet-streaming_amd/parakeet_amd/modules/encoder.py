@@ -50,14 +50,27 @@ class ConformerFeedForward(nn.Module):
         self.dropout = nn.Dropout(dropout)
 
     def forward(self, x: Tensor) -> Tensor:
-        # linear1 with its SiLU is one launch where the library takes it
+        if not torch.jit.is_scripting():
+            y = self._launched(x)
+            if y is not None:
+                return y
+        return self.linear2(self.dropout(self.activation(self.linear1(x))))
+
+    def _launched(self, x: Tensor):
+        """The block with linear1 and its SiLU as one launch, or None where the
+        modules have to run (what :func:`ops.linear_applies` and :meth:`_fused`
+        leave to them; a traced stand-in for x touches no parameter here)."""
+        if type(x) not in (Tensor, nn.Parameter) or not self._fused():
+            return None
         l1, l2 = self.linear1, self.linear2
-        if self._fused() and ops.linear_applies(x, l1.weight, l1.bias, silu=True):
-            rows = x.numel() // x.shape[-1]
-            if ops.plain_module(l2, nn.Linear) and l2.weight.shape[1:] == l1.weight.shape[:1] and ops.layer_applies(x.dtype, x.device, rows, l2.weight, l2.bias):
-                return ops.feed_forward(x, l1.weight, l1.bias, l2.weight, l2.bias)
-            return l2(ops.linear(x, l1.weight, l1.bias, silu=True))
-        return l2(self.dropout(self.activation(l1(x))))
+        w1, b1 = l1.weight, l1.bias
+        if not ops.linear_applies(x, w1, b1, silu=True):
+            return None
+        if ops.plain_module(l2, nn.Linear):
+            w2, b2 = l2.weight, l2.bias
+            if w2.shape[1:] == w1.shape[:1] and ops.layer_applies(x.dtype, x.device, x.numel() // x.shape[-1], w2, b2):
+                return ops.feed_forward(x, w1, b1, w2, b2)
+        return l2(ops.linear(x, w1, b1, silu=True))
 
     def _fused(self) -> bool:
         drop = self.dropout

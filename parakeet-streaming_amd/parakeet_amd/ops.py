@@ -585,8 +585,13 @@ def plain_module(m: torch.nn.Module, cls: type) -> bool:
 
 
 def _plain(t: torch.Tensor) -> bool:
-    """Whether ``t`` is a dense tensor whose memory is its value: no subclass."""
-    return type(t) in (torch.Tensor, torch.nn.Parameter) and t.layout == torch.strided
+    """Whether ``t`` is a dense tensor whose memory is its value: no subclass, and
+    not a function transform's stand-in (vmap or grad over the weights)."""
+    return (
+        type(t) in (torch.Tensor, torch.nn.Parameter)
+        and t.layout == torch.strided
+        and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+    )
 
 
 # past this many products torch's library GEMM is at least as fast as pk_linear:
@@ -623,10 +628,10 @@ def layer_applies(dtype: torch.dtype, device: torch.device, rows: int, weight: t
 def linear_applies(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, silu: bool = False) -> bool:
     """Whether :func:`linear` takes this call, and is the faster way to run it;
     otherwise the caller runs torch's own linear, which takes every form."""
-    if x.dtype not in (torch.float16, torch.bfloat16) or x.device.type != "cuda" or x.dim() == 0:
+    if _transformed(x) or x.dtype not in (torch.float16, torch.bfloat16) or x.device.type != "cuda" or x.dim() == 0:
         return False
     k = x.shape[-1]
-    if not _plain(weight) or weight.dim() != 2 or weight.shape[1] != k or (torch.is_grad_enabled() and x.requires_grad) or _transformed(x):
+    if weight.dim() != 2 or weight.shape[1] != k or (torch.is_grad_enabled() and x.requires_grad):
         return False
     return k > 0 and layer_applies(x.dtype, x.device, x.numel() // k, weight, bias, silu)
 

@@ -269,3 +269,24 @@ def test_glu_conv_matches_its_parts(cuda, dtype, B, T, D):
         print(f"  error against float64: fused {e_new:.2e}, parts {e_old:.2e}", flush=True)
         assert e_new <= 1.05 * e_old + 0.1 * eps
         cache = mine
+
+
+@pytest.mark.gpu
+def test_feed_forward_under_transforms_of_its_weights(cuda):
+    """functional_call under vmap and grad over the weights, and a symbolic trace,
+    keep torch's path: 3 fp16 roundings of values below the output's maximum."""
+    from torch.func import functional_call, grad, vmap
+
+    torch.manual_seed(4)
+    with torch.device(cuda):
+        ff = ConformerFeedForward(256, 512, 0.0).half().eval().requires_grad_(False)
+    x = torch.randn(4, 2, 256, device=cuda).half()
+    p = dict(ff.named_parameters())
+    with torch.no_grad():
+        want = ff(x)
+        y = vmap(lambda q: functional_call(ff, q, (x,)))({k: torch.stack([v, v]) for k, v in p.items()})
+        traced = torch.fx.symbolic_trace(ff)(x)
+    bar = 3 * EPS[torch.float16] * float(want.abs().max())
+    assert float((y[1] - want).abs().max()) <= bar and float((traced - want).abs().max()) <= bar
+    g = grad(lambda q: functional_call(ff, q, (x,)).float().square().sum())(p)
+    assert all(v.dtype == torch.float16 and float(v.abs().sum()) > 0 for v in g.values())

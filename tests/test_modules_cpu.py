@@ -176,3 +176,51 @@ def test_stream_tokens_read_like_per_stream_lists():
     assert got.flat().tolist() == sum(want, []) and got.offsets()[-1] == got.total()
     empty = GreedyDecoder._split(tok[:0], cnt[:0], lens[:0], False)
     assert len(empty) == 0 and empty == []
+
+
+# ---------------------------------------------------------------------------
+# ConformerFeedForward under what rewrites or records torch's calls
+
+
+def _ff():
+    from parakeet_amd.modules.encoder import ConformerFeedForward
+
+    torch.manual_seed(3)
+    return ConformerFeedForward(64, 128, 0.0).eval(), torch.randn(2, 3, 64)
+
+
+def test_feed_forward_is_symbolically_traced():
+    ff, x = _ff()
+    g = torch.fx.symbolic_trace(ff)
+    ops = [n.op for n in g.graph.nodes]
+    assert ops == ["placeholder"] + ["call_module"] * 4 + ["output"], g.graph
+    assert torch.equal(g(x), ff(x))
+
+
+def test_feed_forward_is_scripted_traced_and_compiled():
+    ff, x = _ff()
+    want = ff(x)
+    assert torch.equal(torch.jit.script(ff)(x), want)
+    assert torch.equal(torch.jit.trace(ff, x)(x), want)
+    assert torch.equal(torch.compile(ff, backend="eager", fullgraph=True)(x), want)
+
+
+def test_feed_forward_maps_and_differentiates_over_its_weights(monkeypatch):
+    """Under vmap / grad a weight is a stand-in without memory: the launch rule
+    declines it before looking at an address."""
+    from torch.func import functional_call, grad, vmap
+
+    from parakeet_amd import ops
+
+    ff, x = _ff()
+    p = {k: v.detach() for k, v in ff.named_parameters()}
+    # the rule past its device test, as on a HIP device
+    monkeypatch.setattr(ops, "linear_applies", lambda x, w, b, silu=False: ops.layer_applies(x.dtype, x.device, 6, w, b, silu))
+    big = torch.zeros(2, 64, 256)
+    assert vmap(lambda w: torch.tensor(float(ops.layer_applies(w.dtype, w.device, 4, w, None))))(big).sum() == 0
+    assert vmap(lambda b: torch.tensor(float(ops.layer_applies(b.dtype, b.device, 4, big[0], b))))(torch.zeros(2, 64)).sum() == 0
+    stacked = {k: torch.stack([v, v]) for k, v in p.items()}
+    y = vmap(lambda q: functional_call(ff, q, (x,)))(stacked)
+    assert torch.allclose(y[1], ff(x), rtol=0, atol=1e-6)
+    g = grad(lambda q: functional_call(ff, q, (x,)).square().sum())(p)
+    assert all(float(v.abs().sum()) > 0 for v in g.values())
