@@ -554,10 +554,16 @@ def residual_norm2(pend: "Pending", norm2: torch.nn.LayerNorm) -> tuple[torch.Te
     return y, z
 
 
+def _function_modes() -> bool:
+    """Whether a torch-function mode is active that sees a linear layer.  A default
+    device is such a mode too, but one that only fills in factories' devices."""
+    return any(type(m) is not torch.utils._device.DeviceContext for m in torch.overrides._get_current_function_mode_stack())
+
+
 def _transformed(x: torch.Tensor) -> bool:
     """Whether something follows or rewrites the torch calls made on ``x``
     (autocast, tracing, compilation, function transforms, forward-mode
-    derivatives, dispatch modes): a kernel call would pass it by."""
+    derivatives, dispatch and function modes): a kernel call would pass it by."""
     return (
         type(x) not in (torch.Tensor, torch.nn.Parameter)
         or torch.is_autocast_enabled("cuda")
@@ -566,7 +572,7 @@ def _transformed(x: torch.Tensor) -> bool:
         or torch._C._functorch.is_functorch_wrapped_tensor(x)
         or torch.autograd.forward_ad._current_level >= 0
         or torch._C._len_torch_dispatch_stack() > 0
-        or torch._C._len_torch_function_stack() > 0
+        or (torch._C._len_torch_function_stack() > 0 and _function_modes())
     )
 
 

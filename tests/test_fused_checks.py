@@ -159,3 +159,25 @@ def test_feed_forward_of_unequal_layers_is_refused_by_torch(monkeypatch):
     monkeypatch.setattr(ops, "feed_forward", lambda *a: pytest.fail("the launch would read past the hidden rows"))
     with pytest.raises(RuntimeError):
         ff(_half(2, 2, 512))
+
+
+def test_a_default_device_is_not_a_transform():
+    from torch.overrides import TorchFunctionMode
+
+    class Sees(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    x = _half(2, 512)
+    assert not ops._transformed(x)
+    with torch.device("cpu"):
+        assert not ops._transformed(x)
+        with Sees():
+            assert ops._transformed(x)
+    with Sees(), torch.device("cpu"):
+        assert ops._transformed(x)
+    torch.set_default_device("cpu")
+    try:
+        assert not ops._transformed(x)
+    finally:
+        torch.set_default_device(None)
