@@ -366,7 +366,11 @@ class ModelCache:
     def takes_glu_conv(self, x: Tensor) -> bool:
         """Whether :meth:`glu_conv` updates this conv state for x [B, T, D]: the 8
         rows of 9 taps, of x's width and dtype, on its device (any other state goes
-        to :meth:`conv_step`, which takes it or says what is wrong with it)."""
+        to :meth:`conv_step`, which takes it or says what is wrong with it).  A
+        subclass or object with conv methods of its own has them called."""
+        for name in ("conv_ref", "conv_step", "update_conv_cache"):
+            if name in self.__dict__ or getattr(type(self), name) is not getattr(ModelCache, name):
+                return False
         f = self.conv_frames
         return f.dtype == x.dtype and f.device == x.device and f.is_contiguous() and tuple(f.shape[2:]) == (8, x.shape[-1])
 

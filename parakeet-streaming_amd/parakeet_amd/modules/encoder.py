@@ -194,7 +194,7 @@ class ConformerLayer(nn.Module):
         attn, conv = self.self_attn, self.conv
         return (
             isinstance(cache, ModelCache)
-            and "residual_norm" not in self.__dict__
+            and self.residual_norm is ConformerLayer.residual_norm
             and x.is_contiguous()
             and ops.plain_module(attn, ConformerAttention)
             and ops.plain_module(attn.qkv, nn.Linear)
@@ -230,7 +230,8 @@ class ConformerLayer(nn.Module):
             c = ops.norm_silu_linear(y, bn, w2, p2.bias)
         else:
             r, h = ops.norm_linear(r, self.norm_conv, w1, p1.bias, branch=a, in_place=True)
-            c, _ = conv.after_pointwise1(h, pad_mask=pad_mask, cache=cache.conv_ref(self.layer_idx))
+            c, state = conv.after_pointwise1(h, pad_mask=pad_mask, cache=cache.conv_ref(self.layer_idx))
+            cache.update_conv_cache(self.layer_idx, state)
         r, h = ops.norm_linear(r, self.norm_feed_forward2, ff2.linear1.weight, ff2.linear1.bias, branch=c, silu=True, in_place=True)
         return ops.Pending(r, ops.module_linear(h, ff2.linear2), self.norm_out, 0.5)
 

@@ -91,8 +91,9 @@ def test_glu_conv_refuses_a_state_that_does_not_fit(no_launch, monkeypatch, what
 def test_conv_state_of_another_shape_takes_the_conv_step(shape, dtype, takes):
     from parakeet_amd.modules.cache import ModelCache
 
-    cache = types.SimpleNamespace(conv_frames=torch.zeros(shape, dtype=dtype))
-    assert ModelCache.takes_glu_conv(cache, _half(2, 2, 512)) is takes
+    cache = object.__new__(ModelCache)
+    cache.conv_frames = torch.zeros(shape, dtype=dtype)
+    assert cache.takes_glu_conv(_half(2, 2, 512)) is takes
 
 
 def test_glu_conv_applies_looks_at_the_depthwise_parameters():
@@ -181,3 +182,55 @@ def test_a_default_device_is_not_a_transform():
         assert not ops._transformed(x)
     finally:
         torch.set_default_device(None)
+
+
+def test_own_conv_methods_of_a_cache_are_called(monkeypatch):
+    """A cache that keeps its convolution state another way: the layer's fused step
+    takes its conv_ref and hands the new state to its update_conv_cache."""
+    from parakeet_amd.modules.cache import ModelCache
+    from parakeet_amd.modules.encoder import ConformerLayer
+
+    class Dense(ModelCache):
+        def conv_ref(self, layer):
+            return ("state of", layer)
+
+        def update_conv_cache(self, layer, state):
+            self.new = (layer, state)
+
+    cache = object.__new__(Dense)
+    cache.conv_frames = _half(2, 1, 8, 512)
+    x = _half(2, 2, 512)
+    assert not cache.takes_glu_conv(x)
+    plain = object.__new__(ModelCache)
+    plain.conv_frames = cache.conv_frames
+    assert plain.takes_glu_conv(x)
+    plain.conv_step = lambda *a: None
+    assert not plain.takes_glu_conv(x)
+
+    layer = ConformerLayer(1, 512, 1024, 8, 0.0, 9, False).half().eval().requires_grad_(False)
+    monkeypatch.setattr(ops, "norm_linear", lambda x, norm, w, b, **kw: (x, _half(2, 2, w.shape[0])))
+    monkeypatch.setattr(ops, "glu_conv_applies", lambda *a: True)
+    monkeypatch.setattr(layer.self_attn, "attend", lambda *a: x)
+    got = []
+    monkeypatch.setattr(layer.conv, "after_pointwise1", lambda h, pad_mask, cache: (got.append(cache) or x, "next"))
+    layer.fused_step(x, None, None, None, cache)
+    assert got == [("state of", 1)] and cache.new == (1, "next")
+
+
+def test_a_layer_with_its_own_residual_norm_runs_its_modules(monkeypatch):
+    from parakeet_amd.modules.cache import ModelCache
+    from parakeet_amd.modules.encoder import ConformerLayer
+
+    class Own(ConformerLayer):
+        @staticmethod
+        def residual_norm(residual, branch, norm, alpha, in_place=False):
+            return residual, norm(residual)
+
+    monkeypatch.setattr(ops, "linear_applies", lambda *a, **k: True)
+    x, cache = _half(2, 2, 512), object.__new__(ModelCache)
+    make = lambda cls: cls(0, 512, 1024, 8, 0.0, 9, False).half().eval().requires_grad_(False)
+    assert make(ConformerLayer).fuses(x, cache)
+    assert not make(Own).fuses(x, cache)
+    layer = make(ConformerLayer)
+    layer.residual_norm = Own.residual_norm
+    assert not layer.fuses(x, cache)
