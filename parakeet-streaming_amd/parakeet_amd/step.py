@@ -89,7 +89,6 @@ class AttentionStep:
         self._stage_used = [False] * depth
         self._stage_i = 0
         self._args = (AttnArgs * Ly)(*[self._attn_args(layer, rows_per_lane) for layer in range(Ly)])
-        self._stream = ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
         self.batch = 0
         self.graph: torch.cuda.CUDAGraph | None = None
 
@@ -177,12 +176,14 @@ class AttentionStep:
         """All layers' fused append + attention for the batch opened last, sized
         to it: one launch over every layer (their inputs and pages are each
         layer's own), or with ``events``, optional per-layer (start, stop) pairs
-        timing each kernel, one per layer."""
+        timing each kernel, one per layer.  On the current stream, as the upload of
+        :meth:`open`: steps under different streams are ordered by the caller, as
+        any work on the same tensors."""
         B = self.batch
         if B == 0:
             return
         self._set_args(B, None, events)
-        check(lib().pk_paged_relpos_attn_layers(self._args, len(self._args), self._stream), "pk_paged_relpos_attn_layers")
+        check(lib().pk_paged_relpos_attn_layers(self._args, len(self._args), ops._stream(self.device)), "pk_paged_relpos_attn_layers")
 
     def _set_args(self, batch: int, live: int | None, events=None) -> None:
         for layer, a in enumerate(self._args):
@@ -198,9 +199,8 @@ class AttentionStep:
         side = torch.cuda.Stream(self.device)
         side.wait_stream(torch.cuda.current_stream(self.device))
         with torch.cuda.graph(g, stream=side):
-            stream = ctypes.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)
             self._set_args(self.num_slots, self.live.data_ptr())
-            check(L.pk_paged_relpos_attn_layers(self._args, len(self._args), stream), "pk_paged_relpos_attn_layers")
+            check(L.pk_paged_relpos_attn_layers(self._args, len(self._args), ops._stream(self.device)), "pk_paged_relpos_attn_layers")
         torch.cuda.current_stream(self.device).wait_stream(side)
         self.graph = g
 

@@ -163,3 +163,54 @@ def test_layers_in_one_launch_match_layer_by_layer(cuda, dtype, streams, layers,
             assert torch.equal(steps[0].k_pages, other.k_pages) and torch.equal(steps[0].v_pages, other.v_pages)
             for a, b in zip(steps[0].out, other.out):
                 assert torch.equal(a[:n], b[:n])
+
+
+def test_step_launches_on_the_stream_of_the_call(monkeypatch):
+    """The upload of a step's rows and the caller's projections are on the stream
+    that is current at the call; so is the launch that reads them, whichever stream
+    was current when the step was built (CPU: the library replaced)."""
+    import types
+
+    import parakeet_amd.step as S
+
+    seen, current = [], ["at construction"]
+    monkeypatch.setattr(S, "lib", lambda: types.SimpleNamespace(pk_paged_relpos_attn_layers=lambda a, n, s: seen.append((n, s)) or 0))
+    monkeypatch.setattr(ops, "_stream", lambda dev: (dev, current[0]))
+    st = object.__new__(AttentionStep)
+    st.device, st.batch, st._args, st._stream = "dev", 2, (S.AttnArgs * 3)(), ("dev", current[0])
+    st.run()
+    current[0] = "another"
+    st.run()
+    assert seen == [(3, ("dev", "at construction")), (3, ("dev", "another"))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("graph", [False, True])
+def test_steps_under_another_stream(cuda, graph):
+    """Built on the default stream and stepped under another one, behind work that
+    writes the projections there: outputs and pages as a step on one stream alone."""
+    shape = synth.Shape("streams", 3, 512, 8, left=20, dtype=torch.float16)
+    B, T, D = 5, shape.chunk, 512
+    g = torch.Generator(device="cuda").manual_seed(9)
+    pos = torch.randn(2 * shape.window - 1, D, generator=g, device=cuda).half()
+    bias = [torch.randn(8, 64, generator=g, device=cuda).half() for _ in range(3)]
+    x = torch.randn(14, 3, B, T, 3 * D, generator=g, device=cuda).half()
+    big = torch.randn(4096, 4096, generator=g, device=cuda).half()
+    out = []
+    for stream in (torch.cuda.current_stream(), torch.cuda.Stream()):
+        qkv = [torch.zeros(B, T, 3 * D, dtype=torch.float16, device=cuda) for _ in range(3)]
+        st = AttentionStep(shape, B, torch.device("cuda", 0), qkv, pos, bias, bias)
+        st.k_pages.zero_()
+        st.v_pages.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            for i in range(len(x)):
+                for _ in range(4):
+                    big @ big  # the copies below are still to come when the step is called
+                for layer in range(3):
+                    qkv[layer].copy_(x[i, layer])
+                st.step(np.arange(B), graph=graph)
+        torch.cuda.synchronize()
+        out.append([o.clone() for o in st.out] + [st.k_pages, st.v_pages])
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
