@@ -102,7 +102,7 @@ extern "C" int pk_fe_plan(pk_fe_plan_args* a) {
       a->out_row[i] = a->out_rows;
       a->out_rows += out;
     }
-    a->max_new = std::max(a->max_new, a->n_new[i]);
+    a->max_new = i == 0 ? a->n_new[0] : std::max(a->max_new, a->n_new[i]);  // negative: pk_fe_step refuses it
     a->max_frames = std::max(a->max_frames, t.n_frames);
     a->max_out = std::max(a->max_out, out);
     a->total[s] = t.total;

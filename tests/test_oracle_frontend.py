@@ -393,3 +393,17 @@ def test_native_plan_matches_stream_counters():
             z = np.array(bad, dtype=np.int64)
             with pytest.raises(ValueError, match="distinct and in range"):
                 PreEncoder._plan(pre, z, 0 * z + 160, z < -9, np.zeros(128, dtype=np.uint8))
+
+
+def test_native_plan_passes_a_negative_push_on():
+    """A negative sample count reaches pk_fe_step, which refuses it, as the largest
+    count of the batch (CPU: the plan alone)."""
+    import types
+
+    from parakeet_amd.modules.frontend import PreEncoder, StreamCounters
+
+    pre = types.SimpleNamespace(counters=StreamCounters(2, 512, 400, 160), num_slots=2, noise_id=np.zeros(2, np.uint32))
+    for n, largest in (([-5], -5), ([-5, -3], -3), ([-5, 0], 0), ([-5, 7], 7)):
+        slots = np.arange(len(n), dtype=np.int64)
+        args, _ = PreEncoder._plan(pre, slots, np.array(n, np.int64), slots < 0, np.zeros(128, dtype=np.uint8))
+        assert args.max_new == largest
