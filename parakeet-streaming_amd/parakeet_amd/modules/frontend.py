@@ -263,7 +263,7 @@ class ConvSubsampling(nn.Module):
     def conv_weights(self) -> dict:
         w = {}
         for i, m in enumerate(self.conv):
-            if isinstance(m, nn.Conv2d):
+            if i in (0, 2, 3, 5, 6):  # the convolutions, of whatever class; the rest are activations
                 w[f"conv.{i}.weight"], w[f"conv.{i}.bias"] = m.weight, m.bias
         return w
 

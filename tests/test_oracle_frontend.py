@@ -407,3 +407,23 @@ def test_native_plan_passes_a_negative_push_on():
         slots = np.arange(len(n), dtype=np.int64)
         args, _ = PreEncoder._plan(pre, slots, np.array(n, np.int64), slots < 0, np.zeros(128, dtype=np.uint8))
         assert args.max_new == largest
+
+
+def test_conv_weights_of_replaced_convolutions():
+    import torch
+    from torch import nn
+
+    from parakeet_amd.modules.frontend import ConvSubsampling
+
+    class Conv(nn.Module):  # no nn.Conv2d, with its parameters
+        def __init__(self, m):
+            super().__init__()
+            self.weight, self.bias = m.weight, m.bias
+
+    sub = ConvSubsampling(64, 16, 80, 8)
+    want = {k: v.clone() for k, v in sub.conv_weights().items()}
+    assert len(want) == 10
+    for i in (0, 3):
+        sub.conv[i] = Conv(sub.conv[i])
+    got = sub.conv_weights()
+    assert list(got) == list(want) and all(torch.equal(got[k], v) for k, v in want.items())
