@@ -210,8 +210,8 @@ typedef struct pk_attn_args {
 } pk_attn_args;
 int pk_paged_relpos_attn(const pk_attn_args* args, void* stream);
 /* pk_paged_relpos_attn for `count` layers whose calls are independent of each
- * other (none reads or appends what another writes; different layers of a pool),
- * in one launch where they differ in their tensors and layer alone and no call
+ * other (none reads, appends or writes what another writes; different layers of a
+ * pool), in one launch where they differ in their tensors and layer alone and no call
  * asks for events, else one by one.  One dtype and device.  The same outputs. */
 int pk_paged_relpos_attn_layers(const pk_attn_args* args, int32_t count, void* stream);
 
@@ -322,9 +322,10 @@ int pk_conv_step(const pk_conv_args* args, void* stream);
  * norm_self_att, norm_conv, norm_feed_forward2 and norm_out that read them.
  * residual, branch, residual_out, norm_out: [rows][d_model] of `dtype` with row
  * strides in elements (channels contiguous, 16-byte aligned rows);
- * residual_out may be residual (updated in place), or with ln2_weight NULL, where
- * nothing reads it; norm_out may be branch; no other overlap.  ln_weight, ln_bias: [d_model].  d_model a multiple of 8
- * (fp16/bf16) or 4 (fp32), at most 4096 (fp16/bf16) or 2048 (fp32).
+ * residual_out may be residual (updated in place), or NULL where ln2_weight is
+ * set and nothing reads the update; norm_out may be branch; no other overlap.
+ * ln_weight, ln_bias: [d_model].  d_model a multiple of 8 (fp16/bf16) or 4 (fp32),
+ * at most 4096 (fp16/bf16) or 2048 (fp32).
  */
 typedef struct pk_resnorm_args {
   int32_t dtype;

@@ -26,7 +26,6 @@ import math
 import numpy as np
 import torch
 from torch import Tensor, nn
-from torch.nn import functional as F
 
 from .. import ops
 from .._lib import PK_ERR_EXHAUSTED, PK_ERR_STATE, FePlanArgs, check, last_error, lib
@@ -323,7 +322,8 @@ class StreamCounters:
         self.has_cache[slot] = False
 
     def plan(self, slots: np.ndarray, n_new: np.ndarray, final: np.ndarray):
-        """Advances the counters of ``slots`` by one push each.  Returns
+        """Advances the counters of ``slots`` by one push each, in numpy: the form
+        that pk_fe_plan, which a step runs, is tested against.  Returns
         (samples before the push, first frame, frame count, cached frames in the
         window, window rows, dropped outputs, kept outputs, emitted?) per stream."""
         hop, pad = self.hop, self.n_fft // 2
@@ -468,7 +468,7 @@ class PreEncoder:
         return a, out
 
     def _features(self, slots, samples, n_new, final):
-        """The feature half of a step: the push's plan as StreamCounters.plan
+        """:meth:`_push` for tests that look at its plan: as StreamCounters.plan
         returns it, the streams with kept outputs and their first rows."""
         plan, (start, n_frames, n_out, out_row) = self._push(slots, samples, n_new, final)
         rec = self._stage.last().numpy()
