@@ -2168,16 +2168,14 @@ int attn_build(const pk_attn_args* a, AttnK<ST>& k) {
   return PK_OK;
 }
 
-// ls: the layers of a launch over several (else nullptr); k is the first's.  Takes
-// a launch over several only with a matrix-core kernel and one query pair: else
-// PK_ERR_UNSUPPORTED, and the caller launches them one by one.
+// the kernel of a call that attn_build accepts (kAttnNone: rows_per_lane asks for
+// a matrix-core kernel that does not take it)
+enum AttnKernel { kAttnChunk, kAttnPair, kAttnVector, kAttnNone };
 template <typename ST>
-int attn_dispatch(const pk_attn_args* a, AttnK<ST>& k, const LayerSet<ST>* ls, hipStream_t s) {
-  constexpr int VEC = Tr<ST>::VEC;
-  const char* what = "pk_paged_relpos_attn";
-  const int DK = a->head_dim, D = a->num_heads * DK, Lk = a->left + a->chunk;
-  const bool need_pages = a->left > 0 || a->append;
+AttnKernel attn_kernel(const pk_attn_args* a, const AttnK<ST>& k) {
   if constexpr (!std::is_same<ST, float>::value) {
+    const int D = a->num_heads * a->head_dim, Lk = a->left + a->chunk;
+    const bool need_pages = a->left > 0 || a->append;
     // the matrix-core kernel addresses rows through buffer resources: row
     // strides up to kMaxBufferStride bytes and fewer than 2^32 pool rows
     const int64_t es = (int64_t)sizeof(ST);
@@ -2195,26 +2193,48 @@ int attn_dispatch(const pk_attn_args* a, AttnK<ST>& k, const LayerSet<ST>* ls, h
     // -2 asks for it at any chunk it supports, -1 for the two-query kernel
     const bool chunk_ok = mfma_ok && a->chunk <= kChunkMaxT && Lk <= kChunkMaxWindow &&
                           row_bytes(a->query_stride_t) <= kMaxBufferStride;
-    if (a->rows_per_lane == -2) {
-      if (!chunk_ok)
-        return fail(PK_ERR_UNSUPPORTED, "%s: the whole-chunk kernel needs chunk <= %d, window <= %d, one position table",
-                    what, kChunkMaxT, kChunkMaxWindow);
+    if (a->rows_per_lane == -2) return chunk_ok ? kAttnChunk : kAttnNone;
+    if (a->rows_per_lane == 0 && chunk_ok && a->chunk >= 3) return kAttnChunk;
+    if ((a->rows_per_lane == 0 || a->rows_per_lane == -1) && mfma_ok && a->chunk <= 16) return kAttnPair;
+    if (a->rows_per_lane < 0) return kAttnNone;
+  }
+  return kAttnVector;
+}
+
+// Whether a launch over several layers takes the call: the matrix-core kernels,
+// the two-query one with a single query pair (grid z is then free), with the
+// streaming mask from the stream state and no event to record.
+template <typename ST>
+bool attn_groups(const pk_attn_args* a, const AttnK<ST>& k) {
+  if (!k.st_proc || k.mask || !k.pg.rows || a->start_event || a->stop_event || a->rows_per_lane != 0) return false;
+  const AttnKernel kind = attn_kernel(a, k);
+  return kind == kAttnChunk || (kind == kAttnPair && a->chunk <= 2);
+}
+
+// ls: the layers of a launch over several that attn_groups accepts (else nullptr);
+// k is the first's.
+template <typename ST>
+int attn_dispatch(const pk_attn_args* a, AttnK<ST>& k, const LayerSet<ST>* ls, hipStream_t s) {
+  constexpr int VEC = Tr<ST>::VEC;
+  const char* what = "pk_paged_relpos_attn";
+  const int DK = a->head_dim, Lk = a->left + a->chunk;
+  const AttnKernel kind = attn_kernel(a, k);
+  if (kind == kAttnNone && a->rows_per_lane == -2)
+    return fail(PK_ERR_UNSUPPORTED, "%s: the whole-chunk kernel needs chunk <= %d, window <= %d, one position table", what,
+                kChunkMaxT, kChunkMaxWindow);
+  if (kind == kAttnNone)
+    return fail(PK_ERR_UNSUPPORTED, "%s: rows_per_lane %d asks for a matrix-core kernel this call cannot take", what,
+                a->rows_per_lane);
+  if constexpr (!std::is_same<ST, float>::value) {
+    if (kind == kAttnChunk) {
       if (DK == 64) return launch_attn_chunk<ST, 64>(a, k, ls, s);
       return launch_attn_chunk<ST, 128>(a, k, ls, s);
     }
-    if (a->rows_per_lane == 0 && chunk_ok && a->chunk >= 3) {
-      if (DK == 64) return launch_attn_chunk<ST, 64>(a, k, ls, s);
-      return launch_attn_chunk<ST, 128>(a, k, ls, s);
-    }
-    if ((a->rows_per_lane == 0 || a->rows_per_lane == -1) && mfma_ok && a->chunk <= 16 && !(ls && a->chunk > 2)) {
+    if (kind == kAttnPair) {
       if (DK == 64) return launch_attn_mfma<ST, 64>(a, k, ls, s);
       return launch_attn_mfma<ST, 128>(a, k, ls, s);
     }
-    if (a->rows_per_lane < 0)
-      return fail(PK_ERR_UNSUPPORTED, "%s: rows_per_lane %d asks for a matrix-core kernel this call cannot take", what,
-                  a->rows_per_lane);
   }
-  if (ls) return PK_ERR_UNSUPPORTED;
   const int G = DK / VEC;
   const int rlw = 64 / G;
   const int TQ = pick_tq(a->chunk);
@@ -2242,7 +2262,9 @@ int attn_typed(const pk_attn_args* a, hipStream_t s) {
 }
 
 // `n` layers' calls: launches over up to kMaxLaunchLayers of them where they differ
-// in their tensors and layer alone, else one by one.  One grid over the layers has
+// in their tensors and layer alone and attn_groups takes them, else one by one; each
+// call is looked at once (24 fp32 layers 68 us of host time a step; with the rest of
+// the list compared again for every layer that no launch takes with others, 88).  One grid over the layers has
 // no launch gap and no idle tail between them: 24 layers x 230 streams of the large
 // model 380 -> 298 us (2 frames) and 547 -> 428 us (14 frames); for few streams
 // the launches themselves were the time (17 layers of a few streams 101 -> 36 us).
@@ -2256,37 +2278,37 @@ int attn_layers_typed(const pk_attn_args* a, int n, hipStream_t s) {
       ++i;
       continue;
     }
+    if (!attn_groups(a + i, k)) {
+      rc = attn_dispatch<ST>(a + i, k, nullptr, s);
+      if (rc != PK_OK) return rc;
+      ++i;
+      continue;
+    }
     LayerSet<ST> ls;
     ls.n = 0;
-    const bool plain = k.st_proc && !k.mask && k.pg.rows && !a[i].start_event && !a[i].stop_event && a[i].rows_per_lane == 0;
-    for (int j = i; plain && j < n && ls.n < kMaxLaunchLayers; ++j) {
-      // what may differ, taken from the first; layers ascend, so no two share pages
-      pk_attn_args c = a[j];
-      if (j > i && c.layer <= a[j - 1].layer) break;
-      c.layer = a[i].layer;
-      c.query = a[i].query;
-      c.key = a[i].key;
-      c.value = a[i].value;
-      c.bias_u = a[i].bias_u;
-      c.bias_v = a[i].bias_v;
-      c.out = a[i].out;
-      if (std::memcmp(&c, a + i, sizeof(c)) != 0) break;
-      AttnK<ST> kj{};
-      rc = attn_build(a + j, kj);
-      if (rc != PK_OK) return rc;
+    AttnK<ST> kj = k;
+    for (int j = i; j < n && ls.n < kMaxLaunchLayers; ++j) {
+      if (j > i) {
+        // what may differ, taken from the first; layers ascend, so no two share pages
+        pk_attn_args c = a[j];
+        if (c.layer <= a[j - 1].layer) break;
+        c.layer = a[i].layer;
+        c.query = a[i].query;
+        c.key = a[i].key;
+        c.value = a[i].value;
+        c.bias_u = a[i].bias_u;
+        c.bias_v = a[i].bias_v;
+        c.out = a[i].out;
+        if (std::memcmp(&c, a + i, sizeof(c)) != 0) break;
+        kj = AttnK<ST>{};
+        rc = attn_build(a + j, kj);
+        if (rc != PK_OK) return rc;
+      }
       ls.l[ls.n++] = AttnLayer<ST>{kj.q, kj.kn, kj.vn, kj.bu, kj.bv, kj.kp, kj.vp, kj.out};
     }
-    if (ls.n > 1) {
-      rc = attn_dispatch<ST>(a + i, k, &ls, s);
-      if (rc == PK_OK) {
-        i += ls.n;
-        continue;
-      }
-      if (rc != PK_ERR_UNSUPPORTED) return rc;
-    }
-    rc = attn_dispatch<ST>(a + i, k, nullptr, s);
+    rc = attn_dispatch<ST>(a + i, k, ls.n > 1 ? &ls : nullptr, s);
     if (rc != PK_OK) return rc;
-    ++i;
+    i += ls.n;
   }
   return PK_OK;
 }

@@ -214,3 +214,12 @@ def test_steps_under_another_stream(cuda, graph):
         out.append([o.clone() for o in st.out] + [st.k_pages, st.v_pages])
     for a, b in zip(*out):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("right", [14, 15])
+def test_layers_without_a_common_launch(cuda, dtype, right):
+    """Chunks of 15 and 16 frames have no several-layer form: the one call launches
+    its layers one by one, with the same bits."""
+    test_layers_in_one_launch_match_layer_by_layer(cuda, dtype, 5, 3, 512, right)
