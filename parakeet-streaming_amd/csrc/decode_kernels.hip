@@ -77,7 +77,9 @@ constexpr int kPredWaves = 2;          // pred_proj columns per workgroup: 16 a 
 // fp16, tile by tile and compact, at 1.7 | 0.3 | 0.02 tokens a frame: 256 streams 309
 // 315 | 276 291 | 217 228, 512 streams 431 356 | 377 332 | 299 314, 1000 streams 616
 // 473 | 548 364 | 400 345; the large model's 14 frames at 512 streams 3627 2540 | 2990
-// 2350 | 2039 2120
+// 2350 | 2039 2120.  The loss is that of 0.02-0.04 tokens a frame alone, where almost
+// every iteration has a token in few tiles (512 to 640 streams 4-6%, 768 -3%): at 0.1
+// tokens 512 streams take 322 313, at 0.001 222 197
 constexpr int kCompactMinBatch = 512;
 constexpr int kMaxDim = 1024;  // hidden / joint sizes held in LDS
 // per-stream words of the step workspace: flag, token, emitted count, pad

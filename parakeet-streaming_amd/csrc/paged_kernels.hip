@@ -2264,10 +2264,11 @@ int attn_typed(const pk_attn_args* a, hipStream_t s) {
 // `n` layers' calls: launches over up to kMaxLaunchLayers of them where they differ
 // in their tensors and layer alone and attn_groups takes them, else one by one; each
 // call is looked at once (24 fp32 layers 68 us of host time a step; with the rest of
-// the list compared again for every layer that no launch takes with others, 88).  One grid over the layers has
-// no launch gap and no idle tail between them: 24 layers x 230 streams of the large
-// model 380 -> 298 us (2 frames) and 547 -> 428 us (14 frames); for few streams
-// the launches themselves were the time (17 layers of a few streams 101 -> 36 us).
+// the list compared again for every layer that no launch takes with others, 88).
+// One grid over the layers has no launch gap and no idle tail between them: 24 layers
+// x 230 streams of the large model 380 -> 298 us (2 frames) and 547 -> 428 us (14
+// frames); for few streams the launches themselves were the time (17 layers of a few
+// streams 101 -> 36 us).
 template <typename ST>
 int attn_layers_typed(const pk_attn_args* a, int n, hipStream_t s) {
   for (int i = 0; i < n;) {
