@@ -726,7 +726,8 @@ dim3 tile_grid(LinK<ST>& k, int bm, int bn) {
   k.mtiles = (k.M + k.rpt - 1) / k.rpt;
   const int nt = k.N / bn;
   k.xm = xcd_split(k.mtiles, nt, bm, bn);
-  if (k.xm > 0 && k.mtiles / k.xm <= 65535) return dim3(8u, (unsigned)(k.mtiles / k.xm), (unsigned)(nt / (8 / k.xm)));
+  if (k.xm > 0 && k.mtiles / k.xm <= 65535 && nt / (8 / k.xm) <= 65535)  // y and z of a grid
+    return dim3(8u, (unsigned)(k.mtiles / k.xm), (unsigned)(nt / (8 / k.xm)));
   k.xm = 0;
   return dim3((unsigned)(k.mtiles * nt));
 }

@@ -290,3 +290,16 @@ def test_feed_forward_under_transforms_of_its_weights(cuda):
     assert float((y[1] - want).abs().max()) <= bar and float((traced - want).abs().max()) <= bar
     g = grad(lambda q: functional_call(ff, q, (x,)).float().square().sum())(p)
     assert all(v.dtype == torch.float16 and float(v.abs().sum()) > 0 for v in g.values())
+
+
+@pytest.mark.gpu
+def test_linear_with_more_column_tiles_than_a_grid_holds(cuda):
+    """8 row tiles by 65,537 column tiles: the block split over the XCDs would be a
+    grid of 8 x 1 x 65,537 (limit 65,535); the linear tile order takes it."""
+    rows, n, k, dtype = 449, 64 * 65537, 256, torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(8)
+    x = torch.randn(rows, k, generator=g, device=cuda).to(dtype)
+    w = torch.randn(n, k, generator=g, device=cuda, dtype=dtype) / 16
+    y = ops.linear(x, w)
+    for c in (slice(0, 128), slice(n // 2, n // 2 + 128), slice(n - 128, n)):
+        _check(y[:, c], x, w[c], None, dtype, False)
