@@ -340,13 +340,17 @@ __device__ static inline int w_row(int nt_i, int n, int N) {
 // Many rows: BM x BN outputs a workgroup, WM x WN x WK waves, both operands
 // staged in LDS BK columns a stage (S stages in flight, buffer loads straight to
 // LDS).  A row's 16-byte chunks are permuted within each 128 bytes by the row's
-// low three bits, so the 16 rows of an operand read fall on distinct banks.
+// low three bits, so the 16 rows of an operand read fall on distinct banks in stages
+// of 64 columns; in longer ones two rows share each bank (40-46% of LDS's active
+// cycles in the counters, 11-13% of the launch's time active).
 // Small tiles split K over the waves (WK): each staged byte is then read from LDS
 // once or twice, and the sum over the waves costs one exchange at the end.
 // Bound by: latency up to about one tile a CU (128 x 512 -> 2048 with SiLU 4.2 us,
-// torch's GEMM and SiLU 10.2); LDS reads on the large forms (128 x 128 tiles take
-// 0.53 us a stage, of which 0.41 remain with the loads left out and 0.27 with the
-// products left out).  An operand read straight from memory (16 rows x 64 bytes
+// torch's GEMM and SiLU 10.2); on the large forms the chain of a stage, its loads and
+// barrier, then operand reads, then products, with two waves a SIMD or fewer to
+// overlap: counters at 840 x 1024 -> 4096 have the matrix cores busy 19% of the time,
+// LDS active 16%, L2 at 7.3 TB/s and the waves waiting 46% of their cycles (3584 rows
+// 29%, 13%, 5.7 and 35%).  An operand read straight from memory (16 rows x 64 bytes
 // an instruction, half of each 128-byte line) moved 37 GB/s a CU against about 100
 // through LDS: 16 rows x 2048 -> 512 6.1 us so, 4.4 staged (torch's GEMM 7.9).
 // 840 x 1024 -> 4096 with SiLU 13.6 us (518 TFLOP/s) against
@@ -745,8 +749,8 @@ int launch_tile(LinK<ST> k, hipStream_t s) {
 // for each further one resident with it (`occ` fit), and again a - 2 for each
 // further round.  Small tiles read more bytes an output but put more CUs on a
 // short launch, and few long stages (up to 512 columns) wait for fewer barriers;
-// the large ones are bound by LDS reads (a 64x32 wave tile reads 6 KB for 8
-// products).  The cheapest by this model is launched; at the measured shapes it
+// the large ones reuse a byte more often (the 64 x 64 form reads 12.9 TB/s from L2 at
+// 840 x 4096 -> 1024, the 128 x 128 form 7.3 at 840 x 1024 -> 4096).  The cheapest by this model is launched; at the measured shapes it
 // is the fastest form or within 6% of it.
 struct Form {
   int bm, bn, kmul, occ;
