@@ -644,11 +644,11 @@ def linear_applies(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | N
 
 def _linear_args(a: LinearArgs, dt: torch.dtype, dev: torch.device, x: torch.Tensor, rows: int, weight, bias, out, silu: bool) -> None:
     n, k = weight.shape
-    if k != x.shape[-1] or weight.dtype != dt or weight.device != dev:
-        raise ValueError(f"weight {tuple(weight.shape)} {weight.dtype} on {weight.device} does not take x "
-                         f"{tuple(x.shape)} of {dt} on {dev}")
-    if bias is not None and (tuple(bias.shape) != (n,) or bias.dtype != dt or bias.device != dev):
-        raise ValueError(f"bias must be [{n}] of {dt} on {dev}")
+    if k != x.shape[-1] or weight.dtype != dt or weight.device != dev or weight.stride(1) != 1:
+        raise ValueError(f"weight {tuple(weight.shape)} {weight.dtype} on {weight.device}, strides {weight.stride()}, does not "
+                         f"take x {tuple(x.shape)} of {dt} on {dev}")
+    if bias is not None and (tuple(bias.shape) != (n,) or bias.dtype != dt or bias.device != dev or not bias.is_contiguous()):
+        raise ValueError(f"bias must be contiguous [{n}] of {dt} on {dev}")
     a.dtype, a.device = _DTYPES[dt], dev.index or 0
     a.rows, a.n, a.k = rows, n, k
     a.activation = _lib.ACT_SILU if silu else _lib.ACT_NONE

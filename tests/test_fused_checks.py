@@ -138,6 +138,9 @@ def test_products_refuse_operands_that_do_not_fit(no_launch):
         lambda: ops.linear(x, _half(512, 1024)),
         lambda: ops.linear(x, _half(512, 512).bfloat16()),
         lambda: ops.linear(x, _half(512, 512), _half(256)),
+        lambda: ops.linear(x, _half(512, 1024)[:, ::2]),
+        lambda: ops.linear(x, _half(512, 512).t()),
+        lambda: ops.linear(x, _half(512, 512), _half(1024)[::2]),
         lambda: ops.feed_forward(x, _half(1024, 512), None, _half(512, 512), None),
         lambda: ops.norm_silu_linear(x, n, _half(512, 512), None),
         lambda: ops.norm_silu_linear(x.float(), _ln(256), _half(512, 512), None),
