@@ -303,3 +303,51 @@ def test_linear_with_more_column_tiles_than_a_grid_holds(cuda):
     y = ops.linear(x, w)
     for c in (slice(0, 128), slice(n // 2, n // 2 + 128), slice(n - 128, n)):
         _check(y[:, c], x, w[c], None, dtype, False)
+
+
+@pytest.mark.gpu
+def test_encoder_refuses_what_its_launches_do_not_fit(cuda):
+    """A hooked linear2 or linear_out that returns another dtype or shape, and a
+    cache built for another kernel size: the errors of the separate launches,
+    raised on the host; the encoder steps on afterwards."""
+    from parakeet_amd.modules.encoder import ConformerEncoder
+
+    torch.manual_seed(6)
+
+    def build(kernel):
+        with torch.device(cuda):
+            enc = ConformerEncoder(
+                feat_in=80, hidden_size=512, ff_expansion_factor=4, num_layers=2, num_heads=8, subsampling_factor=8,
+                pos_emb_max_len=500, conv_kernel_size=kernel, att_context_size=[70, 1], subsampling_conv_channels=256, use_bias=False,
+            )
+        for layer in enc.layers:
+            layer.self_attn.pos_bias_u.data.normal_(std=0.02)
+            layer.self_attn.pos_bias_v.data.normal_(std=0.02)
+        return enc.half().eval().requires_grad_(False)
+
+    enc, B = build(9), 3
+    length = torch.full((B,), 2, dtype=torch.int64, device=cuda)
+    x = torch.randn(B, 2, 512, device=cuda).half()
+
+    def state(of):
+        return of.init_streaming_state(batch_size=B, device=cuda, dtype=torch.float16)
+
+    with torch.no_grad():
+        assert enc.layers[0].fuses(x, state(enc).cache)
+        want, _ = enc(x, state(enc), length=length)
+        for module in (enc.layers[0].feed_forward1.linear2, enc.layers[1].self_attn.linear_out, enc.layers[1].feed_forward2.linear2):
+            for change in (lambda o: o.float(), lambda o: o[:1], lambda o: o.mean(1, keepdim=True)):
+                hook = module.register_forward_hook(lambda m, i, o: change(o))
+                with pytest.raises(ValueError, match="must match"):
+                    enc(x, state(enc), length=length)
+                hook.remove()
+        for kernel in (5, 15):
+            with pytest.raises(ValueError, match="dw_weight"):
+                enc(x, state(build(kernel)), length=length)
+        got, _ = enc(x, state(enc), length=length)
+        assert torch.equal(got, want)
+        torch.set_default_device(cuda)
+        try:
+            assert enc.layers[0].fuses(x, state(enc).cache)
+        finally:
+            torch.set_default_device(None)
