@@ -60,22 +60,22 @@ class ConformerFeedForward(nn.Module):
         """The block with linear1 and its SiLU as one launch, or None where the
         modules have to run (what :func:`ops.linear_applies` and :meth:`_fused`
         leave to them; a traced stand-in for x touches no parameter here)."""
-        if type(x) not in (Tensor, nn.Parameter) or not self._fused():
-            return None
         l1, l2 = self.linear1, self.linear2
+        if type(x) not in (Tensor, nn.Parameter) or not self._fused(l1):
+            return None
         w1, b1 = l1.weight, l1.bias
         if not ops.linear_applies(x, w1, b1, silu=True):
             return None
         if ops.plain_module(l2, nn.Linear):
             w2, b2 = l2.weight, l2.bias
             if w2.shape[1:] == w1.shape[:1] and ops.layer_applies(x.dtype, x.device, x.numel() // x.shape[-1], w2, b2):
-                return ops.feed_forward(x, w1, b1, w2, b2)
+                return ops._feed_forward(x, w1, b1, w2, b2)
         return l2(ops.linear(x, w1, b1, silu=True))
 
-    def _fused(self) -> bool:
+    def _fused(self, linear1: nn.Module | None = None) -> bool:
         drop = self.dropout
         return (
-            ops.plain_module(self.linear1, nn.Linear)
+            ops.plain_module(self.linear1 if linear1 is None else linear1, nn.Linear)
             and ops.plain_module(self.activation, nn.SiLU)
             and ops.plain_module(drop, nn.Dropout)
             and not (drop.training and drop.p > 0.0)

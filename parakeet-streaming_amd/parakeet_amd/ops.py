@@ -622,7 +622,7 @@ def layer_applies(dtype: torch.dtype, device: torch.device, rows: int, weight: t
     if max((n - 1) * ld + k, rows * k, rows * n) >= 1 << 31:
         return False
     if bias is not None and (
-        not _plain(bias) or tuple(bias.shape) != (n,) or bias.dtype != dtype or bias.device != device
+        not _plain(bias) or bias.shape != (n,) or bias.dtype != dtype or bias.device != device
         or not bias.is_contiguous() or bias.data_ptr() % 16
     ):
         return False
@@ -642,13 +642,18 @@ def linear_applies(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | N
     return k > 0 and layer_applies(x.dtype, x.device, x.numel() // k, weight, bias, silu)
 
 
-def _linear_args(a: LinearArgs, dt: torch.dtype, dev: torch.device, x: torch.Tensor, rows: int, weight, bias, out, silu: bool) -> None:
+def _check_linear(dt: torch.dtype, dev: torch.device, x: torch.Tensor, weight, bias) -> None:
     n, k = weight.shape
     if k != x.shape[-1] or weight.dtype != dt or weight.device != dev or weight.stride(1) != 1:
         raise ValueError(f"weight {tuple(weight.shape)} {weight.dtype} on {weight.device}, strides {weight.stride()}, does not "
                          f"take x {tuple(x.shape)} of {dt} on {dev}")
     if bias is not None and (tuple(bias.shape) != (n,) or bias.dtype != dt or bias.device != dev or not bias.is_contiguous()):
         raise ValueError(f"bias must be contiguous [{n}] of {dt} on {dev}")
+
+
+def _linear_args(a: LinearArgs, dt: torch.dtype, dev: torch.device, x: torch.Tensor, rows: int, weight, bias, out, silu: bool) -> None:
+    """The arguments of a layer that :func:`_check_linear` or :func:`layer_applies` accepted."""
+    n, k = weight.shape
     a.dtype, a.device = _DTYPES[dt], dev.index or 0
     a.rows, a.n, a.k = rows, n, k
     a.activation = _lib.ACT_SILU if silu else _lib.ACT_NONE
@@ -668,6 +673,11 @@ def linear(
 ) -> torch.Tensor:
     """``x @ weight.T + bias``, and SiLU of it, in one launch, for layers that
     :func:`linear_applies` accepts (feedforward.py:20-26, attention.py:92,122)."""
+    _check_linear(x.dtype, x.device, x, weight, bias)
+    return _linear(x, weight, bias, silu, out)
+
+
+def _linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, silu: bool = False, out: torch.Tensor | None = None) -> torch.Tensor:
     x = _aligned_rows(x)
     n, k = weight.shape
     if out is None:
@@ -683,14 +693,14 @@ def linear(
 def module_linear(x: torch.Tensor, m: torch.nn.Module) -> torch.Tensor:
     """``m(x)`` of a torch ``Linear``: :func:`linear` where it applies."""
     if plain_module(m, torch.nn.Linear) and linear_applies(x, m.weight, m.bias):
-        return linear(x, m.weight, m.bias)
+        return _linear(x, m.weight, m.bias)
     return m(x)
 
 
 def functional_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
     """``torch.nn.functional.linear``: :func:`linear` where it applies."""
     if linear_applies(x, weight, bias):
-        return linear(x, weight, bias)
+        return _linear(x, weight, bias)
     return torch.nn.functional.linear(x, weight, bias)
 
 
@@ -841,6 +851,7 @@ def glu_conv(
     taps, S, Ly, K, dev = _conv_operands(x, conv_cache, dw_weight, vecs, slots, layer, B, D)
     if tuple(weight.shape) != (2 * D, D):
         raise ValueError(f"weight must be [{2 * D}, {D}], got {tuple(weight.shape)}")
+    _check_linear(dt, dev, x, weight, bias)
     fused = bool(lib().pk_linear_takes_norm(rows, 2 * D, D, T))
     y = torch.empty((B, T, D), dtype=torch.float32, device=dev)
     a, c = LinearArgs(), ConvArgs()
@@ -882,6 +893,7 @@ def norm_silu_linear(y: torch.Tensor, norm: torch.nn.LayerNorm, weight: torch.Te
         raise ValueError(f"y must be contiguous float32, got {y.dtype}")
     n, k = weight.shape
     rows, dev, dt = y.numel() // k, y.device, weight.dtype
+    _check_linear(dt, dev, y, weight, bias)
     out = torch.empty((*y.shape[:-1], n), dtype=dt, device=dev)
     a = LinearArgs()
     _linear_args(a, dt, dev, y, rows, weight, bias, out, False)
@@ -897,6 +909,12 @@ def norm_silu_linear(y: torch.Tensor, norm: torch.nn.LayerNorm, weight: torch.Te
 def feed_forward(x: torch.Tensor, w1: torch.Tensor, b1: torch.Tensor | None, w2: torch.Tensor, b2: torch.Tensor | None) -> torch.Tensor:
     """``linear2(SiLU(linear1(x)))`` (feedforward.py:20-26), for two layers that
     :func:`linear_applies` accepts: two launches, one call."""
+    _check_linear(x.dtype, x.device, x, w1, b1)
+    _check_linear(x.dtype, x.device, w1.t(), w2, b2)  # as wide as linear1's outputs
+    return _feed_forward(x, w1, b1, w2, b2)
+
+
+def _feed_forward(x: torch.Tensor, w1: torch.Tensor, b1: torch.Tensor | None, w2: torch.Tensor, b2: torch.Tensor | None) -> torch.Tensor:
     x = _aligned_rows(x)
     rows = x.numel() // w1.shape[1]
     h = torch.empty((rows, w1.shape[0]), dtype=x.dtype, device=x.device)

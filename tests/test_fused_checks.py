@@ -160,7 +160,7 @@ def test_feed_forward_of_unequal_layers_is_refused_by_torch(monkeypatch):
     ff.linear2 = nn.Linear(2048, 512).half().requires_grad_(False)
     monkeypatch.setattr(ops, "linear_applies", lambda *a, **k: True)
     monkeypatch.setattr(ops, "linear", lambda x, w, b, silu=False: torch.nn.functional.silu(torch.nn.functional.linear(x, w, b)))
-    monkeypatch.setattr(ops, "feed_forward", lambda *a: pytest.fail("the launch would read past the hidden rows"))
+    monkeypatch.setattr(ops, "_feed_forward", lambda *a: pytest.fail("the launch would read past the hidden rows"))
     with pytest.raises(RuntimeError):
         ff(_half(2, 2, 512))
 
