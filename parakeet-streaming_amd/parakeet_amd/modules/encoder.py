@@ -10,7 +10,8 @@
   the attention of every layer runs on the paged cache;
 * ``EncoderStepGraph`` replays a recorded step for a fixed batch: the 9 to 14
   launches per layer that ``forward`` issues from Python (15 to 17 where the layer
-  runs module by module) become one HIP graph replay, with the host page work and one upload per step left outside it.
+  runs module by module) become one HIP graph replay, with the host page work and
+  one upload per step left outside it.
 
 The parameters are torch modules with the reference's names (encoder.py:11-81,
 feedforward.py:4-26).  In 16 bits without gradients, a layer's products run on

@@ -32,8 +32,6 @@ layer, q | k | v; batch row b reads row b); the outputs land in per-layer
 
 from __future__ import annotations
 
-import ctypes
-
 import numpy as np
 import torch
 
